@@ -167,6 +167,7 @@ __device__ __forceinline__ Body load_body(const W& w, uint32_t row) {
 __global__ void k_reset_counters(W w) {
     const uint32_t t = threadIdx.x;
     if (t < kPerStepCount) *cw(w.counters, kPerStepSlots[t]) = 0u;
+    if (t == kPerStepCount) *cw(w.counters, DYN_COUNTER_SOLVER_ROWS) = 0u;  // maintained: the solver refills it
 }
 
 // body_edits.wgsl:10-18 mark_disturbed
@@ -1664,23 +1665,24 @@ __global__ void __launch_bounds__(kThreads) k_island_wake(W w) {
     block_count(cw(w.counters, DYN_COUNTER_WOKE_DEFERRED), woke);
 }
 
+// what k_blocks reads of a block's body, in one 48-byte record
+__device__ __forceinline__ void write_block_body(const W& w, uint32_t row, const Body& b) {
+    const v3 com = body_com(b);
+    float4* r = w.bbodies + 3u * row;
+    r[0] = make_float4(com.x, com.y, com.z, b.d.inverse_mass);
+    r[1] = make_float4(b.s.velocity[0], b.s.velocity[1], b.s.velocity[2], body_is_inert(b) ? 1.0f : 0.0f);
+    r[2] = make_float4(b.s.angular_velocity[0], b.s.angular_velocity[1], b.s.angular_velocity[2], 0.0f);
+}
+
 // live.wgsl count, solver_reset.wgsl
 __global__ void __launch_bounds__(kThreads) k_solver_reset(W w) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *cw(w.counters, DYN_COUNTER_SOLVER_ROWS) = 0u;  // maintained: k_rows_count refills it
-    }
     uint32_t live = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < w.n; i += gridDim.x * blockDim.x) {
         w.block_counts[i] = 0u;
         reinterpret_cast<float4*>(w.resolution)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const Body b = load_body(w, i);
         if (i < w.d && body_is_active(b.s, b.d)) ++live;
-        // what k_blocks reads of a block's body, in one 48-byte record
-        const v3 com = body_com(b);
-        float4* r = w.bbodies + 3u * i;
-        r[0] = make_float4(com.x, com.y, com.z, b.d.inverse_mass);
-        r[1] = make_float4(b.s.velocity[0], b.s.velocity[1], b.s.velocity[2], body_is_inert(b) ? 1.0f : 0.0f);
-        r[2] = make_float4(b.s.angular_velocity[0], b.s.angular_velocity[1], b.s.angular_velocity[2], 0.0f);
+        write_block_body(w, i, b);
     }
     block_count(cw(w.counters, DYN_COUNTER_LIVE), live);
 }
@@ -1691,19 +1693,20 @@ __device__ __forceinline__ bool block_resolves(const dyn_contact& c) {
     return c.point_count > 0u && c.sensor == 0u;
 }
 
-// solver_blocks.wgsl:24-48
-__global__ void __launch_bounds__(kThreads) k_blocks(W w) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *w.ncontacts) return;
+// A block's rows, position row and target speeds; false when it does not resolve, else which of its
+// rows are inert.
+__device__ __forceinline__ bool write_block(const W& w, uint32_t i, uint32_t* first, uint32_t* second,
+                                            bool* first_inert, bool* second_inert) {
     const dyn_contact& c = w.contacts[i];
     const uint32_t fb = w.owner[c.a], sb = w.owner[c.b];
+    *first = fb;
+    *second = sb;
     w.blocks[2 * i] = fb;
     w.blocks[2 * i + 1] = sb;
     float4* prow = w.prows + 3u * i;
     if (!block_resolves(c)) {
         prow[0] = make_float4(__uint_as_float(fb), __uint_as_float(sb), __uint_as_float(0u), 0.0f);
-        w.slots[2 * i] = w.slots[2 * i + 1] = kNoSlot;
-        return;
+        return false;
     }
     // the bodies as k_solver_reset recorded them: centre of mass, inverse mass, velocities, inert
     const float4* rf = w.bbodies + 3u * fb;
@@ -1731,6 +1734,21 @@ __global__ void __launch_bounds__(kThreads) k_blocks(W w) {
         if (c.points[pi].depth < 0.0f) target = c.points[pi].depth / w.p.dt;
         else if (speed < -w.p.restitution_threshold) target = -speed * c.restitution;
         w.targets[i * 4u + pi] = target;
+    }
+    *first_inert = fi;
+    *second_inert = si;
+    return true;
+}
+
+// solver_blocks.wgsl:24-48
+__global__ void __launch_bounds__(kThreads) k_blocks(W w) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= *w.ncontacts) return;
+    uint32_t fb, sb;
+    bool fi, si;
+    if (!write_block(w, i, &fb, &sb, &fi, &si)) {
+        w.slots[2 * i] = w.slots[2 * i + 1] = kNoSlot;
+        return;
     }
     // a non-inert row's count is the length of its list; the count before this block's
     // increment is the block's place on it
@@ -1877,9 +1895,9 @@ __device__ __forceinline__ SolverBody load_solver_body(const W& w, uint32_t row)
     return r;
 }
 
-// solver_block_solve.wgsl:24-54 for every claimed row: the frozen or unsplit body of a block.
-__device__ __forceinline__ void solver_bodies_at(const W& w, uint32_t row) {
-    if (row >= w.n || w.block_counts[row] == 0u) return;
+// solver_block_solve.wgsl:24-54 for every claimed row (`blocks` on it): the frozen or unsplit body of
+// a block. Returns the body as loaded (frozen when inert).
+__device__ __forceinline__ Body write_solver_body(const W& w, uint32_t row, uint32_t blocks) {
     Body b = load_body(w, row);
     const bool inert = body_is_inert(b);
     if (inert) body_frozen(b);
@@ -1888,12 +1906,18 @@ __device__ __forceinline__ void solver_bodies_at(const W& w, uint32_t row) {
     p[1] = make_float4(b.d.inverse_inertia[0], b.d.inverse_inertia[1], b.d.inverse_inertia[2],
                        b.d.inverse_inertia[3]);
     p[2] = make_float4(b.d.inverse_inertia[4], b.d.inverse_inertia[5], b.d.inverse_mass,
-                       static_cast<float>(max(w.block_counts[row], 1u)));
+                       static_cast<float>(max(blocks, 1u)));
     p[3] = make_float4(b.s.velocity[0], b.s.velocity[1], b.s.velocity[2], 0.0f);
     p[4] = make_float4(b.s.angular_velocity[0], b.s.angular_velocity[1], b.s.angular_velocity[2], 0.0f);
     float4* o = w.sposes + 2u * row;
     o[0] = make_float4(b.s.position[0], b.s.position[1], b.s.position[2], inert ? 1.0f : 0.0f);
     o[1] = make_float4(b.d.com[0], b.d.com[1], b.d.com[2], 0.0f);
+    return b;
+}
+
+__device__ __forceinline__ void solver_bodies_at(const W& w, uint32_t row) {
+    if (row >= w.n || w.block_counts[row] == 0u) return;
+    write_solver_body(w, row, w.block_counts[row]);
 }
 
 // A claimed row's body as the substep's blocks see it, from the row's two copies above: pose,
@@ -1932,9 +1956,19 @@ __global__ void __launch_bounds__(kThreads) k_solver_bodies(W w) {
     solver_bodies_at(w, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
+// Where the launched passes' block deltas go: the block's words (commit_block).
+struct WordCommit {
+    const W& w;
+    uint32_t ci;
+    bool residual;
+    __device__ __forceinline__ void operator()(uint32_t, uint32_t, bool fi, bool si, v3 da, v3 sa, v3 db, v3 sbv) const {
+        commit_block(w, ci, fi, si, da, sa, db, sbv, residual);
+    }
+};
+
 // solver_contact_block.wgsl:195-233
-__device__ __forceinline__ void warm_at(const W& w, uint32_t ci) {
-    if (ci >= *w.ncontacts) return;
+template <typename Commit>
+__device__ __forceinline__ void warm_block(const W& w, uint32_t ci, const Commit& commit) {
     const dyn_contact& contact = w.contacts[ci];
     if (!block_resolves(contact)) return;
     const uint32_t fb = w.blocks[2 * ci], sb = w.blocks[2 * ci + 1];
@@ -1951,10 +1985,15 @@ __device__ __forceinline__ void warm_at(const W& w, uint32_t ci) {
                                mul(t2, p.accumulated_tangent_2));
         apply_pair_impulse(first, second, aa, ab, impulse);
     }
-    commit_block(w, ci, fi, si, sub(ld3(first.s.velocity), ld3(fl.s.velocity)),
-                 sub(ld3(first.s.angular_velocity), ld3(fl.s.angular_velocity)),
-                 sub(ld3(second.s.velocity), ld3(sl.s.velocity)),
-                 sub(ld3(second.s.angular_velocity), ld3(sl.s.angular_velocity)), false);
+    commit(fb, sb, fi, si, sub(ld3(first.s.velocity), ld3(fl.s.velocity)),
+           sub(ld3(first.s.angular_velocity), ld3(fl.s.angular_velocity)),
+           sub(ld3(second.s.velocity), ld3(sl.s.velocity)),
+           sub(ld3(second.s.angular_velocity), ld3(sl.s.angular_velocity)));
+}
+
+__device__ __forceinline__ void warm_at(const W& w, uint32_t ci) {
+    if (ci >= *w.ncontacts) return;
+    warm_block(w, ci, WordCommit{w, ci, false});
 }
 
 __global__ void __launch_bounds__(kThreads) k_warm(W w) {
@@ -2070,9 +2109,10 @@ __global__ void __launch_bounds__(kThreads) k_solve_prep(W w, uint32_t load_impu
 
 // solver_contact_block.wgsl:31-193 over the block's row: the points' impulses are applied as
 // each point is solved (every point reads only the velocities the block started from, so this
-// adds the same impulses in the same order as applying them all after the loop).
-__device__ __forceinline__ void solve_at(const W& w, uint32_t ci, uint32_t residual) {
-    if (ci >= *w.ncontacts) return;
+// adds the same impulses in the same order as applying them all after the loop). `bodies` gives a
+// row's solver body, `commit` takes the two sides' deltas.
+template <typename Bodies, typename Commit>
+__device__ __forceinline__ void solve_block(const W& w, uint32_t ci, const Bodies& bodies, const Commit& commit) {
     const float4* row = solve_section(w, ci, 0u);
     const float4 h0 = row[0];
     const uint32_t flags = __float_as_uint(h0.z);
@@ -2084,7 +2124,7 @@ __device__ __forceinline__ void solve_at(const W& w, uint32_t ci, uint32_t resid
     const float4 h1 = row[1], h2 = row[2];
     const v3 normal = mk(h1.x, h1.y, h1.z);
     const float relaxation = h1.w, damping_ratio = h2.x;
-    const SolverBody bf = load_solver_body(w, fb), bs = load_solver_body(w, sb);
+    const SolverBody bf = bodies(fb), bs = bodies(sb);
     float split_f[6], split_s[6];
     for (int k = 0; k < 6; ++k) {
         split_f[k] = bf.inertia[k] * bf.count;
@@ -2167,8 +2207,18 @@ __device__ __forceinline__ void solve_at(const W& w, uint32_t ci, uint32_t resid
     imp[0] = make_float4(acc_n[0], acc_n[1], acc_n[2], acc_n[3]);
     imp[1] = make_float4(acc_1[0], acc_1[1], acc_1[2], acc_1[3]);
     imp[2] = make_float4(acc_2[0], acc_2[1], acc_2[2], acc_2[3]);
-    commit_block(w, ci, fi, si, sub(first_v, vf), sub(first_w, wf), sub(second_v, vs), sub(second_w, ws),
-                 residual != 0u);
+    commit(fb, sb, fi, si, sub(first_v, vf), sub(first_w, wf), sub(second_v, vs), sub(second_w, ws));
+}
+
+// A row's solver body as its record holds it.
+struct RecordBodies {
+    const W& w;
+    __device__ __forceinline__ SolverBody operator()(uint32_t row) const { return load_solver_body(w, row); }
+};
+
+__device__ __forceinline__ void solve_at(const W& w, uint32_t ci, uint32_t residual) {
+    if (ci >= *w.ncontacts) return;
+    solve_block(w, ci, RecordBodies{w}, WordCommit{w, ci, residual != 0u});
 }
 
 __global__ void __launch_bounds__(kThreads) k_solve(W w, uint32_t residual) {
@@ -2356,20 +2406,26 @@ __global__ void __launch_bounds__(kThreads) k_advance(W w) {
 }
 
 // position_correction.wgsl:5-46, position_block.wgsl, from the block's position row
-// position_correction.wgsl:5-46 for one block of `count` points: false when it contributes
-// nothing, else its two sides' corrections (inert rows only get their "contributed" mark).
-__device__ __forceinline__ bool position_correction(const W& w, float4 h0, const float4* prow, uint32_t flags,
-                                                    uint32_t count, v3* la_out, v3* lb_out) {
-    const uint32_t fr = __float_as_uint(h0.x), sr = __float_as_uint(h0.y);
-    const bool fi = (flags & 8u) != 0u, si = (flags & 16u) != 0u;
-    const float imf = h0.w;
+// What the position phase reads of a block besides its rows and flags (the block's position row).
+struct PositionRow {
+    float first_mass, second_mass;  // inverse masses, zero for inert rows
+    v3 normal;
+    float4 depths;
+};
+
+__device__ __forceinline__ PositionRow load_position_row(float4 h0, const float4* prow) {
     const float4 h1 = prow[1];
-    const float ims = h1.x;
-    const v3 normal = mk(h1.y, h1.z, h1.w);
-    const float4 depths = prow[2];
-    const float4 rs = reinterpret_cast<const float4*>(w.resolution)[sr];
-    const float4 rf = reinterpret_cast<const float4*>(w.resolution)[fr];
-    const float resolved = dot3(normal, sub(mk(rs.x, rs.y, rs.z), mk(rf.x, rf.y, rf.z)));
+    return PositionRow{h0.w, h1.x, mk(h1.y, h1.z, h1.w), prow[2]};
+}
+
+// position_correction.wgsl:5-46 for one block of `count` points: false when it contributes
+// nothing, else its two sides' corrections. rf, rs: what its rows have resolved so far.
+__device__ __forceinline__ bool position_correction(const W& w, const PositionRow& row, uint32_t count, v3 rf, v3 rs,
+                                                    v3* la_out, v3* lb_out) {
+    const float imf = row.first_mass, ims = row.second_mass;
+    const v3 normal = row.normal;
+    const float4 depths = row.depths;
+    const float resolved = dot3(normal, sub(rs, rf));
     v3 total = zero3v();
     uint32_t contributing = 0;
 #pragma unroll
@@ -2387,9 +2443,6 @@ __device__ __forceinline__ bool position_correction(const W& w, float4 h0, const
     const v3 correction = dv(total, static_cast<float>(contributing));
     const v3 la = mul(neg(correction), imf), lb = mul(correction, ims);
     if (!(dot3(la, la) > 0.0f || dot3(lb, lb) > 0.0f)) return false;
-    // Inert rows get exactly zero words; only their "contributed" mark matters.
-    if (fi) w.contrib[fr] = 1u;
-    if (si) w.contrib[sr] = 1u;
     *la_out = la;
     *lb_out = lb;
     return true;
@@ -2405,7 +2458,18 @@ __device__ __forceinline__ void position_block_at(const W& w, uint32_t ci) {
     v3 la, lb;
     // every entry of the block is written once per pass: "no contribution" unless corrected
     uint4 wa = make_uint4(0u, 0u, 0u, 0u), wb = wa;
-    if (count != 0u && position_correction(w, h0, prow, flags, count, &la, &lb)) {
+    const uint32_t fr = __float_as_uint(h0.x), sr = __float_as_uint(h0.y);
+    bool contributes = false;
+    if (count != 0u) {
+        const float4 rs = reinterpret_cast<const float4*>(w.resolution)[sr];
+        const float4 rf = reinterpret_cast<const float4*>(w.resolution)[fr];
+        contributes = position_correction(w, load_position_row(h0, prow), count, mk(rf.x, rf.y, rf.z),
+                                          mk(rs.x, rs.y, rs.z), &la, &lb);
+    }
+    if (contributes) {
+        // Inert rows get exactly zero words; only their "contributed" mark matters.
+        if (flags & 8u) w.contrib[fr] = 1u;
+        if (flags & 16u) w.contrib[sr] = 1u;
         const float scale = DYN_SOLVER_POSITION_SCALE;
         wa = make_uint4(1u, solver_word(la.x, scale), solver_word(la.y, scale), solver_word(la.z, scale));
         wb = make_uint4(1u, solver_word(lb.x, scale), solver_word(lb.y, scale), solver_word(lb.z, scale));
@@ -2416,6 +2480,20 @@ __device__ __forceinline__ void position_block_at(const W& w, uint32_t ci) {
 
 __global__ void __launch_bounds__(kThreads) k_position_block(W w) {
     position_block_at(w, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// A row's pose after `contributing` blocks sent it the given linear words (position_apply.wgsl; the
+// position blocks send no angular words).
+__device__ __forceinline__ void position_move(v3 p0, float4 q0, uint32_t x, uint32_t y, uint32_t z, uint32_t contributing,
+                                              v3* p1, float4* q1, v3* moved) {
+    const v3 lin = mk(solver_value(x, DYN_SOLVER_POSITION_SCALE), solver_value(y, DYN_SOLVER_POSITION_SCALE),
+                      solver_value(z, DYN_SOLVER_POSITION_SCALE));
+    const float none = solver_value(0u, DYN_SOLVER_POSITION_SCALE);
+    const float cf = static_cast<float>(contributing);
+    const v3 al = dv(lin, cf), aa = dv(mk(none, none, none), cf);
+    *p1 = add(p0, al);
+    *q1 = qnorm(qmul(make_float4(aa.x * 0.5f, aa.y * 0.5f, aa.z * 0.5f, 1.0f), q0));
+    *moved = al;
 }
 
 // position_apply.wgsl over every claimed row
@@ -2451,8 +2529,7 @@ __device__ __forceinline__ void position_apply_at(const W& w, uint32_t t, uint32
         r0 = r;
     }
     uint32_t contributing = 0;
-    uint4 lo = make_uint4(0u, 0u, 0u, 0u);  // linear words, then the (zero) angular x
-    uint2 hi = make_uint2(0u, 0u);          // angular y, z: the position blocks send none
+    uint3 lo = make_uint3(0u, 0u, 0u);
     const uint4* run = w.pwords + start;
     for (uint32_t e = sub; e < count; e += kApplyBatch * lanes) {
         uint4 word[kApplyBatch];
@@ -2492,14 +2569,9 @@ __device__ __forceinline__ void position_apply_at(const W& w, uint32_t t, uint32
             return;
         }
     }
-    const v3 lin = mk(solver_value(lo.x, DYN_SOLVER_POSITION_SCALE), solver_value(lo.y, DYN_SOLVER_POSITION_SCALE),
-                      solver_value(lo.z, DYN_SOLVER_POSITION_SCALE));
-    const v3 ang = mk(solver_value(lo.w, DYN_SOLVER_POSITION_SCALE), solver_value(hi.x, DYN_SOLVER_POSITION_SCALE),
-                      solver_value(hi.y, DYN_SOLVER_POSITION_SCALE));
-    const float cf = static_cast<float>(contributing);
-    const v3 al = dv(lin, cf), aa = dv(ang, cf);
-    const v3 p1 = add(p0, al);
-    const float4 q1 = qnorm(qmul(make_float4(aa.x * 0.5f, aa.y * 0.5f, aa.z * 0.5f, 1.0f), q0));
+    v3 p1, al;
+    float4 q1;
+    position_move(p0, q0, lo.x, lo.y, lo.z, contributing, &p1, &q1, &al);
     if (count == 0u || last) {
         st3(s.position, p1);
         st4(s.orientation, q1);
@@ -2514,6 +2586,8 @@ __device__ __forceinline__ void position_apply_at(const W& w, uint32_t t, uint32
 __global__ void __launch_bounds__(kThreads) k_position_apply(W w, uint32_t first, uint32_t last, uint32_t lanes_log2) {
     position_apply_at(w, blockIdx.x * blockDim.x + threadIdx.x, first, last, lanes_log2);
 }
+
+#include "group_solver.h"
 
 // island_sleep.wgsl
 __global__ void __launch_bounds__(kThreads) k_sleep(W w) {
@@ -2673,6 +2747,14 @@ struct SideStream {
     hipEvent_t fork, join;
 };
 
+// The worlds that k_group_solve or k_group_position takes, a workgroup each, in one launch (largest
+// first, so the longest workgroups start first). No worlds: the launched solver.
+struct GroupPlan {
+    const dyn::GroupWorld* worlds = nullptr;  // null: the one world of all rows
+    uint32_t count = 0, rows = 0;             // worlds, and the most rows of one
+    bool whole = false;                       // the whole solver, not the position iterations alone
+};
+
 struct dyn_world {
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -2737,6 +2819,7 @@ struct dyn_world {
     bool tuning = false;              // steps of dyn_world_tune_solver: no demand is recorded
     float last_dt = 0.0f;             // the dt of the last step
     uint32_t solver_threads = dyn::kThreads;  // workgroup size of the solver substeps' kernels
+    GroupPlan groups;
     // the tape a recorded step writes (dyn::world_record); null when not recording
     float* tape_states = nullptr;
     float* tape_contacts = nullptr;
@@ -3059,7 +3142,7 @@ int island_components(const dyn::W& w, hipStream_t st, float slop) {
 // counts, the contact blocks, the rows' block lists.
 int solver_prepare(const dyn::W& w, hipStream_t st) {
     using namespace dyn;
-    const uint32_t nb = blocks_for(w.n), cb = blocks_for(w.contact_cap);
+    const uint32_t cb = blocks_for(w.contact_cap);
     LAUNCH_ON(st, k_solver_reset, count_blocks(w.n), w);
     LAUNCH_ON(st, k_blocks, cb, w);
     LAUNCH_ON(st, k_rows_count, count_blocks(w.n), w);
@@ -3077,13 +3160,61 @@ int solver_prepare(const dyn::W& w, hipStream_t st) {
         DYN_LAUNCHED(#name);                                                              \
     } while (0)
 
+// Rows a workgroup of k_group_solve and k_group_position can hold: 64 bytes of LDS each.
+constexpr uint32_t kGroupRowLimit = 2304;
+// Worlds of at most this many rows are solved whole by a workgroup: one CU's share of the velocity
+// iterations then takes no longer than launching them (5 us an iteration at 33 contacts, 35 us at
+// 2,664, against about 12 us launched). Larger ones, up to the limit above, run only their position
+// iterations so (103 us for 20 of them at 2,664 contacts, against 5 us a launch and two each).
+constexpr uint32_t kGroupWholeRows = 160;
+
+template <typename Kernel, typename... Args>
+int group_launch(const char* name, Kernel kernel, uint32_t threads, hipStream_t st, const GroupPlan& g, Args... args) {
+    using namespace dyn;
+    const uint32_t lds = g.rows * kGroupRowWords * 4u;
+    if (lds > 60u * 1024u) {
+        DYN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(lds)));
+    }
+    {
+        ProfileScope scope(name, st);
+        kernel<<<g.count, threads, lds, st>>>(args...);
+    }
+    DYN_LAUNCHED("group kernel");
+    return DYN_OK;
+}
+
+int group_solve(const dyn::W& w, hipStream_t st, const GroupPlan& g) {
+    using namespace dyn;
+    const char* name = "k_group_solve";
+    if (g.rows <= 64u) return group_launch(name, k_group_solve<128u>, 128u, st, g, w, g.worlds);
+    return group_launch(name, k_group_solve<256u>, 256u, st, g, w, g.worlds);
+}
+
+int group_position(const dyn::W& w, hipStream_t st, const GroupPlan& g, uint32_t first, uint32_t last) {
+    using namespace dyn;
+    const char* name = "k_group_position";
+    if (g.rows <= 256u) return group_launch(name, k_group_position<256u>, 256u, st, g, w, g.worlds, first, last);
+    return group_launch(name, k_group_position<1024u>, 1024u, st, g, w, g.worlds, first, last);
+}
+
+// The plan of one world of n rows.
+GroupPlan plan_group(uint32_t n) {
+    GroupPlan plan;
+    if (n && n <= kGroupRowLimit) {
+        plan.count = 1u;
+        plan.rows = n;
+        plan.whole = n <= kGroupWholeRows;
+    }
+    return plan;
+}
+
 // The substeps of SolveSubsteps (solver.rs:311-332), then the accumulated impulses back into the
 // contacts. The per-contact and per-row kernels of the substeps index their element by the global
 // thread index alone, so they run in workgroups of `threads` (64, 128 or 256; the solver's
 // autotuned shape) with the same results.
-int solver_substeps(const dyn::W& w, hipStream_t st, uint32_t threads = dyn::kThreads) {
+int solver_substeps(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint32_t threads) {
     using namespace dyn;
-    const uint32_t nb = blocks_for(w.n);
     // lanes a row in the apply kernels: four for a world of up to 2^18 rows (too few rows to keep
     // the GPU's memory pipes busy otherwise; eight were slower), two above (one was slower)
     const uint32_t lanes_log2 = w.n <= (1u << 18) ? 2u : 1u;
@@ -3104,6 +3235,10 @@ int solver_substeps(const dyn::W& w, hipStream_t st, uint32_t threads = dyn::kTh
             LAUNCH_TH(st, k_apply, w.n << lanes_log2, threads, w, it + 1u == w.p.solve_iterations ? 1u : 0u,
                       lanes_log2);
         }
+        if (plan.count) {
+            DYN_TRY(group_position(w, st, plan, sub == 0u ? 1u : 0u, sub + 1u == w.p.substeps ? 1u : 0u));
+            continue;
+        }
         LAUNCH_TH(st, k_advance, w.d, threads, w);
         for (uint32_t it = 0; it < w.p.position_iterations; ++it) {
             LAUNCH_TH(st, k_position_block, w.contact_cap, threads, w);
@@ -3112,8 +3247,57 @@ int solver_substeps(const dyn::W& w, hipStream_t st, uint32_t threads = dyn::kTh
         }
     }
     LAUNCH_TH(st, k_impulses_store, w.contact_cap, threads, w);
-    (void)nb;
     return DYN_OK;
+}
+
+// SolverReset and SolveSubsteps by the plan: worlds solved whole by a workgroup each, or launched pass
+// by pass (with the plan's position iterations).
+int solver(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint32_t threads = dyn::kThreads) {
+    if (plan.whole) return group_solve(w, st, plan);
+    DYN_TRY(solver_prepare(w, st));
+    return solver_substeps(w, st, plan, threads);
+}
+
+// The plan of a batch: every world's colliders, simulated rows and other rows must each be one run
+// (as merge_scenes lays them out) and every row must belong to a world of at most kGroupRowLimit
+// rows; otherwise no launches, and the batch is solved by the launched passes.
+void plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t colliders,
+                 const std::vector<uint32_t>& world_of_row, uint32_t worlds) {
+    using namespace dyn;
+    const W& w = world->w;
+    for (uint32_t i = 1; i < colliders; ++i) {
+        if (collider_worlds[i] < collider_worlds[i - 1]) return;
+    }
+    std::vector<GroupWorld> table(worlds, GroupWorld{});
+    for (uint32_t i = 0; i < colliders; ++i) {
+        GroupWorld& g = table[collider_worlds[i]];
+        if (g.collider_count++ == 0u) g.collider_base = i;
+    }
+    for (uint32_t row = 0; row < w.n; ++row) {
+        if (world_of_row[row] == DYN_NO_BODY) return;
+        GroupWorld& g = table[world_of_row[row]];
+        uint32_t& base = row < w.d ? g.dynamic_base : g.static_base;
+        uint32_t& count = row < w.d ? g.dynamic_count : g.static_count;
+        if (count == 0u) base = row;
+        if (row != base + count) return;
+        ++count;
+    }
+    std::vector<GroupWorld> order;
+    for (const GroupWorld& g : table) {
+        if (g.dynamic_count + g.static_count > kGroupRowLimit) return;
+        if (g.dynamic_count + g.static_count) order.push_back(g);
+    }
+    auto rows = [](const GroupWorld& g) { return g.dynamic_count + g.static_count; };
+    std::stable_sort(order.begin(), order.end(), [&](const GroupWorld& a, const GroupWorld& b) { return rows(a) > rows(b); });
+    GroupWorld* device = nullptr;
+    if (order.empty() || alloc(world, &device, order.size()) != DYN_OK ||
+        hipMemcpy(device, order.data(), sizeof(GroupWorld) * order.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        return;
+    }
+    world->groups.worlds = device;
+    world->groups.count = static_cast<uint32_t>(order.size());
+    world->groups.rows = rows(order[0]);
+    world->groups.whole = rows(order[0]) <= kGroupWholeRows;
 }
 
 void drop_graph(dyn_world* world) {
@@ -3242,12 +3426,11 @@ int world_step(dyn_world* world, float dt) {
     DYN_TRY(island_flatten(w, st, kFlattenPasses - 1u));
     LAUNCH(k_island_aggregate, count_blocks(w.d), w);
     LAUNCH(k_island_wake, count_blocks(w.d), w);
-    DYN_TRY(solver_prepare(w, st));
     if (world->tape_states) {
         LAUNCH(k_tape_record, blocks_for(std::max(w.n, w.contact_cap)), w, world->tape_states, world->tape_contacts,
                world->tape_count, world->tape_error);
     }
-    DYN_TRY(solver_substeps(w, st, world->solver_threads));
+    DYN_TRY(solver(w, st, world->groups, world->solver_threads));
     LAUNCH(k_sleep, count_blocks(w.d), w);
     LAUNCH(k_thaw, cb, w);
     LAUNCH(k_archive, cb, w, world->freeze_flags);
@@ -3435,6 +3618,7 @@ int dyn_world_create(dyn_world** out, void* stream, const dyn_step_params* param
     up(w.row_of_body, row_of_body.data(), sizeof(uint32_t) * id_cap);
     up(w.owner, owners, 4u * collider_count);
     if (rc != DYN_OK) return cleanup(fail(DYN_E_HIP, "dyn_world_create: upload"));
+    world->groups = plan_group(w.n);
     *out = world;
     return DYN_OK;
 }
@@ -3469,6 +3653,8 @@ int dyn_batch_create(dyn_world** out, void* stream, const dyn_step_params* param
         return fail(DYN_E_HIP, "dyn_batch_create: world ids");
     }
     world->w.worlds = worlds;
+    world->groups = GroupPlan{};
+    plan_groups(world, collider_worlds, collider_count, world_of_row, world_count);
     *out = world;
     return DYN_OK;
 }
@@ -3970,8 +4156,7 @@ int dyn_solve(void* stream, const dyn_solve_io* io, float dt) {
     DYN_HIP(hipMemcpyAsync(&bad, words + 1, 4u, hipMemcpyDeviceToHost, st));
     DYN_HIP(hipStreamSynchronize(st));
     if (bad) return fail(DYN_E_INVALID, "dyn_solve: a contact names a collider or body outside the records");
-    DYN_TRY(solver_prepare(w, st));
-    return solver_substeps(w, st);
+    return solver(w, st, plan_group(w.n));
 }
 
 size_t dyn_islands_scratch_bytes(uint32_t bodies) {

@@ -1,0 +1,94 @@
+"""The solver of small worlds (k_group_solve, k_group_position) at the edges of its rules: row counts
+on both sides of each workgroup size and of the limits, more contacts than its threads hold in
+registers, sleeping rows, and batches whose worlds sit on both sides. Bit for bit against the
+oracle's solver, and each world of a batch against itself alone."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from dynamis_amd._native import call
+from dynamis_amd.world import Batch, World
+from tests.solve_cases import NO_SLEEP, drop_scene
+from tests.test_gpu_solve import check_parity
+from tests.worlds import DT, config, cube_drop, encode
+
+pytestmark = pytest.mark.gpu
+
+
+# bodies (a plane more): 64 | 65 rows (128 | 256 threads), 160 | 161 (whole | position only),
+# 256 | 257 (256 | 1,024 threads), 2304 | 2305 (position only | launched)
+@pytest.mark.parametrize("count", [1, 63, 64, 159, 160, 255, 256])
+def test_row_edges(device, oracle, count):
+    check_parity(oracle, drop_scene(count, footprint=1.2 + 0.35 * count ** 0.5), 60, 0 if count == 1 else count // 2)
+
+
+@pytest.mark.parametrize("count", [2303, 2304])
+def test_row_limit(device, oracle, count):
+    # a lattice of touching cubes on the plane: contacts from the first frames on
+    side = 12.0
+    check_parity(oracle, drop_scene(count, footprint=side), 4, 4000)
+
+
+@pytest.mark.parametrize("count,footprint", [(159, 1.5), (255, 1.0)])
+def test_more_contacts_than_registers_hold(device, oracle, count, footprint):
+    # cubes dropped onto one spot overlap one another many times over: above 4 x 256 contacts
+    scene = encode(cube_drop(count, seed=5, footprint=footprint, low=1.0, high=4.0), config(**NO_SLEEP))
+    check_parity(oracle, scene, 2, 1025)
+
+
+def test_sleeping_rows(device, oracle):
+    scene = encode(cube_drop(120, seed=1, footprint=8.0, high=4.0), config())
+    inputs, _ = check_parity(oracle, scene, 200, 100)
+    assert (inputs.states["sleeping"][:scene.dynamic_count] != 0).any()
+
+
+@pytest.mark.parametrize("counts", [(3, 40, 1, 150), (5, 400, 1, 70, 260), (2500, 30)])
+def test_batches_on_both_sides(device, counts):
+    scenes = [encode(cube_drop(n, seed=7 + i, footprint=0.9 * n ** 0.5 + 1.0, low=1.0, high=3.0), config())
+              for i, n in enumerate(counts)]
+    batch = Batch(scenes)
+    alone = []
+    for s in scenes:
+        w = World()
+        w.create(s)
+        alone.append(w)
+    for _ in range(40):
+        batch.step(DT)
+        for w in alone:
+            w.step(DT)
+    states = batch.states()
+    for i, w in enumerate(alone):
+        assert batch.world_states(i, states).tobytes() == w.states().tobytes(), i
+    total = {k: sum(w.measured()[k] for w in alone) for k in ("CONTACTS", "SOLVER_ROWS", "LIVE")}
+    got = batch.measured()
+    assert {k: got[k] for k in total} == total
+    batch.close()
+    for w in alone:
+        w.close()
+
+
+def test_batch_of_scattered_colliders(device):
+    """Colliders of two worlds interleaved: their contacts are no runs, and the launched passes run."""
+    scenes = [encode(cube_drop(30, seed=3 + i, footprint=4.0, low=1.0, high=3.0), config()) for i in range(2)]
+    batch = Batch(scenes)
+    merged, worlds = batch.scene, batch.layout.collider_worlds
+    mixed = np.argsort(np.concatenate([np.arange(31), np.arange(31)]), kind="stable")
+    world = World()
+    world.scene = merged
+    owners, order = merged.owners[mixed].copy(), worlds[mixed].copy()
+    colliders = merged.colliders[mixed].copy()
+    n, k = len(merged.states), len(colliders)
+    call("dyn_batch_create", ctypes.byref(world._handle), None, merged.params.ctypes.data, merged.states.ctypes.data,
+         merged.descs.ctypes.data, n, merged.dynamic_count, colliders.ctypes.data, owners.ctypes.data,
+         order.ctypes.data, k, 2, 8 * n, 32 * n)
+    for _ in range(40):
+        batch.step(DT)
+        world.step(DT)
+    # each world's colliders keep their order, so its steps stay the same
+    assert world.states().tobytes() == batch.states().tobytes()
+    batch.close()
+    world.close()
