@@ -8,7 +8,6 @@
 //   - entry slots come from a prefix sum over per-collider entry counts instead of one atomic
 //     counter, so entries are laid out in collider order and equal keys leave the stable sort in
 //     collider order (the reference's order within a key is whatever its atomics produced);
-//   - the sort's digit histogram is counted while the entries are written, saving a read;
 //   - the sorted keys get a per-level directory of 2^16 hash buckets, so a coarser-level probe
 //     finds its cell's run with two directory reads and a short search inside one bucket instead
 //     of a binary search over the whole region (grid_index.wgsl:231-253);
@@ -217,20 +216,27 @@ __global__ void __launch_bounds__(1024) bp_scan_kernel(const uint32_t* __restric
     if (threadIdx.x >= 2 && threadIdx.x < kCtlWords) sort_ctl[threadIdx.x] = 0;
 }
 
-// collider_emit.wgsl:6-63 with slots from the scan; also counts the sort's key digits.
+// Workgroups up to which the emission also counts the sort's digits, saving a launch and a read of the
+// keys. Every workgroup adds its counts to the same 1,024 words, one atomic after another: at 2^20
+// boxes that made the emission 111 us, against 43 us and a 12 us pass over the keys without it.
+constexpr uint32_t kEmitHistogramBlocks = 128;
+
+// collider_emit.wgsl:6-63 with slots from the scan.
+template <bool kHistogram>
 __global__ void __launch_bounds__(kBpThreads) bp_emit_kernel(
     const dyn_aabb* __restrict__ aabbs, const uint32_t* __restrict__ groups,
     const uint32_t* __restrict__ flags, uint32_t n, uint32_t* counters,
     const uint32_t* __restrict__ cnt_level, const uint32_t* __restrict__ block_offsets,
     uint32_t* __restrict__ entry_keys, uint32_t* __restrict__ entry_order,
-    dyn_grid_entry* __restrict__ entries, uint32_t capacity, uint32_t* sort_hist,
-    const uint32_t* sort_ctl, uint32_t* flags0, const uint32_t* __restrict__ worlds,
-    uint32_t* __restrict__ first_slot) {
-    __shared__ uint32_t s_hist[kEntryPasses][kSortBins];
+    dyn_grid_entry* __restrict__ entries, uint32_t capacity, const uint32_t* __restrict__ worlds,
+    uint32_t* __restrict__ first_slot, uint32_t* sort_hist, const uint32_t* sort_ctl, uint32_t* flags0) {
+    __shared__ uint32_t s_hist[kHistogram ? kEntryPasses : 1u][kSortBins];
     __shared__ uint32_t s_scan[kBpThreads / kWave];
     const uint32_t t = threadIdx.x;
+    if (kHistogram) {
 #pragma unroll
-    for (uint32_t p = 0; p < kEntryPasses; ++p) s_hist[p][t] = 0;
+        for (uint32_t p = 0; p < kEntryPasses; ++p) s_hist[p][t] = 0;
+    }
     const uint32_t i = blockIdx.x * blockDim.x + t;
     const uint32_t packed = i < n ? cnt_level[i] : 0u;
     const uint32_t emitted = packed & 0xFFu;
@@ -270,12 +276,15 @@ __global__ void __launch_bounds__(kBpThreads) bp_emit_kernel(
             float4* rec = reinterpret_cast<float4*>(entries + slot);
             rec[0] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(group));
             rec[1] = make_float4(hi.x, hi.y, hi.z, __uint_as_float(info));
+            if (kHistogram) {
 #pragma unroll
-            for (uint32_t p = 0; p < kEntryPasses; ++p) atomicAdd(&s_hist[p][(key >> (8 * p)) & 0xFFu], 1u);
+                for (uint32_t p = 0; p < kEntryPasses; ++p) atomicAdd(&s_hist[p][(key >> (8 * p)) & 0xFFu], 1u);
+            }
         }
     }
     faults = wave_sum(faults);
     if (lane_id() == 0 && faults) atomicAdd(ctr(counters, DYN_COUNTER_ENTRY_FAULTS), faults);
+    if (!kHistogram) return;
     __syncthreads();
 #pragma unroll
     for (uint32_t p = 0; p < kEntryPasses; ++p) {
@@ -887,7 +896,6 @@ struct BpLayout {
     uint32_t* mate_counts;
     uint32_t* mate_blocks;
     uint32_t* dir;
-    uint32_t* pair_payload;
     dyn_grid_entry* sorted;
     uint2* link_stage;
     uint32_t* level_keys;
@@ -914,7 +922,6 @@ BpLayout bp_layout(uint32_t colliders, uint32_t entry_capacity, uint32_t pair_ca
     l.mate_counts = carve.take<uint32_t>(entry_capacity ? entry_capacity : 1u);
     l.mate_blocks = carve.take<uint32_t>(entry_blocks);
     l.dir = carve.take<uint32_t>(static_cast<size_t>(kGridLevels) * kDirStride);
-    l.pair_payload = carve.take<uint32_t>(pair_capacity ? pair_capacity : 1u);
     l.sorted = carve.take<dyn_grid_entry>(entry_capacity ? entry_capacity : 1u);
     l.link_stage = carve.take<uint2>(static_cast<size_t>(colliders ? colliders : 1u) * kLinkStage);
     l.level_keys = carve.take<uint32_t>(kGridLevels);
@@ -998,18 +1005,33 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
     }
     DYN_LAUNCHED("bp_scan_kernel");
     if (n == 0 || io->entry_capacity == 0) return DYN_OK;
+    const bool small_entries = io->entry_capacity <= kSortSmall;
+    const bool emit_histogram = !small_entries && blocks <= kEmitHistogramBlocks;
     {
         ProfileScope scope("bp_emit_kernel", st);
-        bp_emit_kernel<<<blocks, kBpThreads, 0, st>>>(
-            io->d_aabbs, io->d_groups, io->d_flags, n, counters, l.cnt_level, l.block_offsets,
-            io->d_entry_keys, io->d_entry_order, io->d_entries, io->entry_capacity, l.entry_sort.hist,
-            l.entry_sort.ctl, l.entry_sort.flags, io->d_worlds, l.first_slot);
+        auto launch = [&](auto kernel) {
+            kernel<<<blocks, kBpThreads, 0, st>>>(
+                io->d_aabbs, io->d_groups, io->d_flags, n, counters, l.cnt_level, l.block_offsets, io->d_entry_keys,
+                io->d_entry_order, io->d_entries, io->entry_capacity, io->d_worlds, l.first_slot, l.entry_sort.hist,
+                l.entry_sort.ctl, l.entry_sort.flags);
+        };
+        if (emit_histogram) launch(bp_emit_kernel<true>);
+        else launch(bp_emit_kernel<false>);
     }
     DYN_LAUNCHED("bp_emit_kernel");
     SortDigit digits[kSortMaxPasses];
     sort_digits(kEntryPasses, 0u, digits);
-    DYN_TRY(sort_passes(st, io->d_entry_keys, nullptr, io->d_entry_order, l.entry_sort, digits,
-                        kEntryPasses, io->entry_capacity, kEntrySortNames));
+    if (small_entries) {
+        DYN_TRY(sort_small(st, io->d_entry_keys, nullptr, io->d_entry_order, l.entry_sort.ctl + kCtlLen, nullptr,
+                           io->entry_capacity, digits, kEntryPasses, kEntrySortNames));
+    } else {
+        if (!emit_histogram) {
+            DYN_TRY(sort_histogram(st, io->d_entry_keys, nullptr, l.entry_sort, digits, kEntryPasses, io->entry_capacity,
+                                   kEntrySortNames));
+        }
+        DYN_TRY(sort_passes(st, io->d_entry_keys, nullptr, io->d_entry_order, l.entry_sort, digits, kEntryPasses,
+                            io->entry_capacity, kEntrySortNames));
+    }
     const uint32_t entry_blocks = ceil_div(io->entry_capacity, kBpThreads);
     const uint32_t dir_threads = kGridLevels * kDirStride;
     {
@@ -1087,11 +1109,16 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
         const uint32_t words = dyn_sort_key_words(n);
         sort_digits(words, words, digits);
         const uint32_t* pairs = counters + DYN_COUNTER_PAIRS * DYN_COUNTER_STRIDE_WORDS;
+        // the pairs are their own keys: no payload is moved
+        if (io->pair_capacity <= kSortSmall) {
+            return sort_small(st, io->d_pair_major, io->d_pair_minor, nullptr, pairs, nullptr, io->pair_capacity, digits,
+                              2u * words, kPairSortNames);
+        }
         DYN_TRY(sort_prepare(st, l.pair_sort, pairs, nullptr, io->pair_capacity, kPairSortNames));
         DYN_TRY(sort_histogram(st, io->d_pair_major, io->d_pair_minor, l.pair_sort, digits,
                                2u * words, io->pair_capacity, kPairSortNames));
-        DYN_TRY(sort_passes(st, io->d_pair_major, io->d_pair_minor, l.pair_payload, l.pair_sort,
-                            digits, 2u * words, io->pair_capacity, kPairSortNames));
+        DYN_TRY(sort_passes(st, io->d_pair_major, io->d_pair_minor, nullptr, l.pair_sort, digits, 2u * words,
+                            io->pair_capacity, kPairSortNames));
     }
     return DYN_OK;
 }

@@ -6,10 +6,10 @@
 
 namespace dyn {
 
-constexpr int kSortThreads = 256;                      // 4 waves
-constexpr int kSortItems = 16;                         // keys per lane per tile
-constexpr int kSortTile = kSortThreads * kSortItems;   // 4096 keys per tile
-constexpr int kSortMinTile = kSortThreads * 8;        // narrowest tiling (shorter streams)
+constexpr int kSortThreads = 512;                      // 8 waves; 8 or 16 keys a lane per tile
+constexpr int kSortMinTile = 2048;                     // keys per tile that the look-back words are laid out for
+constexpr int kSmallThreads = 1024;                    // the workgroup that sorts a short list whole
+constexpr uint32_t kSortSmall = 8u * kSmallThreads;    // capacities up to this are sorted so
 constexpr int kSortMaxPasses = 8;                      // 4 minor + 4 major digits
 constexpr int kSortBins = 256;
 constexpr uint32_t kSortMaxCapacity = (1u << 30) - 1;  // look-back values carry 30 bits
@@ -69,8 +69,15 @@ int sort_histogram(hipStream_t stream, const uint32_t* major, const uint32_t* mi
                    const SortScratch& s, const SortDigit* digits, uint32_t passes,
                    uint32_t capacity, const SortNames& names = kGenericSortNames);
 
+// The whole sort in one workgroup and one launch, for capacities up to kSortSmall: len as in
+// sort_prepare, the result in the primaries. `minor` and `payload` may be null.
+int sort_small(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* payload, const uint32_t* d_count,
+               const uint32_t* d_base, uint32_t capacity, const SortDigit* digits, uint32_t passes,
+               const SortNames& names = kGenericSortNames);
+
 // Runs the digit passes (histogram already in s.hist, first pass's look-back words clear) and
-// leaves the result in the primaries. `minor` may be null when the minor lane is not carried.
+// leaves the result in the primaries. `minor` may be null when the minor lane is not carried, or
+// `payload` (with a minor lane) when only the keys are sorted.
 int sort_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* payload,
                 const SortScratch& s, const SortDigit* digits, uint32_t passes,
                 uint32_t capacity, const SortNames& names = kGenericSortNames);

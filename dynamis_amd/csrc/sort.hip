@@ -1,5 +1,5 @@
 // Stable LSD radix sort for gfx950: 8-bit digits, one histogram read for all digits, then one
-// "onesweep" pass per digit. Each pass ranks a 4096-key tile with wave64 ballots (a key's rank
+// "onesweep" pass per digit. Each pass ranks a tile of 4096 or 8192 keys with wave64 ballots (a key's rank
 // among equal digits is the popcount of the lanes below it that hold the same digit, plus the
 // counts of earlier items and earlier waves), publishes the tile's digit counts for a decoupled
 // look-back across tiles, stages the ranked tile in LDS and writes it out digit-run by digit-run
@@ -59,13 +59,17 @@ __global__ void __launch_bounds__(256) sort_prepare_kernel(uint32_t* hist, uint3
     }
 }
 
-__global__ void __launch_bounds__(256) sort_histogram_kernel(const uint32_t* __restrict__ major,
-                                                             const uint32_t* __restrict__ minor,
-                                                             uint32_t* hist, const uint32_t* ctl,
-                                                             uint32_t* flags0, DigitList digits) {
+// Workgroups of the histogram: each adds its 256 counts a pass to the same words, so few large ones.
+constexpr uint32_t kHistogramGroups = 256;
+constexpr uint32_t kHistogramThreads = 1024;
+
+__global__ void __launch_bounds__(kHistogramThreads) sort_histogram_kernel(const uint32_t* __restrict__ major,
+                                                                           const uint32_t* __restrict__ minor,
+                                                                           uint32_t* hist, const uint32_t* ctl,
+                                                                           uint32_t* flags0, DigitList digits) {
     __shared__ uint32_t s_hist[kSortMaxPasses][kSortBins];
     const uint32_t t = threadIdx.x;
-    for (uint32_t p = 0; p < digits.count; ++p) s_hist[p][t] = 0;
+    for (uint32_t k = t; k < digits.count * kSortBins; k += kHistogramThreads) (&s_hist[0][0])[k] = 0;
     __syncthreads();
     const uint32_t len = ctl[kCtlLen];
     const uint32_t base = ctl[kCtlBase];
@@ -74,8 +78,8 @@ __global__ void __launch_bounds__(256) sort_histogram_kernel(const uint32_t* __r
         uses_major |= digits.major[p] != 0;
         uses_minor |= digits.major[p] == 0;
     }
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = blockIdx.x * blockDim.x + t; i < len; i += stride) {
+    const uint32_t stride = gridDim.x * kHistogramThreads;
+    for (uint32_t i = blockIdx.x * kHistogramThreads + t; i < len; i += stride) {
         const uint32_t hi = uses_major ? major[base + i] : 0u;
         const uint32_t lo = uses_minor ? minor[base + i] : 0u;
         for (uint32_t p = 0; p < digits.count; ++p) {
@@ -84,69 +88,117 @@ __global__ void __launch_bounds__(256) sort_histogram_kernel(const uint32_t* __r
         }
     }
     __syncthreads();
-    for (uint32_t p = 0; p < digits.count; ++p) {
-        const uint32_t c = s_hist[p][t];
-        if (c) atomicAdd(&hist[p * kSortBins + t], c);
+    for (uint32_t k = t; k < digits.count * kSortBins; k += kHistogramThreads) {
+        const uint32_t c = (&s_hist[0][0])[k];
+        if (c) atomicAdd(&hist[k], c);
     }
     const uint32_t words = ceil_div(len, kSortMinTile) * kSortBins;
-    for (uint32_t i = blockIdx.x * blockDim.x + t; i < words; i += stride) flags0[i] = 0;
+    for (uint32_t i = blockIdx.x * kHistogramThreads + t; i < words; i += stride) flags0[i] = 0;
 }
 
-template <int ITEMS, bool MOVE_OTHER>
-__global__ void __launch_bounds__(256) sort_pass_kernel(
-    const uint32_t* __restrict__ in_sort, const uint32_t* __restrict__ in_other,
-    const uint32_t* __restrict__ in_pay, uint32_t* __restrict__ out_sort,
-    uint32_t* __restrict__ out_other, uint32_t* __restrict__ out_pay,
-    const uint32_t* __restrict__ hist_pass, uint32_t* flags_pass, uint32_t* flags_next,
-    uint32_t* ctl, uint32_t pass, uint32_t shift) {
+// A lane's rank among its wave's keys of digit d so far: the wave's earlier items (counted in
+// `counts`), then the lanes below it; the counts move on. Lanes and items in order are input order.
+__device__ __forceinline__ uint32_t wave_rank(uint32_t d, bool valid, uint32_t* counts) {
+    const uint64_t live = __ballot(valid);
+    uint32_t low = static_cast<uint32_t>(live), high = static_cast<uint32_t>(live >> 32);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        // all ones where the bit is set: peers keep the lanes whose bit is this lane's, a three-input
+        // bit operation for each half of the wave
+        const uint32_t mine = static_cast<uint32_t>(static_cast<int32_t>(d << (31 - b)) >> 31);
+        const uint64_t m = __ballot(mine != 0u);
+        low &= ~(static_cast<uint32_t>(m) ^ mine);
+        high &= ~(static_cast<uint32_t>(m >> 32) ^ mine);
+    }
+    const uint32_t before = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, 0u));
+    const uint32_t total = __popc(low) + __popc(high);
+    uint32_t prior = 0;
+    if (valid) prior = counts[d];
+    if (valid && before == 0) counts[d] = prior + total;
+    return prior + before;
+}
+
+// One lane of a short list's records moved to their places.
+template <int ITEMS>
+__device__ __forceinline__ void small_exchange(uint32_t (&v)[ITEMS], const uint32_t (&place)[ITEMS], uint32_t rounds,
+                                               uint32_t wave_first, uint32_t len, uint32_t* stage) {
+    const uint32_t lane = lane_id();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (i < static_cast<int>(rounds) && wave_first + i * kWave + lane < len) stage[place[i]] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t local = wave_first + i * kWave + lane;
+        if (i < static_cast<int>(rounds) && local < len) v[i] = stage[local];
+    }
+    __syncthreads();
+}
+
+// Predecessor words a digit's look-back keeps in flight: it walks back over the aggregates of the
+// tiles that run beside it, and one dependent read each (about 0.8 us across XCDs) would serialize
+// the tiles.
+constexpr int kLookBack = 8;
+
+struct PassArgs {
+    const uint32_t *in_sort, *in_other, *in_pay;
+    uint32_t *out_sort, *out_other, *out_pay;
+    const uint32_t* hist;
+    uint32_t *flags, *flags_next, *ctl;
+    uint32_t pass, shift;
+};
+
+// One digit pass over tiles of kSortThreads * ITEMS keys. A workgroup with no tile leaves at once,
+// and where every tile has a workgroup of its own, each takes one ticket only: the tickets are
+// atomics on one word, 15 to 20 ns each, and 1,024 workgroups' tickets cost an empty pass 18 us.
+// The three lanes go through one staging buffer in turn, and no load sits in a branch, so the other
+// lanes' words arrive while the keys are ranked. 3,000,017 records of three lanes: 46.6 -> 31.6 us a
+// pass (72 MB moved, 2.3 TB/s; what is left is the chain of a tile: ticket, load, ranking, look-back).
+template <int ITEMS, bool MOVE_OTHER, bool PAYLOAD>
+__device__ __forceinline__ void sort_pass(const PassArgs& a, uint32_t* s_stage) {
     constexpr int TILE = kSortThreads * ITEMS;
     constexpr int WAVES = kSortThreads / kWave;
-    __shared__ uint32_t s_key[TILE];
-    __shared__ uint32_t s_other[MOVE_OTHER ? TILE : 1];
-    __shared__ uint32_t s_pay[TILE];
     __shared__ uint32_t s_wave[WAVES][kSortBins];
     __shared__ uint32_t s_start[kSortBins];
     __shared__ uint32_t s_global[kSortBins];
-    __shared__ uint32_t s_digit_base[kSortBins];
     __shared__ uint32_t s_scan[WAVES];
     __shared__ uint32_t s_tile;
-
+    const uint32_t *__restrict__ in_sort = a.in_sort, *__restrict__ in_other = a.in_other, *__restrict__ in_pay = a.in_pay;
+    uint32_t *__restrict__ out_sort = a.out_sort, *__restrict__ out_other = a.out_other, *__restrict__ out_pay = a.out_pay;
+    uint32_t *flags_pass = a.flags, *flags_next = a.flags_next, *ctl = a.ctl;
+    const uint32_t pass = a.pass, shift = a.shift;
     const uint32_t t = threadIdx.x;
     const uint32_t lane = lane_id();
     const uint32_t wave = t / kWave;
     const uint32_t len = ctl[kCtlLen];
     const uint32_t base = ctl[kCtlBase];
     const uint32_t ntiles = ceil_div(len, TILE);
-    const uint64_t below = (1ull << lane) - 1ull;
+    if (blockIdx.x >= ntiles) return;
 
-    bool based = false;
+    // Global start of every digit: exclusive scan of this pass's histogram.
+    const uint32_t digit_base = block_exclusive_sum<kSortThreads>(t < kSortBins ? a.hist[t] : 0u, s_scan, nullptr);
     for (;;) {
         if (t == 0) s_tile = atomicAdd(&ctl[kCtlTiles + pass], 1u);
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) s_wave[w][t] = 0;
+        for (uint32_t k = t; k < WAVES * kSortBins; k += kSortThreads) (&s_wave[0][0])[k] = 0u;
         __syncthreads();
         const uint32_t tile = s_tile;
         if (tile >= ntiles) break;
-        if (!based) {
-            // Global start of every digit: exclusive scan of this pass's histogram (only
-            // workgroups that hold a tile need it).
-            s_digit_base[t] = block_exclusive_sum<kSortThreads>(hist_pass[t], s_scan, nullptr);
-            based = true;
-        }
         const uint32_t first = tile * TILE;
         const uint32_t tile_n = min(static_cast<uint32_t>(TILE), len - first);
-        if (flags_next) flags_next[tile * kSortBins + t] = 0;
+        if (flags_next && t < kSortBins) flags_next[tile * kSortBins + t] = 0;
 
-        uint32_t key[ITEMS], other[ITEMS], pay[ITEMS], rank[ITEMS];
+        uint32_t key[ITEMS], other[ITEMS], pay[ITEMS], place[ITEMS];
         const uint32_t wave_first = wave * (ITEMS * kWave);
+        // Lanes past the tile's end read its last record again, so that no load sits in a branch: the
+        // other lanes' words stay in flight while the keys are ranked.
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) key[i] = in_sort[base + first + min(wave_first + i * kWave + lane, tile_n - 1u)];
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t local = wave_first + i * kWave + lane;
-            const bool valid = local < tile_n;
-            const uint32_t at = base + first + local;
-            key[i] = valid ? in_sort[at] : 0u;
-            pay[i] = valid ? in_pay[at] : 0u;
-            if (MOVE_OTHER) other[i] = valid ? in_other[at] : 0u;
+            const uint32_t from = base + first + min(wave_first + i * kWave + lane, tile_n - 1u);
+            if (PAYLOAD) pay[i] = in_pay[from];
+            if (MOVE_OTHER) other[i] = in_other[from];
         }
         // Rank within the wave: items in order, lanes in order, which is input order.
 #pragma unroll
@@ -154,87 +206,205 @@ __global__ void __launch_bounds__(256) sort_pass_kernel(
             const uint32_t local = wave_first + i * kWave + lane;
             const bool valid = local < tile_n;
             const uint32_t d = (key[i] >> shift) & 0xFFu;
-            uint64_t peers = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (d >> b) & 1u;
-                const uint64_t m = __ballot(bit);
-                peers &= bit ? m : ~m;
-            }
-            const uint32_t before = __popcll(peers & below);
-            const uint32_t total = __popcll(peers);
-            uint32_t prior = 0;
-            if (valid) prior = s_wave[wave][d];
-            if (valid && before == 0) s_wave[wave][d] = prior + total;
-            rank[i] = prior + before;
+            place[i] = wave_rank(d, valid, s_wave[wave]);
         }
         __syncthreads();
 
         // Digit t: per-wave offsets, tile count, tile-local start.
         uint32_t count = 0;
+        if (t < kSortBins) {
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const uint32_t c = s_wave[w][t];
-            s_wave[w][t] = count;
-            count += c;
+            for (int w = 0; w < WAVES; ++w) {
+                const uint32_t c = s_wave[w][t];
+                s_wave[w][t] = count;
+                count += c;
+            }
+            // the tile's counts as early as possible: later tiles wait for them
+            atomic_store_agent(&flags_pass[tile * kSortBins + t], (tile == 0u ? kFlagPrefix : kFlagAggregate) | count);
         }
         const uint32_t start = block_exclusive_sum<kSortThreads>(count, s_scan, nullptr);
-        s_start[t] = start;
-
-        // Decoupled look-back over earlier tiles for digit t.
-        uint32_t* mine = &flags_pass[tile * kSortBins + t];
-        uint32_t excl = 0;
-        if (tile == 0) {
-            atomic_store_agent(mine, kFlagPrefix | count);
-        } else {
-            atomic_store_agent(mine, kFlagAggregate | count);
-            int64_t j = static_cast<int64_t>(tile) - 1;
+        if (t < kSortBins) s_start[t] = start;
+        __syncthreads();
+        // the keys to their local places, which do not need the look-back
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t local = wave_first + i * kWave + lane;
+            if (local < tile_n) {
+                const uint32_t d = (key[i] >> shift) & 0xFFu;
+                place[i] += s_start[d] + s_wave[wave][d];
+                s_stage[place[i]] = key[i];
+            }
+        }
+        if (t < kSortBins) {
+            // Decoupled look-back over earlier tiles for digit t, kLookBack of them at a time.
+            uint32_t excl = 0;
             uint32_t spins = 0;
-            while (j >= 0) {
-                const uint32_t v = atomic_load_agent(&flags_pass[j * kSortBins + t]);
-                const uint32_t status = v >> 30;
-                if (status == 0) {
+            bool open = tile != 0u;
+            int64_t j = static_cast<int64_t>(tile) - 1;
+            while (open) {
+                uint32_t v[kLookBack];
+#pragma unroll
+                for (int b = 0; b < kLookBack; ++b) {
+                    v[b] = j >= b ? atomic_load_agent(&flags_pass[(j - b) * kSortBins + t]) : kFlagPrefix;
+                }
+                bool waits = false;
+#pragma unroll
+                for (int b = 0; b < kLookBack; ++b) {
+                    if (!open || waits) continue;
+                    const uint32_t status = v[b] >> 30;
+                    if (status == 0u) {
+                        waits = true;
+                        continue;
+                    }
+                    excl += v[b] & kFlagValue;
+                    --j;
+                    if (status == 2u) open = false;
+                }
+                if (waits) {
                     if (++spins > kSpinLimit) {
                         atomicOr(&ctl[kCtlError], 1u);
                         atomicAdd(&g_sort_faults, 1u);
                         break;
                     }
                     __builtin_amdgcn_s_sleep(1);
-                    continue;
                 }
-                excl += v & kFlagValue;
-                if (status == 2) break;
-                --j;
             }
-            atomic_store_agent(mine, kFlagPrefix | ((excl + count) & kFlagValue));
+            if (tile != 0u) {
+                atomic_store_agent(&flags_pass[tile * kSortBins + t], kFlagPrefix | ((excl + count) & kFlagValue));
+            }
+            s_global[t] = digit_base + excl - start;
         }
-        s_global[t] = s_digit_base[t] + excl - start;
         __syncthreads();
+        // Where the staged record t + k * kSortThreads goes. Always below len when the look-back
+        // completed; the guard keeps a timed-out look-back (ctl error word set) from writing outside
+        // the stream.
+        uint32_t at[ITEMS];
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t j = t + k * kSortThreads;
+            at[k] = len;
+            if (j < tile_n) {
+                const uint32_t staged = s_stage[j];
+                at[k] = s_global[(staged >> shift) & 0xFFu] + j;
+                if (at[k] < len) out_sort[base + at[k]] = staged;
+            }
+        }
+        if (PAYLOAD) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                if (wave_first + i * kWave + lane < tile_n) s_stage[place[i]] = pay[i];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < ITEMS; ++k) {
+                if (at[k] < len) out_pay[base + at[k]] = s_stage[t + k * kSortThreads];
+            }
+        }
+        if (MOVE_OTHER) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                if (wave_first + i * kWave + lane < tile_n) s_stage[place[i]] = other[i];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < ITEMS; ++k) {
+                if (at[k] < len) out_other[base + at[k]] = s_stage[t + k * kSortThreads];
+            }
+        }
+        if (gridDim.x >= ntiles) break;  // a workgroup per tile: this was its only one
+        __syncthreads();
+    }
+}
 
+// Streams of up to this many live records use 8 keys a lane also where the capacity (all that the
+// host knows) asks for 16: 200,000 records in a stream of 4,194,304 took 119 us with 16 and 93 us with
+// 8, 1,500,000 165 and 162 us, 3,000,017 208 and 237 us.
+constexpr uint32_t kNarrowBelow = 1572864u;
+
+template <int ITEMS, bool MOVE_OTHER, bool PAYLOAD>
+__global__ void __launch_bounds__(kSortThreads, 4) sort_pass_kernel(PassArgs a) {
+    __shared__ uint32_t s_stage[kSortThreads * ITEMS];
+    if (ITEMS > 8 && a.ctl[kCtlLen] <= kNarrowBelow) sort_pass<8, MOVE_OTHER, PAYLOAD>(a, s_stage);
+    else sort_pass<ITEMS, MOVE_OTHER, PAYLOAD>(a, s_stage);
+}
+
+// A short list sorted whole by one workgroup: every digit pass ranks the records where they are in
+// registers and exchanges them through LDS, so nothing but the input and the result touches memory,
+// in one launch instead of 2 + passes (+ 1 for an odd count). What bounds it is the latency of a
+// pass (six barriers, the ranking's ballots and the exchange).
+template <int ITEMS>
+__global__ void __launch_bounds__(kSmallThreads) sort_small_kernel(uint32_t* major, uint32_t* minor, uint32_t* payload,
+                                                                   const uint32_t* d_count, const uint32_t* d_base,
+                                                                   uint32_t capacity, DigitList digits) {
+    constexpr int WAVES = kSmallThreads / kWave;
+    __shared__ uint32_t s_stage[kSmallThreads * ITEMS];
+    __shared__ uint32_t s_wave[WAVES][kSortBins];
+    __shared__ uint32_t s_start[kSortBins];
+    __shared__ uint32_t s_scan[WAVES];
+    const uint32_t t = threadIdx.x;
+    const uint32_t lane = lane_id();
+    const uint32_t wave = t / kWave;
+    uint32_t base = d_base ? d_base[0] : 0u;
+    if (base > capacity) base = capacity;
+    const uint32_t count = d_count ? d_count[0] : capacity;
+    const uint32_t len = min(count, capacity - base);
+    // rounds of a wave: the records spread evenly over the waves, a wave's ones consecutive
+    const uint32_t rounds = ceil_div(len, kSmallThreads);
+    const uint32_t wave_first = wave * rounds * kWave;
+    if (len == 0u) return;
+    uint32_t rec_major[ITEMS], rec_minor[ITEMS], rec_pay[ITEMS], place[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        rec_major[i] = rec_minor[i] = rec_pay[i] = place[i] = 0u;
+        if (i >= static_cast<int>(rounds)) continue;
+        const uint32_t from = base + min(wave_first + i * kWave + lane, len - 1u);  // past the end: the last again
+        rec_major[i] = major[from];
+        if (minor) rec_minor[i] = minor[from];
+        if (payload) rec_pay[i] = payload[from];
+    }
+    for (uint32_t p = 0; p < digits.count; ++p) {
+        const uint32_t shift = digits.shift[p];
+        const bool on_major = digits.major[p] != 0u;
+        for (uint32_t k = t; k < WAVES * kSortBins; k += kSmallThreads) (&s_wave[0][0])[k] = 0u;
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t local = wave_first + i * kWave + lane;
-            if (local < tile_n) {
-                const uint32_t d = (key[i] >> shift) & 0xFFu;
-                const uint32_t lp = s_start[d] + s_wave[wave][d] + rank[i];
-                s_key[lp] = key[i];
-                s_pay[lp] = pay[i];
-                if (MOVE_OTHER) s_other[lp] = other[i];
+            if (i >= static_cast<int>(rounds)) continue;
+            const uint32_t d = ((on_major ? rec_major[i] : rec_minor[i]) >> shift) & 0xFFu;
+            place[i] = wave_rank(d, wave_first + i * kWave + lane < len, s_wave[wave]);
+        }
+        __syncthreads();
+        uint32_t total = 0;
+        if (t < kSortBins) {
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) {
+                const uint32_t c = s_wave[w][t];
+                s_wave[w][t] = total;
+                total += c;
             }
         }
+        const uint32_t start = block_exclusive_sum<kSmallThreads>(total, s_scan, nullptr);
+        if (t < kSortBins) s_start[t] = start;
         __syncthreads();
-        for (uint32_t j = t; j < tile_n; j += kSortThreads) {
-            const uint32_t k = s_key[j];
-            const uint32_t place = s_global[(k >> shift) & 0xFFu] + j;
-            // Always below len when the look-back completed; the guard keeps a timed-out
-            // look-back (ctl error word set) from writing outside the stream.
-            if (place >= len) continue;
-            const uint32_t at = base + place;
-            out_sort[at] = k;
-            out_pay[at] = s_pay[j];
-            if (MOVE_OTHER) out_other[at] = s_other[j];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (i >= static_cast<int>(rounds)) continue;
+            const uint32_t d = ((on_major ? rec_major[i] : rec_minor[i]) >> shift) & 0xFFu;
+            place[i] += s_start[d] + s_wave[wave][d];
         }
-        __syncthreads();
+        small_exchange<ITEMS>(rec_major, place, rounds, wave_first, len, s_stage);
+        if (minor) small_exchange<ITEMS>(rec_minor, place, rounds, wave_first, len, s_stage);
+        if (payload) small_exchange<ITEMS>(rec_pay, place, rounds, wave_first, len, s_stage);
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t local = wave_first + i * kWave + lane;
+        if (i >= static_cast<int>(rounds) || local >= len) continue;
+        major[base + local] = rec_major[i];
+        if (minor) minor[base + local] = rec_minor[i];
+        if (payload) payload[base + local] = rec_pay[i];
     }
 }
 
@@ -248,7 +418,7 @@ __global__ void __launch_bounds__(256) sort_copy_kernel(const uint32_t* __restri
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < len; i += stride) {
         to_major[base + i] = from_major[base + i];
-        to_pay[base + i] = from_pay[base + i];
+        if (to_pay) to_pay[base + i] = from_pay[base + i];
         if (to_minor) to_minor[base + i] = from_minor[base + i];
     }
 }
@@ -261,6 +431,11 @@ DigitList make_list(const SortDigit* digits, uint32_t passes) {
         list.shift[p] = digits[p].shift;
     }
     return list;
+}
+
+uint32_t histogram_groups(uint32_t capacity) {
+    const uint32_t want = ceil_div(capacity ? capacity : 1u, 4u * kHistogramThreads);
+    return want < kHistogramGroups ? want : kHistogramGroups;
 }
 
 uint32_t stream_groups(uint32_t capacity) {
@@ -316,7 +491,7 @@ int sort_histogram(hipStream_t stream, const uint32_t* major, const uint32_t* mi
                    uint32_t capacity, const SortNames& names) {
     {
         ProfileScope scope(names.histogram, stream);
-        sort_histogram_kernel<<<stream_groups(capacity), 256, 0, stream>>>(
+        sort_histogram_kernel<<<histogram_groups(capacity), kHistogramThreads, 0, stream>>>(
             major, minor, s.hist, s.ctl, s.flags, make_list(digits, passes));
     }
     DYN_LAUNCHED("sort_histogram_kernel");
@@ -327,16 +502,14 @@ template <int ITEMS>
 static int launch_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* payload,
                          const SortScratch& s, const SortDigit* digits, uint32_t passes,
                          uint32_t capacity, const SortNames& names, uint32_t group_cap) {
-    constexpr int TILE = kSortThreads * ITEMS;
-    const uint32_t tiles = ceil_div(capacity ? capacity : 1u, TILE);
-    // Persistent workgroups take tiles in order (any count makes progress: a tile's look-back
-    // only waits on earlier tiles, which running groups hold).
+    // Persistent workgroups take tiles in order (any count makes progress: a tile's look-back only
+    // waits on earlier tiles, which running groups hold). The tiles of 8 keys a lane: a stream with
+    // few live records takes those whatever ITEMS is.
+    constexpr uint32_t kTile = kSortThreads * 8;
+    static_assert(kTile >= kSortMinTile, "the look-back words are laid out for the narrowest tiling");
+    const uint32_t tiles = ceil_div(capacity ? capacity : 1u, kTile);
     const uint32_t groups = tiles < group_cap ? tiles : group_cap;
-    // The look-back words are laid out for the narrowest tiling, so every tiling fits.
     const size_t flag_stride = static_cast<size_t>(s.max_tiles) * kSortBins;
-    if (static_cast<size_t>(tiles) * kSortBins > flag_stride) {
-        return fail(DYN_E_INVALID, "sort: tiling exceeds the look-back layout");
-    }
     uint32_t* src[3] = {major, minor, payload};
     uint32_t* dst[3] = {s.major, s.minor, s.payload};
     const bool carry_minor = minor != nullptr;
@@ -349,20 +522,15 @@ static int launch_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, u
         uint32_t* out_other = on_major ? dst[1] : dst[0];
         uint32_t* flags_pass = s.flags + p * flag_stride;
         uint32_t* flags_next = (p + 1 < passes) ? s.flags + (p + 1) * flag_stride : nullptr;
-        if (carry_minor) {
-            {
-                ProfileScope scope(names.pass, stream);
-                sort_pass_kernel<ITEMS, true><<<groups, kSortThreads, 0, stream>>>(
-                    in_sort, in_other, src[2], out_sort, out_other, dst[2], s.hist + p * kSortBins,
-                    flags_pass, flags_next, s.ctl, p, digits[p].shift);
-            }
-        } else {
-            {
-                ProfileScope scope(names.pass, stream);
-                sort_pass_kernel<ITEMS, false><<<groups, kSortThreads, 0, stream>>>(
-                    in_sort, nullptr, src[2], out_sort, nullptr, dst[2], s.hist + p * kSortBins,
-                    flags_pass, flags_next, s.ctl, p, digits[p].shift);
-            }
+        {
+            ProfileScope scope(names.pass, stream);
+            const PassArgs args{in_sort, carry_minor ? in_other : nullptr, src[2],
+                                out_sort, carry_minor ? out_other : nullptr, dst[2],
+                                s.hist + p * kSortBins, flags_pass, flags_next, s.ctl, p, digits[p].shift};
+            auto launch = [&](auto kernel) { kernel<<<groups, kSortThreads, 0, stream>>>(args); };
+            if (carry_minor && payload) launch(sort_pass_kernel<ITEMS, true, true>);
+            else if (carry_minor) launch(sort_pass_kernel<ITEMS, true, false>);
+            else launch(sort_pass_kernel<ITEMS, false, true>);
         }
         DYN_LAUNCHED("sort_pass_kernel");
         for (int l = 0; l < 3; ++l) {
@@ -384,8 +552,8 @@ static int launch_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, u
 
 // ---- tiling: the autotuner's table ---------------------------------------------------------------
 //
-// A pass's tiling is keys per lane (8: 2048-key tiles, 16: 4096-key tiles) and the cap on its
-// persistent workgroups. The tuner times every candidate on the device for a capacity bucket
+// A pass's tiling is keys per lane (8: 4096-key tiles; 16: 8192-key tiles, for streams with enough live
+// records) and the cap on its persistent workgroups. The tuner times every candidate on the device for a capacity bucket
 // (ceil(log2(capacity))) and keeps the fastest per (device, bucket); untuned buckets use the
 // default: narrow tiles up to 2^21 keys (more of the chip busy on shorter streams), 1024 groups
 // (about four per CU).
@@ -427,6 +595,24 @@ int passes_with(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* 
                 SortTiling t) {
     if (t.items == 8u) return launch_passes<8>(stream, major, minor, payload, s, digits, passes, capacity, names, t.groups);
     return launch_passes<16>(stream, major, minor, payload, s, digits, passes, capacity, names, t.groups);
+}
+
+int sort_small(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* payload, const uint32_t* d_count,
+               const uint32_t* d_base, uint32_t capacity, const SortDigit* digits, uint32_t passes,
+               const SortNames& names) {
+    if (capacity > kSortSmall) return fail(DYN_E_INVALID, "sort: too many records for one workgroup");
+    const DigitList list = make_list(digits, passes);
+    {
+        ProfileScope scope(names.pass, stream);
+        auto launch = [&](auto kernel) {
+            kernel<<<1, kSmallThreads, 0, stream>>>(major, minor, payload, d_count, d_base, capacity, list);
+        };
+        if (capacity <= 2u * kSmallThreads) launch(sort_small_kernel<2>);
+        else if (capacity <= 4u * kSmallThreads) launch(sort_small_kernel<4>);
+        else launch(sort_small_kernel<8>);
+    }
+    DYN_LAUNCHED("sort_small_kernel");
+    return DYN_OK;
 }
 
 int sort_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, uint32_t* payload,
@@ -615,6 +801,9 @@ int dyn_sort_pairs(void* stream, uint32_t* d_major, uint32_t* d_minor, uint32_t*
     SortDigit digits[kSortMaxPasses];
     sort_digits(major_words, minor_words, digits);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (capacity <= kSortSmall) {
+        return sort_small(st, d_major, d_minor, d_payload, d_count, d_base, capacity, digits, passes);
+    }
     DYN_TRY(sort_prepare(st, s, d_count, d_base, capacity));
     DYN_TRY(sort_histogram(st, d_major, d_minor, s, digits, passes, capacity));
     DYN_TRY(sort_passes(st, d_major, d_minor, d_payload, s, digits, passes, capacity));
