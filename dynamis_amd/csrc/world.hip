@@ -88,13 +88,12 @@ struct W {
     dyn_contact* raw;
     uint32_t* valid;
     uint8_t* pkind;        // per convex pair: the unordered class of its two shape kinds
-    uint32_t* worklist;    // convex pairs grouped by kind class (k_class_scatter)
+    uint32_t* worklist;    // pair lists (WorkList): every candidate pair by kind class, then GJK's open
+                           // pairs, then the penetrating pairs (front) and the hits (from the end)
     uint32_t* class_hist;  // per kind class and block of pairs: count, then offset in the class;
                            // then the classes' totals
-    uint32_t* work_total;  // device words: entries on the worklist of modes 0-2, the hull-class GJK pairs,
-                           // the resumed GJK pairs (mode 4), the EPA polytopes given a wave, the
-                           // candidate pairs (mode 6)
-    uint32_t* work_minor;  // the sort's unused minor lane
+    uint32_t* work_total;  // device words: the lists' lengths (WorkTotal)
+    uint32_t* work_minor;  // pair lists: GJK's pairs, then the wave EPA's (front), the plane pairs (from the end)
     uint32_t* dest;
     dyn_contact* contacts;
     uint2* ckeys;          // per contact: its collider pair (a, b), the key the relay searches
@@ -415,7 +414,6 @@ constexpr uint32_t kPairEpa = 3;      // GJK found it penetrating; simplex parke
 constexpr uint32_t kPairEpaDone = 4;  // EPA result parked for k_narrow_finish
 constexpr uint32_t kPairHit = 5;      // GJK hit within the margin parked for k_narrow_finish
 constexpr uint32_t kPairPlane = 6;    // plane against a hull or cylinder, for k_narrow_finish
-constexpr uint32_t kPairGjkResume = 7;  // GJK's state parked for k_narrow_convex_resume
 constexpr uint32_t kPairEpaWave = 8;    // EPA result of the wave kernel parked for k_narrow_finish_tail
 
 // Material, identity and anchors of a generated manifold (narrowphase.wgsl:665-684).
@@ -483,13 +481,87 @@ __device__ __forceinline__ bool bounds_apart(const Shape& a, const Shape& b, con
            amn.y - bmx.y > reach || bmn.z - amx.z > reach || amn.z - bmx.z > reach;
 }
 
-// ---- convex worklists: pairs grouped by the kinds of their shapes ---------------------------
+// ---- pair lists: every candidate pair grouped by the kinds of its shapes, and the convex path's ----
+//
+// k_class_* group all candidate pairs by kind class, so that a wave of k_narrow runs one generator.
+// From there each kernel hands its pairs on by appending them to the next one's list (BlockLists): a
+// workgroup adds its takers with one atomic, so lists keep their chunks of one class, and the marks of
+// all pairs need not be counted, scanned and scattered again for every kernel (12 launches and 120 us
+// of a 755 us pass over 114,000 pairs). Two arrays of pair_cap words hold them all: no pair is on two
+// lists that share an array at one time.
+
+// Words of work_total. kTotalGjk to kTotalEpaWave are also what dyn_world_read_work reports (the
+// second as all manifold pairs).
+enum WorkTotal : uint32_t {
+    kTotalGjk = 0,      // work_minor, front
+    kTotalPlane = 1,    // work_minor, from the end
+    kTotalEpa = 2,      // worklist, front
+    kTotalHull = 3,     // GJK pairs of the hull classes
+    kTotalResume = 4,   // worklist, front (until k_work_split)
+    kTotalEpaWave = 5,  // work_minor, front (after k_work_split)
+    kTotalAll = 6,      // worklist (until k_narrow has read it)
+    kTotalHit = 7,      // worklist, from the end
+    kTotalWords = 8
+};
+constexpr uint32_t kNoList = 0xFFFFFFFFu;
+
+struct ListTarget {
+    uint32_t* total;
+    uint32_t* list;
+    uint32_t end;  // non-zero: entries go down from list[end - 1]
+};
+
+// A workgroup's takers for kLists lists, appended by the last of its waves to arrive (no wave waits).
+template <uint32_t kLists>
+struct BlockLists {
+    uint32_t n[kLists], arrived, hull;
+    uint32_t item[kLists][kThreads];
+
+    __device__ __forceinline__ void begin() {
+        if (threadIdx.x < kLists) n[threadIdx.x] = 0u;
+        if (threadIdx.x == 0) arrived = hull = 0u;
+        __syncthreads();
+    }
+    // Every lane of the workgroup calls it once, with the list its pair goes to or kNoList.
+    __device__ __forceinline__ void finish(uint32_t list, uint32_t index, bool is_hull, uint32_t* hull_total,
+                                           const ListTarget (&targets)[kLists]) {
+        const uint32_t lane = lane_id();
+#pragma unroll
+        for (uint32_t k = 0; k < kLists; ++k) {
+            const uint64_t takers = __ballot(list == k);
+            if (takers == 0ull) continue;
+            uint32_t at = 0;
+            if (lane == 0u) at = atomicAdd(&n[k], static_cast<uint32_t>(__popcll(takers)));
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (list == k) item[k][at + __popcll(takers & ((1ull << lane) - 1ull))] = index;
+        }
+        const uint64_t hulls = __ballot(is_hull);
+        if (lane == 0u && hulls) atomicAdd(&hull, static_cast<uint32_t>(__popcll(hulls)));
+        __threadfence_block();
+        uint32_t before = 0;
+        if (lane == 0u) before = atomicAdd(&arrived, 1u);
+        if (__builtin_amdgcn_readfirstlane(before) + 1u != kThreads / kWave) return;
+        __threadfence_block();
+#pragma unroll
+        for (uint32_t k = 0; k < kLists; ++k) {
+            const uint32_t count = n[k];
+            if (count == 0u) continue;
+            uint32_t first = 0;
+            if (lane == 0u) first = atomicAdd(targets[k].total, count);
+            first = __builtin_amdgcn_readfirstlane(first);
+            for (uint32_t j = lane; j < count; j += kWave) {
+                const uint32_t at = first + j;
+                targets[k].list[targets[k].end ? targets[k].end - 1u - at : at] = item[k][j];
+            }
+        }
+        if (lane == 0u && hull_total && hull) atomicAdd(hull_total, hull);
+    }
+};
 
 constexpr uint32_t kClasses = 32;       // unordered pairs of 7 kind slots (28) and spare
 constexpr uint32_t kHullClasses = 21;   // the classes of pairs with a hull come last, from here
 constexpr uint32_t kClassItems = 16;
 constexpr uint32_t kClassBlock = kThreads * kClassItems;  // 4096 pairs per block
-constexpr uint32_t kNoClass = 0xFFu;
 
 __device__ __forceinline__ uint32_t kind_slot(uint32_t kind) {
     switch (kind) {
@@ -516,21 +588,14 @@ __device__ __forceinline__ uint8_t kind_class(uint32_t first_kind, uint32_t seco
     return static_cast<uint8_t>(a * 6u - (a * (a - 1u)) / 2u + (b - a));
 }
 
-// The pairs a narrowphase kernel takes: kPairGjk (mode 0), the pairs k_narrow_finish completes
-// (mode 1), kPairEpa (mode 2), kPairGjkResume (mode 4), every candidate pair (mode 6, for
-// k_narrow; its marks are not written yet).
-constexpr uint32_t kWorkAllPairs = 6;
-__device__ __forceinline__ uint32_t work_class(const W& w, uint32_t index, uint32_t mode) {
-    if (mode == kWorkAllPairs) return static_cast<uint32_t>(w.pkind[index]);
-    const uint32_t v = w.valid[index];
-    const bool take = mode == 0u   ? v == kPairGjk
-                      : mode == 1u ? (v == kPairEpaDone || v == kPairHit || v == kPairPlane)
-                      : mode == 4u ? v == kPairGjkResume
-                                   : v == kPairEpa;
-    return take ? static_cast<uint32_t>(w.pkind[index]) : kNoClass;
+// A candidate pair's kind class (class 0 for pairs naming colliders outside the records).
+__device__ __forceinline__ uint32_t pair_class(const W& w, uint32_t index) {
+    const uint32_t fs = w.pmaj[index], ss = w.pmin[index];
+    return (fs < w.k && ss < w.k) ? kind_class(w.co[fs].kind, w.co[ss].kind) : 0u;
 }
 
-__global__ void __launch_bounds__(kThreads) k_class_count(W w, uint32_t mode) {
+// Every candidate pair's class, and each block's counts of them.
+__global__ void __launch_bounds__(kThreads) k_class_count(W w) {
     __shared__ uint32_t hist[kClasses];
     if (threadIdx.x < kClasses) hist[threadIdx.x] = 0u;
     __syncthreads();
@@ -539,8 +604,9 @@ __global__ void __launch_bounds__(kThreads) k_class_count(W w, uint32_t mode) {
     for (uint32_t j = 0; j < kClassItems; ++j) {
         const uint32_t index = base + j * kThreads + threadIdx.x;
         if (index >= live) break;
-        const uint32_t c = work_class(w, index, mode);
-        if (c != kNoClass) atomicAdd(&hist[c], 1u);
+        const uint32_t c = pair_class(w, index);
+        w.pkind[index] = static_cast<uint8_t>(c);
+        atomicAdd(&hist[c], 1u);
     }
     __syncthreads();
     if (threadIdx.x < kClasses) w.class_hist[threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
@@ -548,7 +614,8 @@ __global__ void __launch_bounds__(kThreads) k_class_count(W w, uint32_t mode) {
 
 // One workgroup per kind class: the class's block counts become offsets within the class, and
 // the class's total goes to class_hist[kClasses * blocks + class].
-__global__ void __launch_bounds__(1024) k_class_scan(uint32_t* class_hist, uint32_t blocks) {
+__global__ void __launch_bounds__(1024) k_class_scan(uint32_t* class_hist, uint32_t blocks, uint32_t* totals) {
+    if (blockIdx.x == 0 && threadIdx.x < kTotalWords) totals[threadIdx.x] = 0u;
     __shared__ uint32_t s_scan[1024 / kWave];
     __shared__ uint32_t s_carry;
     uint32_t* row = class_hist + static_cast<size_t>(blockIdx.x) * blocks;
@@ -569,7 +636,7 @@ __global__ void __launch_bounds__(1024) k_class_scan(uint32_t* class_hist, uint3
 // After k_class_scan: each block places its pairs of every class at the class's start (the
 // totals of the classes before it) plus its offset within the class (in any order within the
 // block: every pair's result goes to its own slot); block 0 writes the worklist's length.
-__global__ void __launch_bounds__(kThreads) k_class_scatter(W w, uint32_t mode) {
+__global__ void __launch_bounds__(kThreads) k_class_scatter(W w) {
     static_assert(kClasses <= kWave, "one wave sums the class totals");
     __shared__ uint32_t cursor[kClasses];
     if (threadIdx.x < kWave) {
@@ -577,7 +644,7 @@ __global__ void __launch_bounds__(kThreads) k_class_scatter(W w, uint32_t mode) 
         const uint32_t total = c < kClasses ? w.class_hist[static_cast<size_t>(kClasses) * gridDim.x + c] : 0u;
         const uint32_t inclusive = wave_inclusive_sum(total);
         if (c < kClasses) cursor[c] = inclusive - total + w.class_hist[c * gridDim.x + blockIdx.x];
-        if (blockIdx.x == 0u && c == kWave - 1u) w.work_total[mode] = inclusive;
+        if (blockIdx.x == 0u && c == kWave - 1u) w.work_total[kTotalAll] = inclusive;
     }
     __syncthreads();
     const uint32_t live = min(*cw(w.counters, DYN_COUNTER_PAIRS), w.pair_cap);
@@ -585,43 +652,53 @@ __global__ void __launch_bounds__(kThreads) k_class_scatter(W w, uint32_t mode) 
     for (uint32_t j = 0; j < kClassItems; ++j) {
         const uint32_t index = base + j * kThreads + threadIdx.x;
         if (index >= live) break;
-        const uint32_t c = work_class(w, index, mode);
-        if (c != kNoClass) w.worklist[atomicAdd(&cursor[c], 1u)] = index;
+        w.worklist[atomicAdd(&cursor[w.pkind[index]], 1u)] = index;
     }
 }
 
-// Analytic pairs; convex-path pairs are marked for the kernels below.
-// Every candidate pair's kind class (pairs naming colliders outside the records: class 0), so
-// k_narrow's worklist groups its pairs by kind and a wave runs one generator.
-__global__ void __launch_bounds__(kThreads) k_pair_class(W w) {
-    const uint32_t index = blockIdx.x * blockDim.x + threadIdx.x;
+// The three passes above in one workgroup, for small pair capacities.
+constexpr uint32_t kClassSmall = 16384;
+__global__ void __launch_bounds__(1024) k_class_small(W w) {
+    __shared__ uint32_t cursor[kClasses];
+    const uint32_t t = threadIdx.x;
+    if (t < kClasses) cursor[t] = 0u;
+    if (t < kTotalWords) w.work_total[t] = 0u;
+    __syncthreads();
     const uint32_t live = min(*cw(w.counters, DYN_COUNTER_PAIRS), w.pair_cap);
-    if (index >= live) return;
-    const uint32_t fs = w.pmaj[index], ss = w.pmin[index];
-    w.pkind[index] = (fs < w.k && ss < w.k) ? kind_class(w.co[fs].kind, w.co[ss].kind) : 0u;
+    for (uint32_t index = t; index < live; index += 1024u) {
+        const uint32_t c = pair_class(w, index);
+        w.pkind[index] = static_cast<uint8_t>(c);
+        atomicAdd(&cursor[c], 1u);
+    }
+    __syncthreads();
+    if (t < kWave) {
+        const uint32_t total = t < kClasses ? cursor[t] : 0u;
+        const uint32_t inclusive = wave_inclusive_sum(total);
+        if (t < kClasses) cursor[t] = inclusive - total;
+        if (t == 0u) w.work_total[kTotalAll] = live;
+    }
+    __syncthreads();
+    for (uint32_t index = t; index < live; index += 1024u) w.worklist[atomicAdd(&cursor[w.pkind[index]], 1u)] = index;
 }
 
-// One thread per candidate pair of the kind-grouped worklist (every pair's result goes to its
-// own slot, so the order changes nothing).
-__global__ void __launch_bounds__(kThreads) k_narrow(W w) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= w.work_total[kWorkAllPairs]) return;
-    const uint32_t index = w.worklist[t];
+// An analytic pair's manifold; a convex-path pair's list: 0 GJK's, 1 the plane pairs'.
+__device__ __forceinline__ uint32_t narrow_pair(const W& w, uint32_t index) {
     w.valid[index] = kPairNone;
     const uint32_t fs = w.pmaj[index], ss = w.pmin[index];
     uint32_t fb, sb;
-    if (!pair_admitted(w, fs, ss, &fb, &sb)) return;
+    if (!pair_admitted(w, fs, ss, &fb, &sb)) return kNoList;
     const dyn_collider fc = w.co[fs], sc = w.co[ss];
     const Body first = load_body(w, fb), second = load_body(w, sb);
     const float margin = pair_margin(w, first, second);
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
-    if (convex_path(fc, sc)) {  // pkind holds the pair's class (k_pair_class)
+    if (convex_path(fc, sc)) {
         if (fc.kind == DYN_SHAPE_PLANE || sc.kind == DYN_SHAPE_PLANE) {
             w.valid[index] = kPairPlane;
-        } else if (!bounds_apart(world_collider(first.s, fc), world_collider(second.s, sc), shapes, margin)) {
-            w.valid[index] = kPairGjk;
+            return 1u;
         }
-        return;
+        if (bounds_apart(world_collider(first.s, fc), world_collider(second.s, sc), shapes, margin)) return kNoList;
+        w.valid[index] = kPairGjk;
+        return 0u;
     }
     Manifold m;
     m.count = 0;
@@ -647,8 +724,25 @@ __global__ void __launch_bounds__(kThreads) k_narrow(W w) {
             mirror(m);
         } else if (a == DYN_SHAPE_CAPSULE && b == DYN_SHAPE_CAPSULE) capsule_capsule(m, first, fc, second, sc, margin);
     }
-    if (m.count == 0u) return;
-    write_contact(w, index, fs, ss, first, second, fc, sc, m, mirrored_features);
+    if (m.count != 0u) write_contact(w, index, fs, ss, first, second, fc, sc, m, mirrored_features);
+    return kNoList;
+}
+
+// One thread per candidate pair of the kind-grouped list (every pair's result goes to its own slot,
+// so the order changes nothing).
+__global__ void __launch_bounds__(kThreads) k_narrow(W w) {
+    __shared__ BlockLists<2> lists;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t total = w.work_total[kTotalAll];
+    if (blockIdx.x * blockDim.x >= total) return;
+    lists.begin();
+    uint32_t index = 0u, list = kNoList;
+    if (t < total) {
+        index = w.worklist[t];
+        list = narrow_pair(w, index);
+    }
+    lists.finish(list, index, list == 0u && w.pkind[index] >= kHullClasses, &w.work_total[kTotalHull],
+                 {{&w.work_total[kTotalGjk], w.work_minor, 0u}, {&w.work_total[kTotalPlane], w.work_minor, w.pair_cap}});
 }
 
 // Intermediate results of a convex pair, parked in the pair's raw contact slot (which only its
@@ -760,41 +854,41 @@ __device__ inline void convex_pair_after_gjk(const W& w, const ConvexPair& c, co
 // GJK of the pairs marked kPairGjk (convex_hit, convex.wgsl:584-618), one thread per pair of the
 // worklist, for its first kGjkFirstIterations iterations: a pair GJK answers by then goes on to
 // the probe and is parked for EPA or the manifold kernel (or ends); a pair that needs more parks
-// its GJK state (kPairGjkResume) for k_narrow_convex_resume.
+// its GJK state for k_narrow_convex_resume.
 // Three waves a SIMD (168 registers, a few spilled): the loop is vector-ALU bound and the third
 // wave hides more of its latency than the spills cost (k_narrow_convex 708 -> 627 us and the
 // resume kernel 338 -> 277 us on the settled 100k pile; four waves, 128 registers, were slower).
-__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w, uint32_t class_blocks) {
+__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w) {
+    __shared__ BlockLists<1> lists;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0u) {
-        uint32_t hull = 0;  // GJK pairs of the hull classes
-        for (uint32_t c = kHullClasses; c < kClasses; ++c) hull += w.class_hist[kClasses * class_blocks + c];
-        w.work_total[3] = hull;
-        w.work_total[5] = 0u;  // EPA polytopes k_narrow_epa_small gives up, counted there
+    const uint32_t total = w.work_total[kTotalGjk];
+    if (blockIdx.x * blockDim.x >= total) return;
+    lists.begin();
+    uint32_t index = 0u, list = kNoList;
+    if (t < total) {
+        index = w.work_minor[t];
+        w.valid[index] = kPairNone;
+        const ConvexPair c = load_convex_pair(w, index);
+        const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
+        GjkState g;
+        gjk_begin<1>(c.first, c.second, shapes, &g);
+        Closest closest;
+        if (gjk_run<1>(c.first, c.second, shapes, &g, kGjkFirstIterations, &closest)) {
+            convex_pair_after_gjk(w, c, shapes, closest, g);
+        } else {
+            park_gjk(parked(w, index), g);
+            list = 0u;
+        }
     }
-    if (t >= w.work_total[0]) return;
-    const uint32_t index = w.worklist[t];
-    w.valid[index] = kPairNone;
-    const ConvexPair c = load_convex_pair(w, index);
-    const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
-    GjkState g;
-    gjk_begin<1>(c.first, c.second, shapes, &g);
-    Closest closest;
-    if (!gjk_run<1>(c.first, c.second, shapes, &g, kGjkFirstIterations, &closest)) {
-        park_gjk(parked(w, index), g);
-        w.valid[index] = kPairGjkResume;
-        return;
-    }
-    convex_pair_after_gjk(w, c, shapes, closest, g);
+    lists.finish(list, index, false, nullptr, {{&w.work_total[kTotalResume], w.worklist, 0u}});
 }
 
-// The remaining GJK iterations of the pairs k_narrow_convex parked (kPairGjkResume), from their
+// The remaining GJK iterations of the pairs k_narrow_convex parked, from their
 // parked state, then the rest of convex_hit as in k_narrow_convex.
 __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= w.work_total[4]) return;
+    if (t >= w.work_total[kTotalResume]) return;
     const uint32_t index = w.worklist[t];
-    w.valid[index] = kPairNone;
     const ConvexPair c = load_convex_pair(w, index);
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     GjkState g;
@@ -802,6 +896,23 @@ __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
     Closest closest;
     gjk_run<1>(c.first, c.second, shapes, &g, kGjkIterations, &closest);
     convex_pair_after_gjk(w, c, shapes, closest, g);
+}
+
+// After GJK: its penetrating pairs to the front of worklist, its hits to the end.
+__global__ void __launch_bounds__(kThreads) k_work_split(W w) {
+    __shared__ BlockLists<2> lists;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t total = w.work_total[kTotalGjk];
+    if (blockIdx.x * blockDim.x >= total) return;
+    lists.begin();
+    uint32_t index = 0u, list = kNoList;
+    if (t < total) {
+        index = w.work_minor[t];
+        const uint32_t mark = w.valid[index];
+        list = mark == kPairEpa ? 0u : (mark == kPairHit ? 1u : kNoList);
+    }
+    lists.finish(list, index, false, nullptr,
+                 {{&w.work_total[kTotalEpa], w.worklist, 0u}, {&w.work_total[kTotalHit], w.worklist, w.pair_cap}});
 }
 
 constexpr uint32_t kEpaWaves = 4;  // waves per workgroup of k_narrow_epa and k_narrow_epa_small
@@ -819,14 +930,14 @@ __device__ __forceinline__ void park_epa(float* park, const Epa& r) {
 
 // EPA of the pairs marked kPairEpa, kEpaGroup lanes per pair, the groups striding over the
 // worklist. A pair whose polytope outgrows the small capacities keeps its mark and is listed for
-// k_narrow_epa (work_total[5] entries of work_minor); the others are parked (lane 0 of the group)
+// k_narrow_epa (kTotalEpaWave entries of work_minor); the others are parked (lane 0 of the group)
 // and marked kPairEpaDone.
 __global__ void __launch_bounds__(kEpaWaves * kWave) k_narrow_epa_small(W w, uint32_t vertex_limit) {
     constexpr uint32_t kGroupsPerBlock = kEpaWaves * kWave / kEpaGroup;
     __shared__ EpaSmallShared epa[kGroupsPerBlock];
     const uint32_t slot = threadIdx.x / kEpaGroup;
     const uint32_t q = threadIdx.x % kEpaGroup;
-    const uint32_t total = w.work_total[2];
+    const uint32_t total = w.work_total[kTotalEpa];
     const uint32_t groups = gridDim.x * kGroupsPerBlock;
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     for (uint32_t t = blockIdx.x * kGroupsPerBlock + slot; t < total; t += groups) {
@@ -837,7 +948,7 @@ __global__ void __launch_bounds__(kEpaWaves * kWave) k_narrow_epa_small(W w, uin
         float* park = parked(w, index);
         Epa r;
         if (!epa_small(wf, wsd, shapes, park, vertex_limit, epa[slot], &r)) {
-            if (q == 0u) w.work_minor[atomicAdd(&w.work_total[5], 1u)] = index;
+            if (q == 0u) w.work_minor[atomicAdd(&w.work_total[kTotalEpaWave], 1u)] = index;
             continue;
         }
         if (q == 0u) {
@@ -853,7 +964,7 @@ __global__ void __launch_bounds__(kEpaWaves * kWave) k_narrow_epa(W w) {
     __shared__ EpaShared epa[kEpaWaves];
     const uint32_t lane = lane_id();
     const uint32_t wave = threadIdx.x / kWave;
-    const uint32_t total = w.work_total[5];
+    const uint32_t total = w.work_total[kTotalEpaWave];
     const uint32_t waves = gridDim.x * kEpaWaves;
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     for (uint32_t t = blockIdx.x * kEpaWaves + wave; t < total; t += waves) {
@@ -921,17 +1032,21 @@ __device__ __forceinline__ void finish_pair(const W& w, uint32_t index, uint32_t
 
 __global__ void __launch_bounds__(kThreads, 4) k_narrow_finish(W w) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= w.work_total[1]) return;
-    const uint32_t index = w.worklist[t];
+    // the penetrating pairs (but for those k_narrow_finish_tail takes), the hits, the plane pairs
+    const uint32_t epa = w.work_total[kTotalEpa], hits = w.work_total[kTotalHit], planes = w.work_total[kTotalPlane];
+    if (t >= epa + hits + planes) return;
+    const uint32_t index = t < epa ? w.worklist[t]
+                           : t < epa + hits ? w.worklist[w.pair_cap - 1u - (t - epa)]
+                                            : w.work_minor[w.pair_cap - 1u - (t - epa - hits)];
     const uint32_t mark = w.valid[index];
     if (mark != kPairEpaDone && mark != kPairHit && mark != kPairPlane) return;
     finish_pair(w, index, mark);
 }
 
 // The manifolds of the polytopes k_narrow_epa expanded (listed in work_minor). Their marks keep
-// them off k_narrow_finish's worklist, so the two can run side by side on two streams.
+// them from k_narrow_finish, so the two can run side by side on two streams.
 __global__ void __launch_bounds__(kThreads, 4) k_narrow_finish_tail(W w) {
-    const uint32_t total = w.work_total[5];
+    const uint32_t total = w.work_total[kTotalEpaWave];
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
         const uint32_t index = w.work_minor[t];
         if (w.valid[index] == kPairEpaWave) finish_pair(w, index, kPairEpaDone);
@@ -3005,24 +3120,32 @@ int scan(dyn_world* world, const uint32_t* flags, const uint32_t* count, uint32_
     return scan(world->w, world->stream, flags, count, limit, dest, total, counts);
 }
 
-// The worklist of convex pairs of one mode, grouped by kind class: block histograms, their
-// per-class scans, the scatter (total in work_total[mode]).
-int worklist(const dyn::W& w, hipStream_t st, uint32_t mode) {
+// Every candidate pair on the worklist, grouped by kind class: block histograms, their per-class
+// scans, the scatter.
+int class_worklist(const dyn::W& w, hipStream_t st) {
     using namespace dyn;
-    const uint32_t blocks = ceil_div(w.pair_cap ? w.pair_cap : 1u, kClassBlock);
+    if (w.pair_cap <= kClassSmall) {
+        {
+            ProfileScope scope("k_class_small", st);
+            k_class_small<<<1, 1024, 0, st>>>(w);
+        }
+        DYN_LAUNCHED("k_class_small");
+        return DYN_OK;
+    }
+    const uint32_t blocks = ceil_div(w.pair_cap, kClassBlock);
     {
         ProfileScope scope("k_class_count", st);
-        k_class_count<<<blocks, kThreads, 0, st>>>(w, mode);
+        k_class_count<<<blocks, kThreads, 0, st>>>(w);
     }
     DYN_LAUNCHED("k_class_count");
     {
         ProfileScope scope("k_class_scan", st);
-        k_class_scan<<<kClasses, 1024, 0, st>>>(w.class_hist, blocks);
+        k_class_scan<<<kClasses, 1024, 0, st>>>(w.class_hist, blocks, w.work_total);
     }
     DYN_LAUNCHED("k_class_scan");
     {
         ProfileScope scope("k_class_scatter", st);
-        k_class_scatter<<<blocks, kThreads, 0, st>>>(w, mode);
+        k_class_scatter<<<blocks, kThreads, 0, st>>>(w);
     }
     DYN_LAUNCHED("k_class_scatter");
     return DYN_OK;
@@ -3040,7 +3163,7 @@ int worklist(const dyn::W& w, hipStream_t st, uint32_t mode) {
 
 // The narrowphase of the candidate pairs on pmaj/pmin (narrowphase.wgsl:518-685): k_narrow
 // writes the analytic manifolds and marks the convex-path pairs, which (when `convex`) GJK, EPA
-// and the convex manifolds take up over class-grouped worklists. Afterwards valid[i] is
+// and the convex manifolds take up over their lists. Afterwards valid[i] is
 // kPairContact where raw[i] holds pair i's contact and kPairNone elsewhere, for every pair below
 // the PAIRS counter (and the capacity).
 // With `side` (a second stream and two events) the wave EPA kernel and the manifolds of its
@@ -3049,16 +3172,12 @@ int worklist(const dyn::W& w, hipStream_t st, uint32_t mode) {
 int narrowphase(const dyn::W& w, hipStream_t st, bool convex, const SideStream* side = nullptr) {
     using namespace dyn;
     const uint32_t pb = blocks_for(w.pair_cap);
-    LAUNCH_ON(st, k_pair_class, pb, w);
-    DYN_TRY(worklist(w, st, kWorkAllPairs));
+    DYN_TRY(class_worklist(w, st));
     LAUNCH_ON(st, k_narrow, pb, w);
     if (!convex) return DYN_OK;
-    DYN_TRY(worklist(w, st, 0u));
-    const uint32_t class_blocks = ceil_div(w.pair_cap ? w.pair_cap : 1u, kClassBlock);
-    LAUNCH_ON(st, k_narrow_convex, pb, w, class_blocks);
-    DYN_TRY(worklist(w, st, 4u));
+    LAUNCH_ON(st, k_narrow_convex, pb, w);
     LAUNCH_ON(st, k_narrow_convex_resume, pb, w);
-    DYN_TRY(worklist(w, st, 2u));
+    LAUNCH_ON(st, k_work_split, pb, w);
     {
         constexpr uint32_t kPairsPerBlock = kEpaWaves * kWave / kEpaGroup;
         const uint32_t small_groups = min(ceil_div(w.pair_cap ? w.pair_cap : 1u, kPairsPerBlock), 2048u);
@@ -3082,7 +3201,6 @@ int narrowphase(const dyn::W& w, hipStream_t st, bool convex, const SideStream* 
     DYN_LAUNCHED("k_narrow_epa");
     LAUNCH_ON(tail, k_narrow_finish_tail, min(pb, 64u), w);
     if (side) DYN_HIP(hipEventRecord(side->join, side->stream));
-    DYN_TRY(worklist(w, st, 1u));
     LAUNCH_ON(st, k_narrow_finish, pb, w);
     if (side) DYN_HIP(hipStreamWaitEvent(st, side->join, 0));
     return DYN_OK;
@@ -3561,7 +3679,7 @@ int dyn_world_create(dyn_world** out, void* stream, const dyn_step_params* param
     A(w.row_start, body_count);
     A(w.contrib, body_count);
     A(w.scan_total, 4);
-    A(w.work_total, 8);
+    A(w.work_total, kTotalWords);
     A(world->snap_header, 4);
     A(world->words, 8);
     A(world->entry_keys, world->entry_cap);
@@ -3825,7 +3943,11 @@ int dyn_world_step(dyn_world* world, float dt) {
 int dyn_world_read_work(dyn_world* world, uint32_t* out) {
     if (!world || !out) return dyn::fail(DYN_E_INVALID, "dyn_world_read_work: null argument");
     DYN_HIP(hipStreamSynchronize(world->stream));
-    DYN_HIP(hipMemcpy(out, world->w.work_total, 6u * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    uint32_t totals[dyn::kTotalWords];
+    DYN_HIP(hipMemcpy(totals, world->w.work_total, sizeof totals, hipMemcpyDeviceToHost));
+    std::copy(totals, totals + 6, out);
+    // the manifold kernel's pairs: the planes', the hits, and the polytopes not given a wave
+    out[1] = totals[dyn::kTotalPlane] + totals[dyn::kTotalHit] + totals[dyn::kTotalEpa] - totals[dyn::kTotalEpaWave];
     return DYN_OK;
 }
 
@@ -4002,7 +4124,7 @@ NarrowLayout narrow_layout(uint32_t pair_capacity, void* base) {
     l.worklist = reinterpret_cast<uint32_t*>(take(4u * cap));
     l.class_hist = reinterpret_cast<uint32_t*>(take(4u * kClasses * (static_cast<size_t>(ceil_div(
                                                                           static_cast<uint32_t>(cap), kClassBlock)) + 1u)));
-    l.work_total = reinterpret_cast<uint32_t*>(take(4u * 8u));
+    l.work_total = reinterpret_cast<uint32_t*>(take(4u * kTotalWords));
     l.work_minor = reinterpret_cast<uint32_t*>(take(4u * cap));
     l.bytes = at;
     return l;
