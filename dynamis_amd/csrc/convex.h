@@ -2,7 +2,7 @@
 // kind (hulls by a linear scan of their vertices), GJK closest points, EPA penetration, the
 // direction probe fallback, and manifolds from clipped feature rings. Semantics:
 // crates/dynamis-shader/shaders/convex.wgsl:1-1071 and crates/dynamis-rigid/shaders/
-// narrowphase.wgsl:479-512. GJK, the probe and the manifolds run one thread per pair; EPA runs one
+// narrowphase.wgsl:479-512. GJK and its probe run four lanes per pair (one in a long list), the manifolds one; EPA runs one
 // wavefront per penetrating pair, with the polytope in the wave's LDS and the lanes scanning a
 // hull's vertices and EPA's faces in parallel, reduced to the element the reference's sequential
 // scan picks (the first maximum or minimum).
@@ -386,19 +386,224 @@ __device__ inline SimplexResult simplex_closest(const SimplexPoint* s, uint32_t 
     return r;
 }
 
-template <int kLanes = 1>
-__device__ inline SimplexPoint support_pair(const Shape& a, const Shape& b, const ShapeSet& ss, v3 dir) {
-    SimplexPoint p;
-    p.a = support<kLanes>(a, ss, dir);
-    p.b = support<kLanes>(b, ss, neg(dir));
-    p.w = sub(p.a, p.b);
-    return p;
-}
-
 __device__ __forceinline__ float shape_scale(const Shape& w) {
     float scale = w.radius + w.half_height;
     scale = fmx(scale, fmx(fmx(w.half_extents.x, w.half_extents.y), w.half_extents.z));
     return fmx(scale, 1e-4f) * fmx(fmx(w.scale.x, w.scale.y), w.scale.z);
+}
+
+// ---- GJK by quads ------------------------------------------------------------------------------
+//
+// Four lanes share a pair. All of them hold the simplex and its closest point (the same bits); side
+// q & 1 evaluates one shape's support, the other side the other's, and lane q takes vertex q, edges q
+// and 4 + q and triangle q of the closest-point search and face q of the containment test, whose
+// results the lanes compare by (length, place in the sequential order): the first minimum, which is
+// what the sequential search keeps. One thread per pair walks 14 features and two supports an
+// iteration in a row: 12 us of latency, which the waves of a short list do not hide (k_narrow_convex
+// of 114,000 candidate pairs 148 -> 95 us and k_narrow_convex_resume 212 -> 107 us by quads). The
+// quad does about 1.7 times the vector work a pair, so long lists, which are bound by it, keep one
+// thread a pair (the 100,000-body pile's k_narrow_convex: 395 us, by quads 678 us).
+
+// Lane value of the lane DPP control `kCtrl` names (quad permutes and the half-row mirror stay
+// inside an aligned group of 8 lanes).
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, 0xF, 0xF, false));
+}
+constexpr int kDppQuadSwap1 = 0xB1;     // quad_perm [1, 0, 3, 2]
+constexpr int kDppQuadSwap2 = 0x4E;     // quad_perm [2, 3, 0, 1]
+constexpr int kDppHalfMirror = 0x141;  // row_half_mirror: lane 7 - l of each 8 lanes
+
+constexpr int kQuadSideFirst = 0xA0;   // quad_perm [0, 0, 2, 2]
+constexpr int kQuadSideSecond = 0xF5;  // quad_perm [1, 1, 3, 3]
+constexpr int kQuadLow = 0x44;         // quad_perm [0, 1, 0, 1]
+constexpr int kQuadHigh = 0xEE;        // quad_perm [2, 3, 2, 3]
+
+template <int kCtrl>
+__device__ __forceinline__ float dpp_f32(float v) { return __uint_as_float(dpp_u32<kCtrl>(__float_as_uint(v))); }
+template <int kCtrl>
+__device__ __forceinline__ v3 dpp_v3(v3 v) { return mk(dpp_f32<kCtrl>(v.x), dpp_f32<kCtrl>(v.y), dpp_f32<kCtrl>(v.z)); }
+
+// A pair as a quad holds it: this lane's side's shape, and what both sides are read for.
+struct QuadPair {
+    Shape mine;
+    uint32_t q;  // lane of the quad; the side is q & 1
+    v3 first_center, second_center;
+    float first_scale, second_scale;  // shape_scale
+};
+
+__device__ __forceinline__ QuadPair quad_pair(const Shape& mine, uint32_t q) {
+    QuadPair p;
+    p.mine = mine;
+    p.q = q;
+    p.first_center = dpp_v3<kQuadSideFirst>(mine.center);
+    p.second_center = dpp_v3<kQuadSideSecond>(mine.center);
+    const float scale = shape_scale(mine);
+    p.first_scale = dpp_f32<kQuadSideFirst>(scale);
+    p.second_scale = dpp_f32<kQuadSideSecond>(scale);
+    return p;
+}
+
+// The two sides' support points along the side's direction (the second's is the negated one).
+__device__ __forceinline__ void quad_support(const QuadPair& p, const ShapeSet& ss, v3 dir, v3* a, v3* b) {
+    const v3 point = support<1>(p.mine, ss, pick3((p.q & 1u) != 0u, neg(dir), dir));
+    *a = dpp_v3<kQuadSideFirst>(point);
+    *b = dpp_v3<kQuadSideSecond>(point);
+}
+
+__device__ __forceinline__ SimplexPoint quad_support_pair(const QuadPair& p, const ShapeSet& ss, v3 dir) {
+    SimplexPoint r;
+    quad_support(p, ss, dir, &r.a, &r.b);
+    r.w = sub(r.a, r.b);
+    return r;
+}
+
+// Whether every lane of the quad agrees (each lane's own value in, the same for all out).
+__device__ __forceinline__ bool quad_all(bool v) {
+    uint32_t u = v ? 1u : 0u;
+    u &= dpp_u32<kDppQuadSwap1>(u);
+    u &= dpp_u32<kDppQuadSwap2>(u);
+    return u != 0u;
+}
+
+// Whether the tetrahedron holds the origin; lane q tests face q (tet_face).
+__device__ inline bool quad_tetra_contains(const SimplexPoint* s, uint32_t q) {
+    const v3 a = pick3(q == 3u, s[1].w, s[0].w);
+    const v3 b = pick3(q == 0u, s[1].w, pick3(q == 1u, s[2].w, s[3].w));
+    const v3 c = pick3(q == 0u || q == 3u, s[2].w, pick3(q == 1u, s[3].w, s[1].w));
+    const v3 normal = cross3(sub(b, a), sub(c, a));
+    const float span = fmx(fmx(len3(sub(b, a)), len3(sub(c, a))), len3(sub(c, b)));
+    const bool outside = len3(normal) <= 1e-6f * span * span || dot3(normal, sub(zero3v(), a)) > 0.0f;
+    return quad_all(!outside);
+}
+
+// A feature's closest point: its length, its place in the search's order above the simplex slots it
+// weighs (0xF: none), the point and the slots' weights.
+struct QuadFeature {
+    float length;
+    uint32_t key;
+    v3 point, weights;
+};
+
+__device__ __forceinline__ void quad_take(QuadFeature* best, float length, uint32_t order, uint32_t slots, v3 point,
+                                          v3 weights) {
+    if (!(length < best->length)) return;
+    best->length = length;
+    best->key = (order << 16) | slots;
+    best->point = point;
+    best->weights = weights;
+}
+
+template <int kCtrl>
+__device__ __forceinline__ void quad_first_min(QuadFeature* f) {
+    const float length = dpp_f32<kCtrl>(f->length);
+    const uint32_t key = dpp_u32<kCtrl>(f->key);
+    const v3 point = dpp_v3<kCtrl>(f->point), weights = dpp_v3<kCtrl>(f->weights);
+    const bool other = length < f->length || (length == f->length && key < f->key);
+    f->length = other ? length : f->length;
+    f->key = other ? key : f->key;
+    f->point = pick3(other, point, f->point);
+    f->weights = pick3(other, weights, f->weights);
+}
+
+__device__ inline SimplexResult quad_simplex_closest(const SimplexPoint* s, uint32_t count, uint32_t q) {
+    SimplexResult r;
+    r.v = mk(kBig, kBig, kBig);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.lambdas[i] = 0.0f;
+    r.penetrating = count == 4u && quad_tetra_contains(s, q);
+    r.point_a = zero3v();
+    r.point_b = zero3v();
+    if (r.penetrating) {
+        r.v = zero3v();
+        return r;
+    }
+    QuadFeature best;
+    best.length = len3(r.v);
+    best.key = 0xFFFFFFFFu;
+    best.point = r.v;
+    best.weights = zero3v();
+    {
+        const v3 p = pick3(q < 2u, pick3(q == 0u, s[0].w, s[1].w), pick3(q == 2u, s[2].w, s[3].w));
+        if (q < count) quad_take(&best, len3(p), q, 0xFF0u | q, p, mk(1.0f, 0.0f, 0.0f));
+    }
+    // edges 01 02 03 12, then 13 23
+#pragma unroll
+    for (uint32_t e = 0; e < 2; ++e) {
+        const uint32_t i = e == 0u ? (q == 3u ? 1u : 0u) : (q == 0u ? 1u : 2u);
+        const uint32_t j = e == 0u ? (q == 3u ? 2u : q + 1u) : 3u;
+        if ((e == 1u && q > 1u) || j >= count) continue;
+        const v3 a = pick3(i == 0u, s[0].w, pick3(i == 1u, s[1].w, s[2].w));
+        const v3 b = pick3(j == 1u, s[1].w, pick3(j == 2u, s[2].w, s[3].w));
+        const v3 ab = sub(b, a);
+        const float denom = dot3(ab, ab);
+        if (denom < 1e-12f) continue;
+        const float t = clampf(-dot3(a, ab) / denom, 0.0f, 1.0f);
+        const v3 point = add(a, mul(ab, t));
+        quad_take(&best, len3(point), 4u + e * 4u + q, 0xF00u | (j << 4) | i, point, mk(1.0f - t, t, 0.0f));
+    }
+    // triangles 012 013 023 123
+    if (count >= 3u) {
+        const uint32_t i = q == 3u ? 1u : 0u, j = q < 2u ? 1u : 2u, k = q == 0u ? 2u : 3u;
+        if (k < count) {
+            v3 weights;
+            const v3 point = closest_on_triangle(zero3v(), pick3(i == 0u, s[0].w, s[1].w), pick3(j == 1u, s[1].w, s[2].w),
+                                                 pick3(k == 2u, s[2].w, s[3].w), &weights);
+            quad_take(&best, len3(point), 10u + q, (k << 8) | (j << 4) | i, point, weights);
+        }
+    }
+    quad_first_min<kDppQuadSwap1>(&best);
+    quad_first_min<kDppQuadSwap2>(&best);
+    r.v = best.point;
+    const uint32_t slots = best.key;  // 0xFFF where no feature was shorter than the start
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        r.lambdas[i] = (slots & 0xFu) == i ? best.weights.x
+                       : ((slots >> 4) & 0xFu) == i ? best.weights.y
+                       : ((slots >> 8) & 0xFu) == i ? best.weights.z
+                                                    : 0.0f;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        if (i < count) {
+            r.point_a = add(r.point_a, smul(r.lambdas[i], s[i].a));
+            r.point_b = add(r.point_b, smul(r.lambdas[i], s[i].b));
+        }
+    }
+    return r;
+}
+
+// ---- GJK over either kind of pair ---------------------------------------------------------------
+
+// A pair as one thread holds it.
+struct ThreadPair {
+    Shape first, second;
+    v3 first_center, second_center;
+    float first_scale, second_scale;
+};
+
+__device__ __forceinline__ ThreadPair thread_pair(const Shape& first, const Shape& second) {
+    return ThreadPair{first, second, first.center, second.center, shape_scale(first), shape_scale(second)};
+}
+
+__device__ __forceinline__ SimplexPoint pair_support(const ThreadPair& p, const ShapeSet& ss, v3 dir) {
+    SimplexPoint r;
+    r.a = support<1>(p.first, ss, dir);
+    r.b = support<1>(p.second, ss, neg(dir));
+    r.w = sub(r.a, r.b);
+    return r;
+}
+
+__device__ __forceinline__ SimplexPoint pair_support(const QuadPair& p, const ShapeSet& ss, v3 dir) {
+    return quad_support_pair(p, ss, dir);
+}
+
+__device__ __forceinline__ SimplexResult pair_closest(const ThreadPair&, const SimplexPoint* s, uint32_t count) {
+    return simplex_closest(s, count);
+}
+
+__device__ __forceinline__ SimplexResult pair_closest(const QuadPair& p, const SimplexPoint* s, uint32_t count) {
+    return quad_simplex_closest(s, count, p.q);
 }
 
 __device__ inline v3 simplex_expand_dir(const SimplexPoint* s, uint32_t count) {
@@ -426,39 +631,30 @@ struct GjkState {
 
 constexpr uint32_t kGjkIterations = 24;  // convex.wgsl:478
 
-// The result convex_closest returns when its loop runs out without an answer (or before it has
-// one): the centres and their normalized offset.
-__device__ inline Closest closest_default(const Shape& first, const Shape& second) {
-    Closest r;
-    r.distance = 0.0f;
-    r.point_a = first.center;
-    r.point_b = second.center;
-    r.normal = sign_normalize(sub(second.center, first.center));
-    r.penetrating = false;
-    return r;
-}
-
 // convex_closest (convex.wgsl:464-521), the part before the loop.
-template <int kLanes = 1>
-__device__ inline void gjk_begin(const Shape& first, const Shape& second, const ShapeSet& ss, GjkState* g) {
-    v3 dir = sub(second.center, first.center);
+template <typename Pair>
+__device__ inline void gjk_begin(const Pair& p, const ShapeSet& ss, GjkState* g) {
+    v3 dir = sub(p.second_center, p.first_center);
     if (len3(dir) < 1e-8f) dir = mk(1.0f, 0.0f, 0.0f);
 #pragma unroll
     for (uint32_t i = 1; i < 4; ++i) g->simplex[i].w = g->simplex[i].a = g->simplex[i].b = zero3v();
-    g->simplex[0] = support_pair<kLanes>(first, second, ss, dir);
+    g->simplex[0] = pair_support(p, ss, dir);
     g->count = 1;
-    g->closest = simplex_closest(g->simplex, g->count);
+    g->closest = pair_closest(p, g->simplex, g->count);
     g->iter = 0;
 }
 
 // The loop of convex_closest from iteration g->iter up to (not including) `limit`. Returns true
-// with *r set when the loop has ended (answered, or all kGjkIterations run), false when it
-// stopped at `limit` with the state in *g.
-template <int kLanes = 1>
-__device__ inline bool gjk_run(const Shape& first, const Shape& second, const ShapeSet& ss, GjkState* g,
-                               uint32_t limit, Closest* r) {
-    *r = closest_default(first, second);
-    const float tiny = 1e-4f * fmn(shape_scale(first), shape_scale(second));
+// with *r set when the loop has ended (answered, or all kGjkIterations run: the centres and their
+// normalized offset), false when it stopped at `limit` with the state in *g.
+template <typename Pair>
+__device__ inline bool gjk_run(const Pair& p, const ShapeSet& ss, GjkState* g, uint32_t limit, Closest* r) {
+    r->distance = 0.0f;
+    r->point_a = p.first_center;
+    r->point_b = p.second_center;
+    r->normal = sign_normalize(sub(p.second_center, p.first_center));
+    r->penetrating = false;
+    const float tiny = 1e-4f * fmn(p.first_scale, p.second_scale);
     SimplexPoint* simplex = g->simplex;
     uint32_t count = g->count;
     SimplexResult closest = g->closest;
@@ -469,7 +665,7 @@ __device__ inline bool gjk_run(const Shape& first, const Shape& second, const Sh
         if (closest.penetrating || len3(closest.v) < tiny) {
             while (count < 4u) {
                 const v3 d = simplex_expand_dir(simplex, count);
-                set_slot(simplex, count, support_pair<kLanes>(first, second, ss, d));
+                set_slot(simplex, count, pair_support(p, ss, d));
                 ++count;
             }
             r->penetrating = true;
@@ -480,17 +676,13 @@ __device__ inline bool gjk_run(const Shape& first, const Shape& second, const Sh
             break;
         }
         const v3 nv = neg(closest.v);
-        const SimplexPoint sp = support_pair<kLanes>(first, second, ss, nv);
-        if (dot3(sp.w, nv) <= dot3(closest.v, nv) + 1e-4f * fmx(1.0f, dot3(closest.v, closest.v))) {
-            r->distance = len3(closest.v);
-            r->point_a = closest.point_a;
-            r->point_b = closest.point_b;
-            if (r->distance > 1e-6f) r->normal = sign_normalize(sub(closest.point_b, closest.point_a));
-            done = true;
-            break;
+        const SimplexPoint sp = pair_support(p, ss, nv);
+        bool answered = dot3(sp.w, nv) <= dot3(closest.v, nv) + 1e-4f * fmx(1.0f, dot3(closest.v, closest.v));
+        if (!answered) {
+            count = simplex_reduce(simplex, closest.lambdas);
+            answered = simplex_holds(simplex, count, sp.w, p.second_scale);
         }
-        count = simplex_reduce(simplex, closest.lambdas);
-        if (simplex_holds(simplex, count, sp.w, shape_scale(second))) {
+        if (answered) {
             r->distance = len3(closest.v);
             r->point_a = closest.point_a;
             r->point_b = closest.point_b;
@@ -500,25 +692,12 @@ __device__ inline bool gjk_run(const Shape& first, const Shape& second, const Sh
         }
         set_slot(simplex, count, sp);
         ++count;
-        closest = simplex_closest(simplex, count);
+        closest = pair_closest(p, simplex, count);
     }
     g->count = count;
     g->closest = closest;
     g->iter = iter;
     return done || iter >= kGjkIterations;
-}
-
-template <int kLanes = 1>
-__device__ inline Closest convex_closest(const Shape& first, const Shape& second, const ShapeSet& ss,
-                                         SimplexPoint* simplex, uint32_t* out_count) {
-    GjkState g;
-    gjk_begin<kLanes>(first, second, ss, &g);
-    Closest r;
-    gjk_run<kLanes>(first, second, ss, &g, kGjkIterations, &r);
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) simplex[i] = g.simplex[i];
-    *out_count = g.count;
-    return r;
 }
 
 // ---- EPA (convex.wgsl:286-437), one wave per polytope ------------------------------------------
@@ -770,16 +949,6 @@ __device__ __forceinline__ v3 small_w(const EpaSmallShared& e, uint32_t i) {
     return mk(p.x, p.y, p.z);
 }
 
-// Lane value of the lane DPP control `kCtrl` names (quad permutes and the half-row mirror stay
-// inside an aligned group of 8 lanes).
-template <int kCtrl>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, 0xF, 0xF, false));
-}
-constexpr int kDppQuadSwap1 = 0xB1;     // quad_perm [1, 0, 3, 2]
-constexpr int kDppQuadSwap2 = 0x4E;     // quad_perm [2, 3, 0, 1]
-constexpr int kDppHalfMirror = 0x141;  // row_half_mirror: lane 7 - l of each 8 lanes
-
 __device__ __forceinline__ void group8_min_first(float* best, uint32_t* index) {
     uint32_t b = __float_as_uint(*best), i = *index;
     const auto step = [&](uint32_t ob, uint32_t oi) {
@@ -950,10 +1119,9 @@ __device__ inline bool epa_small(const Shape& first, const Shape& second, const 
 
 // ---- penetration probe and convex_hit (convex.wgsl:523-618) ----------------------------------
 
-template <int kLanes = 1>
 __device__ __forceinline__ float support_projection_depth(const Shape& a, const Shape& b, const ShapeSet& ss, v3 dir) {
     const v3 n = norm3(dir);
-    return dot3(sub(support<kLanes>(a, ss, n), support<kLanes>(b, ss, neg(n))), n);
+    return dot3(sub(support<1>(a, ss, n), support<1>(b, ss, neg(n))), n);
 }
 
 struct Probe {
@@ -961,10 +1129,9 @@ struct Probe {
     v3 normal;
 };
 
-template <int kLanes = 1>
 __device__ __forceinline__ void probe_direction(const Shape& first, const Shape& second, const ShapeSet& ss,
                                                 v3 direction, Probe* best) {
-    const float depth = support_projection_depth<kLanes>(first, second, ss, direction);
+    const float depth = support_projection_depth(first, second, ss, direction);
     if (depth < best->depth) {
         best->depth = depth;
         best->normal = norm3(direction);
@@ -977,7 +1144,6 @@ __device__ __forceinline__ void probe_direction(const Shape& first, const Shape&
 // are generated. With `until_separated` the scan stops at the first direction whose overlap is
 // not positive: the depth is then not positive either, which is all the GJK half of convex_hit
 // reads of it (the normal of such a probe is never used).
-template <int kLanes = 1>
 __device__ inline Probe penetration_probe(const Shape& first, const Shape& second, const ShapeSet& ss,
                                           const SimplexPoint* s, uint32_t count, bool until_separated) {
     Probe best;
@@ -991,22 +1157,80 @@ __device__ inline Probe penetration_probe(const Shape& first, const Shape& secon
         const v3 c = t == 0u ? s[2].w : s[3].w;
         const v3 normal = cross3(sub(b, a), sub(c, a));
         if (len3(normal) > 1e-8f) {
-            probe_direction<kLanes>(first, second, ss, normal, &best);
+            probe_direction(first, second, ss, normal, &best);
             if (until_separated && !(best.depth > 0.0f)) return best;
         }
     }
     const v3 center_dir = sub(second.center, first.center);
     if (len3(center_dir) > 1e-8f) {
-        probe_direction<kLanes>(first, second, ss, center_dir, &best);
+        probe_direction(first, second, ss, center_dir, &best);
         if (until_separated && !(best.depth > 0.0f)) return best;
     }
     for (uint32_t i = 0; i < 6; ++i) {
         const float sgn = (i & 1u) ? -1.0f : 1.0f;
         const v3 axis = i < 2u ? mk(sgn, 0.0f, 0.0f) : (i < 4u ? mk(0.0f, sgn, 0.0f) : mk(0.0f, 0.0f, sgn));
-        probe_direction<kLanes>(first, second, ss, axis, &best);
+        probe_direction(first, second, ss, axis, &best);
         if (until_separated && !(best.depth > 0.0f)) return best;
     }
     return best;
+}
+
+// The same probe by a quad, two directions at a time (lanes 0 and 1 the first, 2 and 3 the second).
+// It stops at the first direction whose overlap is not positive: the depth is then not positive
+// either, which is all the GJK half of convex_hit reads of it (the normal of such a probe is never
+// used).
+__device__ inline Probe quad_penetration_probe(const QuadPair& p, const ShapeSet& ss, const SimplexPoint* s,
+                                               uint32_t count) {
+    Probe best;
+    best.depth = kBig;
+    best.normal = mk(0.0f, 1.0f, 0.0f);
+    const bool high = p.q >= 2u;
+    const v3 center_dir = sub(p.second_center, p.first_center);
+    for (uint32_t pair = 0; pair < 6; ++pair) {
+        // directions 2 * pair and 2 * pair + 1 of: four triangles, the centre line, six axes
+        const uint32_t d = 2u * pair + (high ? 1u : 0u);
+        v3 direction = center_dir;
+        bool valid;
+        if (pair < 2u) {
+            const uint32_t needs = d == 0u ? 3u : 4u;
+            if (count < (pair == 0u ? 3u : 4u)) continue;  // neither triangle exists
+            const v3 a = pick3(d == 3u, s[1].w, s[0].w), b = pick3(d < 2u, s[1].w, s[2].w);
+            const v3 c = pick3(d == 0u, s[2].w, s[3].w);
+            direction = cross3(sub(b, a), sub(c, a));
+            valid = count >= needs && len3(direction) > 1e-8f;
+        } else {
+            const uint32_t i = d - 5u;  // axis (d 4: the centre line)
+            const float sgn = (i & 1u) ? -1.0f : 1.0f;
+            if (d > 4u) direction = mk(i < 2u ? sgn : 0.0f, i >= 2u && i < 4u ? sgn : 0.0f, i >= 4u ? sgn : 0.0f);
+            valid = d == 4u ? len3(direction) > 1e-8f : d < 11u;
+        }
+        const v3 n = norm3(direction);
+        v3 a, b;
+        quad_support(p, ss, n, &a, &b);
+        const float depth = valid ? dot3(sub(a, b), n) : kBig;
+        const float low_depth = dpp_f32<kQuadLow>(depth), high_depth = dpp_f32<kQuadHigh>(depth);
+        const v3 low_normal = dpp_v3<kQuadLow>(n), high_normal = dpp_v3<kQuadHigh>(n);
+        if (low_depth < best.depth) {
+            best.depth = low_depth;
+            best.normal = low_normal;
+        }
+        if (high_depth < best.depth) {
+            best.depth = high_depth;
+            best.normal = high_normal;
+        }
+        if (!(best.depth > 0.0f)) return best;
+    }
+    return best;
+}
+
+__device__ __forceinline__ Probe pair_probe(const ThreadPair& p, const ShapeSet& ss, const SimplexPoint* s,
+                                            uint32_t count) {
+    return penetration_probe(p.first, p.second, ss, s, count, true);
+}
+
+__device__ __forceinline__ Probe pair_probe(const QuadPair& p, const ShapeSet& ss, const SimplexPoint* s,
+                                            uint32_t count) {
+    return quad_penetration_probe(p, ss, s, count);
 }
 
 __device__ inline Hit make_hit(float distance, v3 point, v3 normal) {
@@ -1019,14 +1243,13 @@ __device__ inline Hit make_hit(float distance, v3 point, v3 normal) {
 
 // convex_hit (convex.wgsl:584-618), GJK half: answers every pair GJK does not find penetrating
 // (returns true with the hit); for a penetrating pair returns false with GJK's final simplex,
-// which EPA (one wave) and convex_hit_finish take up.
-template <int kLanes = 1>
-__device__ inline bool convex_hit_after_gjk(const Shape& first, const Shape& second, const ShapeSet& ss,
-                                            const Closest& closest, Hit* hit, const SimplexPoint* simplex,
-                                            const uint32_t* count) {
+// which EPA and convex_hit_finish take up.
+template <typename Pair>
+__device__ inline bool convex_hit_after_gjk(const Pair& p, const ShapeSet& ss, const Closest& closest, Hit* hit,
+                                            const SimplexPoint* simplex, uint32_t count) {
     if (closest.penetrating) return false;
-    const v3 centers = sub(second.center, first.center);
-    const Probe probe = penetration_probe<kLanes>(first, second, ss, simplex, *count, true);
+    const v3 centers = sub(p.second_center, p.first_center);
+    const Probe probe = pair_probe(p, ss, simplex, count);
     if (probe.depth > 0.0f) {
         const v3 normal = dot3(probe.normal, centers) < 0.0f ? neg(probe.normal) : probe.normal;
         *hit = make_hit(-probe.depth, mul(add(closest.point_a, closest.point_b), 0.5f), normal);
@@ -1036,13 +1259,6 @@ __device__ inline bool convex_hit_after_gjk(const Shape& first, const Shape& sec
         *hit = make_hit(kBig, zero3v(), zero3v());  // NO_HIT
     }
     return true;
-}
-
-template <int kLanes = 1>
-__device__ inline bool convex_hit_gjk(const Shape& first, const Shape& second, const ShapeSet& ss, Hit* hit,
-                                      SimplexPoint* simplex, uint32_t* count) {
-    const Closest closest = convex_closest<kLanes>(first, second, ss, simplex, count);
-    return convex_hit_after_gjk<kLanes>(first, second, ss, closest, hit, simplex, count);
 }
 
 // convex_hit, the rest of a penetrating pair once EPA has run on the simplex.

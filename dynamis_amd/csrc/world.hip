@@ -588,10 +588,14 @@ __device__ __forceinline__ uint8_t kind_class(uint32_t first_kind, uint32_t seco
     return static_cast<uint8_t>(a * 6u - (a * (a - 1u)) / 2u + (b - a));
 }
 
-// A candidate pair's kind class (class 0 for pairs naming colliders outside the records).
+// A candidate pair's kind class (class 0 for pairs naming colliders outside the records, whose place
+// collider 0 takes in the reads so that they sit in no branch).
 __device__ __forceinline__ uint32_t pair_class(const W& w, uint32_t index) {
     const uint32_t fs = w.pmaj[index], ss = w.pmin[index];
-    return (fs < w.k && ss < w.k) ? kind_class(w.co[fs].kind, w.co[ss].kind) : 0u;
+    const bool known = fs < w.k && ss < w.k;
+    if (w.k == 0u) return 0u;
+    const uint32_t c = kind_class(w.co[known ? fs : 0u].kind, w.co[known ? ss : 0u].kind);
+    return known ? c : 0u;
 }
 
 // Every candidate pair's class, and each block's counts of them.
@@ -601,12 +605,20 @@ __global__ void __launch_bounds__(kThreads) k_class_count(W w) {
     __syncthreads();
     const uint32_t live = min(*cw(w.counters, DYN_COUNTER_PAIRS), w.pair_cap);
     const uint32_t base = blockIdx.x * kClassBlock;
+    // a block is few waves and its pairs' kinds two dependent reads away: all its reads in flight at once
+    // (114,000 pairs are 28 blocks; 21 us one pair after another)
+    uint32_t kinds[kClassItems];
+#pragma unroll
     for (uint32_t j = 0; j < kClassItems; ++j) {
         const uint32_t index = base + j * kThreads + threadIdx.x;
-        if (index >= live) break;
-        const uint32_t c = pair_class(w, index);
-        w.pkind[index] = static_cast<uint8_t>(c);
-        atomicAdd(&hist[c], 1u);
+        kinds[j] = base < live ? pair_class(w, min(index, live - 1u)) : 0u;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kClassItems; ++j) {
+        const uint32_t index = base + j * kThreads + threadIdx.x;
+        if (index >= live) continue;
+        w.pkind[index] = static_cast<uint8_t>(kinds[j]);
+        atomicAdd(&hist[kinds[j]], 1u);
     }
     __syncthreads();
     if (threadIdx.x < kClasses) w.class_hist[threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
@@ -759,9 +771,15 @@ __device__ __forceinline__ float* parked(const W& w, uint32_t index) {
 constexpr uint32_t kParkedGjkFloats = 36u + 3u + 4u + 1u + 3u + 3u + 2u;
 static_assert(kParkedGjkFloats * 4u <= sizeof(dyn_contact), "GJK's state fits the pair's raw slot");
 
-__device__ inline void park_gjk(float* park, const GjkState& g) {
+// Which simplex slots a lane parks: a quad's lane q slot q, a pair's only thread (kWholePair) all.
+constexpr uint32_t kWholePair = 4;
+__device__ __forceinline__ bool parks_slot(uint32_t q, uint32_t slot) { return q == slot || q == kWholePair; }
+__device__ __forceinline__ bool parks_rest(uint32_t q) { return q == 0u || q == kWholePair; }
+
+__device__ inline void park_gjk(float* park, const GjkState& g, uint32_t q) {
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
+        if (!parks_slot(q, i)) continue;
         const v3 p[3] = {g.simplex[i].w, g.simplex[i].a, g.simplex[i].b};
 #pragma unroll
         for (uint32_t k = 0; k < 3; ++k) {
@@ -770,6 +788,7 @@ __device__ inline void park_gjk(float* park, const GjkState& g) {
             park[9 * i + 3 * k + 2] = p[k].z;
         }
     }
+    if (!parks_rest(q)) return;
     const SimplexResult& c = g.closest;
     const float tail[kParkedGjkFloats - 36u] = {c.v.x, c.v.y, c.v.z, c.lambdas[0], c.lambdas[1], c.lambdas[2],
                                                  c.lambdas[3], c.penetrating ? 1.0f : 0.0f, c.point_a.x,
@@ -802,14 +821,40 @@ __device__ inline void unpark_gjk(const float* park, GjkState* g) {
 // kernel do not wait on the few pairs that run to the 24-iteration cap.
 constexpr uint32_t kGjkFirstIterations = 8;
 
+constexpr uint32_t kQuad = 4;                     // lanes per pair
+constexpr uint32_t kQuadPairs = kThreads / kQuad;  // pairs of a workgroup
+// GJK lists longer than this are run one thread a pair (convex.h says why): four lanes a pair then fill
+// the GPU many times over (2^17 pairs are 8,192 waves of quads, 8 a SIMD).
+constexpr uint32_t kLongGjk = 1u << 17;
+
+template <typename Pair>
 struct ConvexPair {
     uint32_t index;
-    Shape first, second;
+    Pair shapes;
     float margin;
 };
 
-__device__ inline ConvexPair load_convex_pair(const W& w, uint32_t index) {
-    ConvexPair c;
+// Each lane of the quad loads its side.
+__device__ inline ConvexPair<QuadPair> load_quad_pair(const W& w, uint32_t index, uint32_t q) {
+    ConvexPair<QuadPair> c;
+    c.index = index;
+    const uint32_t slot = (q & 1u) ? w.pmin[index] : w.pmaj[index];
+    const uint32_t body = w.owner[slot];
+    const dyn_collider col = w.co[slot];
+    const dyn_body_state st = w.st[body];
+    c.shapes = quad_pair(world_collider(st, col), q);
+    c.margin = w.p.contact_margin;
+    const uint32_t flags = w.de[body].flags;
+    const v3 velocity = ld3(st.velocity);
+    const v3 first = dpp_v3<kQuadSideFirst>(velocity), second = dpp_v3<kQuadSideSecond>(velocity);
+    if ((dpp_u32<kQuadSideFirst>(flags) | dpp_u32<kQuadSideSecond>(flags)) & DYN_BODY_CCD) {
+        c.margin += len3(sub(second, first)) * w.p.dt;  // pair_margin
+    }
+    return c;
+}
+
+__device__ inline ConvexPair<ThreadPair> load_thread_pair(const W& w, uint32_t index) {
+    ConvexPair<ThreadPair> c;
     c.index = index;
     const uint32_t fs = w.pmaj[index], ss = w.pmin[index];
     const uint32_t fb = w.owner[fs], sb = w.owner[ss];
@@ -819,28 +864,29 @@ __device__ inline ConvexPair load_convex_pair(const W& w, uint32_t index) {
     if ((w.de[fb].flags & DYN_BODY_CCD) || (w.de[sb].flags & DYN_BODY_CCD)) {
         c.margin += len3(sub(ld3(sst.velocity), ld3(fst.velocity))) * w.p.dt;  // pair_margin
     }
-    c.first = world_collider(fst, fc);
-    c.second = world_collider(sst, sc);
+    c.shapes = thread_pair(world_collider(fst, fc), world_collider(sst, sc));
     return c;
 }
 
 // The rest of convex_hit once GJK has answered: a penetrating pair's simplex is parked for
-// k_narrow_epa, a hit within the margin for k_narrow_finish; separated pairs end here.
-__device__ inline void convex_pair_after_gjk(const W& w, const ConvexPair& c, const ShapeSet& shapes,
+// EPA, a hit within the margin for k_narrow_finish; separated pairs end here.
+template <typename Pair>
+__device__ inline void convex_pair_after_gjk(const W& w, const ConvexPair<Pair>& c, uint32_t q, const ShapeSet& shapes,
                                              const Closest& closest, const GjkState& g) {
     Hit hit;
     float* park = parked(w, c.index);
-    if (!convex_hit_after_gjk<1>(c.first, c.second, shapes, closest, &hit, g.simplex, &g.count)) {
+    if (!convex_hit_after_gjk(c.shapes, shapes, closest, &hit, g.simplex, g.count)) {
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
+            if (!parks_slot(q, i)) continue;
             park[3 * i] = g.simplex[i].w.x;
             park[3 * i + 1] = g.simplex[i].w.y;
             park[3 * i + 2] = g.simplex[i].w.z;
         }
-        w.valid[c.index] = kPairEpa;
+        if (parks_rest(q)) w.valid[c.index] = kPairEpa;
         return;
     }
-    if (!(hit.distance <= c.margin)) return;
+    if (!parks_rest(q) || !(hit.distance <= c.margin)) return;
     park[0] = hit.distance;
     park[1] = hit.point.x;
     park[2] = hit.point.y;
@@ -851,51 +897,67 @@ __device__ inline void convex_pair_after_gjk(const W& w, const ConvexPair& c, co
     w.valid[c.index] = kPairHit;
 }
 
-// GJK of the pairs marked kPairGjk (convex_hit, convex.wgsl:584-618), one thread per pair of the
-// worklist, for its first kGjkFirstIterations iterations: a pair GJK answers by then goes on to
-// the probe and is parked for EPA or the manifold kernel (or ends); a pair that needs more parks
-// its GJK state for k_narrow_convex_resume.
-// Three waves a SIMD (168 registers, a few spilled): the loop is vector-ALU bound and the third
-// wave hides more of its latency than the spills cost (k_narrow_convex 708 -> 627 us and the
-// resume kernel 338 -> 277 us on the settled 100k pile; four waves, 128 registers, were slower).
-__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w) {
-    __shared__ BlockLists<1> lists;
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t total = w.work_total[kTotalGjk];
-    if (blockIdx.x * blockDim.x >= total) return;
-    lists.begin();
-    uint32_t index = 0u, list = kNoList;
-    if (t < total) {
-        index = w.work_minor[t];
-        w.valid[index] = kPairNone;
-        const ConvexPair c = load_convex_pair(w, index);
-        const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
-        GjkState g;
-        gjk_begin<1>(c.first, c.second, shapes, &g);
-        Closest closest;
-        if (gjk_run<1>(c.first, c.second, shapes, &g, kGjkFirstIterations, &closest)) {
-            convex_pair_after_gjk(w, c, shapes, closest, g);
-        } else {
-            park_gjk(parked(w, index), g);
-            list = 0u;
-        }
+// A pair's first GJK iterations; true when it needs more, its state parked.
+template <typename Pair>
+__device__ inline bool narrow_convex_pair(const W& w, const ConvexPair<Pair>& c, uint32_t q) {
+    const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
+    GjkState g;
+    gjk_begin(c.shapes, shapes, &g);
+    Closest closest;
+    if (gjk_run(c.shapes, shapes, &g, kGjkFirstIterations, &closest)) {
+        convex_pair_after_gjk(w, c, q, shapes, closest, g);
+        return false;
     }
-    lists.finish(list, index, false, nullptr, {{&w.work_total[kTotalResume], w.worklist, 0u}});
+    park_gjk(parked(w, c.index), g, q);
+    return true;
 }
 
-// The remaining GJK iterations of the pairs k_narrow_convex parked, from their
-// parked state, then the rest of convex_hit as in k_narrow_convex.
+// GJK of the pairs marked kPairGjk (convex_hit, convex.wgsl:584-618), a quad per pair or (in a long
+// list) a thread, for its first kGjkFirstIterations iterations: a pair GJK answers by then goes on to
+// the probe and is parked for EPA or the manifold kernel (or ends); a pair that needs more parks its
+// GJK state for k_narrow_convex_resume.
+// Three waves a SIMD (168 registers, a few spilled): the loop is vector-ALU bound and the third
+// wave hides more of its latency than the spills cost (708 -> 627 us on a settled 100k pile; four
+// waves, 128 registers, were slower).
+__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w) {
+    __shared__ BlockLists<1> lists;
+    const uint32_t total = w.work_total[kTotalGjk];
+    const bool quads = total <= kLongGjk;
+    if (blockIdx.x * (quads ? kQuadPairs : kThreads) >= total) return;
+    lists.begin();
+    uint32_t index = 0u;
+    bool open = false;
+    if (quads) {
+        const uint32_t t = blockIdx.x * kQuadPairs + threadIdx.x / kQuad, q = threadIdx.x % kQuad;
+        if (t < total) {
+            index = w.work_minor[t];
+            if (q == 0u) w.valid[index] = kPairNone;
+            open = narrow_convex_pair(w, load_quad_pair(w, index, q), q) && q == 0u;
+        }
+    } else {
+        const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
+        if (t < total) {
+            index = w.work_minor[t];
+            w.valid[index] = kPairNone;
+            open = narrow_convex_pair(w, load_thread_pair(w, index), kWholePair);
+        }
+    }
+    lists.finish(open ? 0u : kNoList, index, false, nullptr, {{&w.work_total[kTotalResume], w.worklist, 0u}});
+}
+
+// The remaining GJK iterations of the pairs k_narrow_convex parked, a quad per pair, from their parked
+// state, then the rest of convex_hit as in k_narrow_convex.
 __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) / kQuad, q = threadIdx.x % kQuad;
     if (t >= w.work_total[kTotalResume]) return;
     const uint32_t index = w.worklist[t];
-    const ConvexPair c = load_convex_pair(w, index);
+    const ConvexPair<QuadPair> c = load_quad_pair(w, index, q);
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     GjkState g;
     unpark_gjk(parked(w, index), &g);
     Closest closest;
-    gjk_run<1>(c.first, c.second, shapes, &g, kGjkIterations, &closest);
-    convex_pair_after_gjk(w, c, shapes, closest, g);
+    gjk_run(c.shapes, shapes, &g, kGjkIterations, &closest);
+    convex_pair_after_gjk(w, c, q, shapes, closest, g);
 }
 
 // After GJK: its penetrating pairs to the front of worklist, its hits to the end.
@@ -3175,8 +3237,9 @@ int narrowphase(const dyn::W& w, hipStream_t st, bool convex, const SideStream* 
     DYN_TRY(class_worklist(w, st));
     LAUNCH_ON(st, k_narrow, pb, w);
     if (!convex) return DYN_OK;
-    LAUNCH_ON(st, k_narrow_convex, pb, w);
-    LAUNCH_ON(st, k_narrow_convex_resume, pb, w);
+    const uint32_t qb = ceil_div(static_cast<uint64_t>(w.pair_cap ? w.pair_cap : 1u) * kQuad, kThreads);
+    LAUNCH_ON(st, k_narrow_convex, qb, w);
+    LAUNCH_ON(st, k_narrow_convex_resume, qb, w);
     LAUNCH_ON(st, k_work_split, pb, w);
     {
         constexpr uint32_t kPairsPerBlock = kEpaWaves * kWave / kEpaGroup;

@@ -1,0 +1,57 @@
+"""The narrowphase's pair lists and its two kinds of GJK at their edges: pair capacities on both sides of
+the one-workgroup grouping, and a list long enough for one thread a pair (above 131,072 GJK pairs). The
+same pairs repeated give the same contacts in every copy, and the first copy is held to the oracle by
+the stage's own tests."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from dynamis_amd.narrowphase import Narrowphase
+from dynamis_amd.world import World
+from tests.narrow_cases import DT, pile_scene, with_states
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pile(device):
+    scene = pile_scene(3000, seed=5, hull_sources=64, spacing=1.5)
+    with World() as world:
+        world.create(scene)
+        for _ in range(60):
+            world.step(DT)
+        return with_states(scene, world.states()), world.pairs()
+
+
+def run(scene, pairs, capacity):
+    stage = Narrowphase(scene, capacity)
+    stage.run(pairs)
+    raw, valid = stage.read()
+    return raw, valid
+
+
+@pytest.mark.parametrize("count,capacity", [(1, 1), (255, 256), (257, 16384), (257, 16385), (4097, 16384),
+                                            (4097, 16385), (5000, 70001)])
+def test_capacities(pile, count, capacity):
+    scene, pairs = pile
+    pairs = pairs[:: max(1, len(pairs) // count)][:count]
+    want_raw, want_valid = run(scene, pairs, 65536)
+    raw, valid = run(scene, pairs, capacity)
+    assert np.array_equal(valid, want_valid)
+    hit = valid == 1
+    assert raw[hit].tobytes() == want_raw[hit].tobytes()
+
+
+def test_long_list(pile):
+    scene, pairs = pile
+    want_raw, want_valid = run(scene, pairs, len(pairs))
+    hit = want_valid == 1
+    assert hit.sum() > 1000
+    copies = 1 + 700000 // len(pairs)  # about a third of the pairs go to GJK
+    raw, valid = run(scene, np.tile(pairs, (copies, 1)), copies * len(pairs))
+    for c in range(copies):
+        part = slice(c * len(pairs), (c + 1) * len(pairs))
+        assert np.array_equal(valid[part], want_valid)
+        assert raw[part][hit].tobytes() == want_raw[hit].tobytes()
