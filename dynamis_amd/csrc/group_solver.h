@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(T) k_group_solve(W w, const GroupWorld* worlds
     if (t == 0u && totals[1]) atomicAdd(cw(w.counters, DYN_COUNTER_SOLVER_ROWS), totals[1]);
     uint32_t linear = 0, angular = 0;
     for (uint32_t sub = 0; sub < w.p.substeps; ++sub) {
-        // k_integrate, k_solver_bodies
+        // k_integrate
         for (uint32_t r = t; r < l.rows; r += T) {
             const uint32_t row = l.global(r);
             if (r < l.g.dynamic_count) integrate_at(w, row);

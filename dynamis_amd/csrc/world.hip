@@ -94,7 +94,6 @@ struct W {
                            // then the classes' totals
     uint32_t* work_total;  // device words: the lists' lengths (WorkTotal)
     uint32_t* work_minor;  // pair lists: GJK's pairs, then the wave EPA's (front), the plane pairs (from the end)
-    uint32_t* dest;
     dyn_contact* contacts;
     uint2* ckeys;          // per contact: its collider pair (a, b), the key the relay searches
     uint32_t* matched;
@@ -145,7 +144,8 @@ struct W {
                             // position pass
     uint32_t* contrib;      // inert rows: marked when a block of theirs contributed
     uint32_t* scan_blocks;   // per-block sums of compaction scans
-    uint32_t* scan_total;    // two words: totals of the last scans
+    uint32_t* scan_total;    // totals of the compactions' scanned block sums
+    uint32_t* list_cursor;   // the next free list entry while k_rows_count places the rows' runs
     uint32_t* relay_src;     // while a tape is recorded: per contact point, the archive point relayed into it
     // Body edits queued by dyn_world_edit for the next step: runs (row, first edit, edit count)
     // sorted by row over the edits in queue order; *edit_runs_count runs (0: no edits).
@@ -259,9 +259,18 @@ __device__ inline void apply_edits(const W& w, uint32_t row, dyn_body_state& s, 
     }
 }
 
+// The island pass's start: every simulated row its own island (island_init.wgsl).
+__device__ __forceinline__ void island_reset_at(const W& w, uint32_t i) {
+    if (i < kFlattenPasses * kFlattenFlags) w.flat_flags[i] = 0u;  // launched with at least kThreads lanes
+    if (i >= w.d) return;
+    w.parents[i] = i;
+    w.istate[i] = 0u;
+}
+
 // clear_inputs.wgsl, body_edits.wgsl, activity.wgsl (all rows), begin_step.wgsl (dynamic rows)
 __global__ void __launch_bounds__(kThreads) k_begin(W w) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    island_reset_at(w, i);
     bool awake = false;
     if (i < w.n) {
         dyn_body_state s = w.st[i];
@@ -1120,114 +1129,125 @@ __global__ void __launch_bounds__(kThreads, 4) k_narrow_finish_tail(W w) {
 constexpr int kScanItems = 4;
 constexpr int kScanBlock = kThreads * kScanItems;  // 1024 flags per block
 
-// flags[i] for i < *count (or < limit when count is null); with kCounts the values are counts
-// and the scan sums them instead of the set flags.
-template <bool kCounts>
-__global__ void __launch_bounds__(kThreads) k_scan_count(const uint32_t* __restrict__ flags,
-                                                         const uint32_t* count, uint32_t limit,
-                                                         uint32_t* block_sums) {
+// The set flags of each kScanBlock of flags[i], i < *count.
+__global__ void __launch_bounds__(kThreads) k_scan_count(const uint32_t* __restrict__ flags, const uint32_t* count,
+                                                         uint32_t limit, uint32_t* block_sums) {
     __shared__ uint32_t s_scan[kThreads / kWave];
-    const uint32_t n = count ? min(*count, limit) : limit;
+    const uint32_t n = min(*count, limit);
     const uint32_t first = blockIdx.x * kScanBlock + threadIdx.x * kScanItems;
     uint32_t sum = 0;
 #pragma unroll
     for (int j = 0; j < kScanItems; ++j) {
         const uint32_t i = first + j;
-        if (i < n) sum += kCounts ? flags[i] : (flags[i] ? 1u : 0u);
+        if (i < n) sum += flags[i] ? 1u : 0u;
     }
     uint32_t total = 0;
     block_exclusive_sum<kThreads>(sum, s_scan, &total);
     if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
 }
 
-__global__ void __launch_bounds__(1024) k_scan_blocks(uint32_t* block_sums, uint32_t blocks,
-                                                      uint32_t* total_out) {
+// Block sums of a compaction. The pass that moves the records adds up the sums before its block by
+// itself where there are few (a launch saved); more than kInlineSums are scanned first
+// (k_scan_blocks): every block would read half of them.
+constexpr uint32_t kInlineSums = 4096;
+struct ScanSums {
+    uint32_t* sums;
+    uint32_t groups;   // sums of kScanBlock flags each
+    uint32_t* total;   // set by k_scan_blocks
+    __host__ __device__ bool scanned() const { return groups > kInlineSums; }
+};
+
+__global__ void __launch_bounds__(1024) k_scan_blocks(ScanSums a, ScanSums b) {
     __shared__ uint32_t s_scan[1024 / kWave];
     __shared__ uint32_t s_carry;
+    const ScanSums s = blockIdx.x == 0 ? a : b;
     if (threadIdx.x == 0) s_carry = 0;
-    for (uint32_t first = 0; first < blocks; first += 1024) {
-        const uint32_t b = first + threadIdx.x;
-        const uint32_t v = b < blocks ? block_sums[b] : 0u;
+    for (uint32_t first = 0; first < s.groups; first += 1024) {
+        const uint32_t g = first + threadIdx.x;
+        const uint32_t v = g < s.groups ? s.sums[g] : 0u;
         uint32_t total = 0;
         const uint32_t excl = block_exclusive_sum<1024>(v, s_scan, &total);
-        if (b < blocks) block_sums[b] = s_carry + excl;
+        if (g < s.groups) s.sums[g] = s_carry + excl;
         __syncthreads();
         if (threadIdx.x == 0) s_carry += total;
         __syncthreads();
     }
-    if (threadIdx.x == 0) *total_out = s_carry;
+    if (threadIdx.x == 0) *s.total = s_carry;
 }
 
-// dest[i] = rank of flag i among set flags (kNoSlot when clear), or with kCounts the sum of
-// the counts before i; the same partition as k_scan_count, whose block sums k_scan_blocks
-// turned into offsets.
-template <bool kCounts>
-__global__ void __launch_bounds__(kThreads) k_scan_dest(const uint32_t* __restrict__ flags,
-                                                        const uint32_t* count, uint32_t limit,
-                                                        const uint32_t* __restrict__ block_offsets,
-                                                        uint32_t* dest) {
-    __shared__ uint32_t s_scan[kThreads / kWave];
-    const uint32_t n = count ? min(*count, limit) : limit;
-    const uint32_t first = blockIdx.x * kScanBlock + threadIdx.x * kScanItems;
-    uint32_t f[kScanItems];
-    uint32_t sum = 0;
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        const uint32_t i = first + j;
-        f[j] = i < n ? (kCounts ? flags[i] : (flags[i] ? 1u : 0u)) : 0u;
-        sum += f[j];
+// For the workgroup of flags [first, first + kThreads): the set flags before `first`, and (with `all`)
+// of the whole list. Every lane calls it.
+__device__ inline uint32_t scan_before(const ScanSums& s, const uint32_t* __restrict__ flags, uint32_t live,
+                                       uint32_t first, uint32_t* s_scan, uint32_t* all) {
+    const uint32_t group = first / kScanBlock;
+    uint32_t before = 0, rest = 0;
+    for (uint32_t i = group * kScanBlock + threadIdx.x; i < first; i += kThreads) {  // its group's flags before it
+        if (i < live && flags[i]) ++before;
     }
-    uint32_t at = block_offsets[blockIdx.x] + block_exclusive_sum<kThreads>(sum, s_scan, nullptr);
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        const uint32_t i = first + j;
-        if (i < n) {
-            dest[i] = (kCounts || f[j]) ? at : kNoSlot;
-            at += f[j];
+    if (!s.scanned()) {
+        const uint32_t end = all ? s.groups : min(group, s.groups);
+        for (uint32_t g = threadIdx.x; g < end; g += kThreads) {
+            const uint32_t v = s.sums[g];
+            if (g < group) before += v;
+            else rest += v;
         }
     }
+    uint32_t total = 0;
+    block_exclusive_sum<kThreads>(before, s_scan, &total);
+    uint32_t base = total;
+    if (s.scanned()) {
+        if (group < s.groups) base += s.sums[group];
+        if (all) *all = *s.total;
+    } else if (all) {
+        uint32_t partial = 0;
+        for (uint32_t i = group * kScanBlock + threadIdx.x; i < first; i += kThreads) {
+            if (i < live && flags[i]) ++partial;
+        }
+        uint32_t in_group = 0;
+        block_exclusive_sum<kThreads>(partial, s_scan, &in_group);
+        block_exclusive_sum<kThreads>(rest, s_scan, &total);
+        *all = base - in_group + total;
+    }
+    return base;
 }
 
 // compact_scatter.wgsl: valid raw contacts in pair order; carried impulses cleared (the raw
 // record already has them at zero).
-// The workgroup lists its pairs' (raw slot, destination) and copies the records together, its
-// lanes on consecutive 16-byte pieces, instead of each lane walking its own 352-byte record.
+// The workgroup lists its pairs' raw slots, which go to consecutive contacts, and copies the records
+// together, its lanes on consecutive 16-byte pieces, instead of each lane walking its own 352-byte
+// record. The last workgroup writes the totals.
 static_assert(sizeof(dyn_contact) % sizeof(float4) == 0, "contacts copy in 16-byte pieces");
-__global__ void __launch_bounds__(kThreads) k_contacts_scatter(W w) {
+__global__ void __launch_bounds__(kThreads) k_contacts_scatter(W w, ScanSums sums) {
     constexpr uint32_t kPieces = sizeof(dyn_contact) / sizeof(float4);
-    __shared__ uint2 job[kThreads];
-    __shared__ uint32_t jobs;
-    if (threadIdx.x == 0) jobs = 0u;
-    __syncthreads();
-    const uint32_t index = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint32_t job[kThreads];
+    __shared__ uint32_t s_scan[kThreads / kWave];
+    const uint32_t first = blockIdx.x * kThreads, index = first + threadIdx.x;
     const uint32_t live = min(*cw(w.counters, DYN_COUNTER_PAIRS), w.pair_cap);
-    if (index < live && w.valid[index] == kPairContact) {
-        const uint32_t at = w.dest[index];
-        if (at < w.contact_cap) job[atomicAdd(&jobs, 1u)] = make_uint2(index, at);
+    const bool last = blockIdx.x + 1u == gridDim.x;
+    if (first >= live && !last) return;
+    const uint32_t base = scan_before(sums, w.valid, live, first, s_scan, nullptr);
+    const bool mine = index < live && w.valid[index] == kPairContact;
+    uint32_t found = 0;
+    const uint32_t rank = block_exclusive_sum<kThreads>(mine ? 1u : 0u, s_scan, &found);
+    if (mine) job[rank] = index;
+    if (last && threadIdx.x == 0) {
+        const uint32_t total = base + found, kept = min(total, w.contact_cap);
+        *cw(w.counters, DYN_COUNTER_CONTACTS) = total;
+        *cw(w.counters, DYN_COUNTER_REFUSED_CONTACTS) = total - kept;
+        *w.ncontacts = kept;
+        *cw(w.counters, DYN_COUNTER_BLOCKS) = kept;
     }
     __syncthreads();
-    const uint32_t n = jobs;
-    for (uint32_t item = threadIdx.x; item < n * kPieces; item += blockDim.x) {
+    const uint32_t n = base < w.contact_cap ? min(found, w.contact_cap - base) : 0u;
+    for (uint32_t item = threadIdx.x; item < n * kPieces; item += kThreads) {
         const uint32_t k = item / kPieces, piece = item - k * kPieces;
-        const uint2 jb = job[k];
-        reinterpret_cast<float4*>(w.contacts + jb.y)[piece] = reinterpret_cast<const float4*>(w.raw + jb.x)[piece];
+        reinterpret_cast<float4*>(w.contacts + base + k)[piece] = reinterpret_cast<const float4*>(w.raw + job[k])[piece];
     }
     if (threadIdx.x < n) {
-        const uint2 jb = job[threadIdx.x];
-        const dyn_contact& c = w.raw[jb.x];
-        w.ckeys[jb.y] = make_uint2(c.a, c.b);
-        w.matched[jb.y] = 0u;
+        const dyn_contact& c = w.raw[job[threadIdx.x]];
+        w.ckeys[base + threadIdx.x] = make_uint2(c.a, c.b);
+        w.matched[base + threadIdx.x] = 0u;
     }
-}
-
-__global__ void k_contacts_total(W w) {
-    if (threadIdx.x != 0) return;
-    const uint32_t total = w.scan_total[0];
-    *cw(w.counters, DYN_COUNTER_CONTACTS) = total;
-    const uint32_t kept = min(total, w.contact_cap);
-    *cw(w.counters, DYN_COUNTER_REFUSED_CONTACTS) = total - kept;
-    *w.ncontacts = kept;
-    *cw(w.counters, DYN_COUNTER_BLOCKS) = kept;
 }
 
 // ---- warm start and identity (identity.wgsl, contact_relay.wgsl, contact_begin.wgsl) ------
@@ -1548,11 +1568,7 @@ __global__ void __launch_bounds__(kThreads) k_tape_record(W w, float* states, fl
 // ---- islands (island_*.wgsl) ------------------------------------------------------------------
 
 __global__ void __launch_bounds__(kThreads) k_island_init(W w) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < kFlattenPasses * kFlattenFlags) w.flat_flags[i] = 0u;  // launched with at least kThreads lanes
-    if (i >= w.d) return;
-    w.parents[i] = i;
-    w.istate[i] = 0u;
+    island_reset_at(w, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // The root of a node by a read-only walk. Halving the path on the way (pointing each visited
@@ -1617,6 +1633,12 @@ __device__ __forceinline__ uint2 island_edge_at(const W& w, uint32_t i, float sl
 // seeding and hooking rounds most contacts' rows share a parent and return at once.
 __global__ void __launch_bounds__(kThreads) k_island_link(W w, float slop) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w.nresting && i < *w.nresting) {  // a world's resting archive (the stage has none)
+        const dyn_contact& c = w.resting[i];
+        const uint32_t r1 = resolve_row(w, c.first_body_id, c.first_generation);
+        const uint32_t r2 = resolve_row(w, c.second_body_id, c.second_generation);
+        if (r1 != DYN_NO_BODY && r2 != DYN_NO_BODY) island_couple(w, r1, r2);
+    }
     if (i >= min(*w.ncontacts, w.contact_cap)) return;
     const uint2 e = island_edge_at(w, i, slop);
     if (e.x == kNoSlot) return;
@@ -1719,16 +1741,6 @@ __global__ void __launch_bounds__(kThreads) k_islands_stage_reset(W w) {
         *cw(w.counters, DYN_COUNTER_ISLANDS) = 0u;
         *cw(w.counters, DYN_COUNTER_ISLAND_FAULTS) = 0u;
     }
-}
-
-__global__ void __launch_bounds__(kThreads) k_island_link_resting(W w) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *w.nresting) return;
-    const dyn_contact& c = w.resting[i];
-    const uint32_t r1 = resolve_row(w, c.first_body_id, c.first_generation);
-    const uint32_t r2 = resolve_row(w, c.second_body_id, c.second_generation);
-    if (r1 == DYN_NO_BODY || r2 == DYN_NO_BODY) return;
-    island_couple(w, r1, r2);
 }
 
 // island_flatten.wgsl, with walks of up to kFlattenHops hops in place of one: round `round` of a
@@ -1853,6 +1865,7 @@ __device__ __forceinline__ void write_block_body(const W& w, uint32_t row, const
 
 // live.wgsl count, solver_reset.wgsl
 __global__ void __launch_bounds__(kThreads) k_solver_reset(W w) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *w.list_cursor = 0u;
     uint32_t live = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < w.n; i += gridDim.x * blockDim.x) {
         w.block_counts[i] = 0u;
@@ -1936,13 +1949,40 @@ __global__ void __launch_bounds__(kThreads) k_blocks(W w) {
     w.slots[2 * i + 1] = slot_s;
 }
 
+// Every row's list length and first entry. A row's run may lie anywhere, so a workgroup takes the
+// entries of its rows with one atomic instead of a scan over all rows (three launches saved).
+constexpr uint32_t kRowItems = 4;
 __global__ void __launch_bounds__(kThreads) k_rows_count(W w) {
+    __shared__ uint32_t s_scan[kThreads / kWave];
+    __shared__ uint32_t s_first;
     uint32_t claimed = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < w.n; i += gridDim.x * blockDim.x) {
-        const uint32_t blocks = w.block_counts[i];
-        const bool listed = blocks != 0u && !(!kind_simulates(w.de[i]) || w.st[i].sleeping != 0u);
-        w.list_counts[i] = listed ? blocks : 0u;
-        claimed += blocks != 0u ? 1u : 0u;
+    for (uint32_t base = blockIdx.x * kThreads * kRowItems; base < w.n; base += gridDim.x * kThreads * kRowItems) {
+        uint32_t length[kRowItems];
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kRowItems; ++j) {
+            const uint32_t i = base + threadIdx.x * kRowItems + j;
+            length[j] = 0u;
+            if (i >= w.n) continue;
+            const uint32_t blocks = w.block_counts[i];
+            const bool listed = blocks != 0u && !(!kind_simulates(w.de[i]) || w.st[i].sleeping != 0u);
+            length[j] = listed ? blocks : 0u;
+            w.list_counts[i] = length[j];
+            sum += length[j];
+            claimed += blocks != 0u ? 1u : 0u;
+        }
+        uint32_t total = 0;
+        uint32_t at = block_exclusive_sum<kThreads>(sum, s_scan, &total);
+        if (threadIdx.x == 0) s_first = total ? atomicAdd(w.list_cursor, total) : 0u;
+        __syncthreads();
+        at += s_first;
+#pragma unroll
+        for (uint32_t j = 0; j < kRowItems; ++j) {
+            const uint32_t i = base + threadIdx.x * kRowItems + j;
+            if (i < w.n) w.row_start[i] = at;
+            at += length[j];
+        }
+        __syncthreads();
     }
     block_count(cw(w.counters, DYN_COUNTER_SOLVER_ROWS), claimed);
 }
@@ -2026,7 +2066,7 @@ __device__ __forceinline__ float normal_delta(float relaxation, float damping_ra
 //
 // Within one substep's iterations (solver_block_solve.wgsl:56-101) only the velocities and the
 // accumulated impulses change: the bodies' poses, the masses, the split counts and every
-// quantity of a block built from them stay put. k_solver_bodies and k_solve_prep evaluate those
+// quantity of a block built from them stay put. k_integrate and k_solve_prep evaluate those
 // once per substep with exactly the expressions solver_contact_block.wgsl evaluates in every
 // iteration, and k_solve reads them back, so the iterations produce the same bits.
 
@@ -2129,10 +2169,6 @@ __device__ __forceinline__ Body posed_body(const W& w, uint32_t row, bool* inert
     return b;
 }
 
-__global__ void __launch_bounds__(kThreads) k_solver_bodies(W w) {
-    solver_bodies_at(w, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
 // Where the launched passes' block deltas go: the block's words (commit_block).
 struct WordCommit {
     const W& w;
@@ -2171,10 +2207,6 @@ __device__ __forceinline__ void warm_block(const W& w, uint32_t ci, const Commit
 __device__ __forceinline__ void warm_at(const W& w, uint32_t ci) {
     if (ci >= *w.ncontacts) return;
     warm_block(w, ci, WordCommit{w, ci, false});
-}
-
-__global__ void __launch_bounds__(kThreads) k_warm(W w) {
-    warm_at(w, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // A block's point pi: its local anchors and depth, from the contact record or from the copy the
@@ -2281,7 +2313,9 @@ __device__ __forceinline__ void solve_prep_at(const W& w, uint32_t ci, uint32_t 
 }
 
 __global__ void __launch_bounds__(kThreads) k_solve_prep(W w, uint32_t load_impulses) {
-    solve_prep_at(w, blockIdx.x * blockDim.x + threadIdx.x, load_impulses);
+    const uint32_t ci = blockIdx.x * blockDim.x + threadIdx.x;
+    solve_prep_at(w, ci, load_impulses);
+    if (load_impulses) warm_at(w, ci);  // the step's first substep starts from the impulses
 }
 
 // solver_contact_block.wgsl:31-193 over the block's row: the points' impulses are applied as
@@ -2432,7 +2466,7 @@ __global__ void __launch_bounds__(kThreads) k_impulses_store(W w) {
 // (integer sums: any order gives the same words).
 constexpr uint32_t kApplyBatch = 8;
 
-// The velocities live in the row's solver record (k_solver_bodies copies them from the body
+// The velocities live in the row's solver record (k_integrate copies them from the body
 // state at the substep's start) while the iterations run: only the substep's last apply
 // (`commit`) writes them to the body state, for every claimed row, as the same bits an update of
 // both after every apply would leave there.
@@ -2445,7 +2479,23 @@ __device__ __forceinline__ uint32_t row_lanes_sum(uint32_t v, uint32_t lanes_log
     return v;
 }
 
-__device__ __forceinline__ void apply_at(const W& w, uint32_t t, uint32_t commit, uint32_t lanes_log2) {
+// substep_advance.wgsl
+__device__ __forceinline__ void advance_at(const W& w, uint32_t row) {
+    if (row >= w.d) return;
+    dyn_body_state s = w.st[row];
+    if (!body_is_active(s, w.de[row])) return;
+    const float h = w.p.substep_dt;
+    st3(s.position, add(ld3(s.position), mul(ld3(s.velocity), h)));
+    const q4 spin = make_float4(s.angular_velocity[0], s.angular_velocity[1], s.angular_velocity[2], 0.0f);
+    const q4 q = ld4(s.orientation);
+    const q4 dq = qmul(spin, q);
+    const float k = 0.5f * h;
+    st4(s.orientation, qnorm(make_float4(q.x + k * dq.x, q.y + k * dq.y, q.z + k * dq.z, q.w + k * dq.w)));
+    w.st[row] = s;
+}
+
+__device__ __forceinline__ void apply_at(const W& w, uint32_t t, uint32_t commit, uint32_t advance,
+                                         uint32_t lanes_log2) {
     const uint32_t lanes = 1u << lanes_log2;
     const uint32_t row = t >> lanes_log2, sub = t & (lanes - 1u);
     const bool live = row < w.n;
@@ -2495,7 +2545,11 @@ __device__ __forceinline__ void apply_at(const W& w, uint32_t t, uint32_t commit
         s4 = row_lanes_sum(s4, lanes_log2);
         s5 = row_lanes_sum(s5, lanes_log2);
     }
-    if (sub != 0u || count == 0u) return;
+    if (sub != 0u || !live) return;
+    if (count == 0u) {
+        if (advance) advance_at(w, row);
+        return;
+    }
     v3 v = v0, av = av0;
     if ((s0 | s1 | s2 | s3 | s4 | s5) != 0u) {
         const v3 lin = mk(solver_value(s0, DYN_SOLVER_VELOCITY_SCALE), solver_value(s1, DYN_SOLVER_VELOCITY_SCALE),
@@ -2514,10 +2568,11 @@ __device__ __forceinline__ void apply_at(const W& w, uint32_t t, uint32_t commit
         st3(s.velocity, v);
         st3(s.angular_velocity, av);
     }
+    if (advance) advance_at(w, row);
 }
 
-__global__ void __launch_bounds__(kThreads) k_apply(W w, uint32_t commit, uint32_t lanes_log2) {
-    apply_at(w, blockIdx.x * blockDim.x + threadIdx.x, commit, lanes_log2);
+__global__ void __launch_bounds__(kThreads) k_apply(W w, uint32_t commit, uint32_t advance, uint32_t lanes_log2) {
+    apply_at(w, blockIdx.x * blockDim.x + threadIdx.x, commit, advance, lanes_log2);
 }
 
 // substep_integrate.wgsl:15-76 over the awake dynamic rows (no fields)
@@ -2559,23 +2614,11 @@ __device__ __forceinline__ void integrate_at(const W& w, uint32_t row) {
     w.st[row] = s;
 }
 
+// A substep's start for every row: integration, then what its blocks read of the row.
 __global__ void __launch_bounds__(kThreads) k_integrate(W w) {
-    integrate_at(w, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// substep_advance.wgsl
-__device__ __forceinline__ void advance_at(const W& w, uint32_t row) {
-    if (row >= w.d) return;
-    dyn_body_state s = w.st[row];
-    if (!body_is_active(s, w.de[row])) return;
-    const float h = w.p.substep_dt;
-    st3(s.position, add(ld3(s.position), mul(ld3(s.velocity), h)));
-    const q4 spin = make_float4(s.angular_velocity[0], s.angular_velocity[1], s.angular_velocity[2], 0.0f);
-    const q4 q = ld4(s.orientation);
-    const q4 dq = qmul(spin, q);
-    const float k = 0.5f * h;
-    st4(s.orientation, qnorm(make_float4(q.x + k * dq.x, q.y + k * dq.y, q.z + k * dq.z, q.w + k * dq.w)));
-    w.st[row] = s;
+    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
+    integrate_at(w, row);
+    solver_bodies_at(w, row);
 }
 
 __global__ void __launch_bounds__(kThreads) k_advance(W w) {
@@ -2796,105 +2839,113 @@ __global__ void __launch_bounds__(kThreads) k_sleep(W w) {
 
 // ---- commit: thaw, archive, static wake clear, freeze (commit.rs:187-209) ---------------
 
-// rest_flags[i] = keep resting manifold i (both bodies inactive at the step's start)
-__global__ void __launch_bounds__(kThreads) k_thaw(W w) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *w.nresting) return;
+// Whether resting manifold i stays (both bodies inactive at the step's start).
+__device__ __forceinline__ bool keeps_resting(const W& w, uint32_t i) {
     const dyn_contact& c = w.resting[i];
     const uint32_t r1 = resolve_row(w, c.first_body_id, c.first_generation);
     const uint32_t r2 = resolve_row(w, c.second_body_id, c.second_generation);
-    const bool keep = r1 != DYN_NO_BODY && r2 != DYN_NO_BODY && w.activity[r1] == 0u && w.activity[r2] == 0u;
-    w.rest_flags[i] = keep ? 1u : 0u;
+    return r1 != DYN_NO_BODY && r2 != DYN_NO_BODY && w.activity[r1] == 0u && w.activity[r2] == 0u;
 }
 
-// contact_archive.wgsl + freeze_contacts.wgsl flags (freeze flags after the resting flags)
-// contact_archive.wgsl keeps the step's contacts for the next step's relay: here the contact and
-// archive buffers trade places at the end of the step (swap_contact_buffers) instead of copying,
-// so this pass only marks the contacts freeze_contacts.wgsl:13-45 moves to the resting archive.
-__global__ void __launch_bounds__(kThreads) k_archive(W w, uint32_t* freeze_flags) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *w.ncontacts) return;
-    const uint2 ab = w.ckeys[i];
-    const uint32_t f = w.owner[ab.x], s = w.owner[ab.y];
-    const bool frozen = !body_is_active(w.st[f], w.de[f]) && !body_is_active(w.st[s], w.de[s]);
-    freeze_flags[i] = frozen ? 1u : 0u;
-}
-
-__global__ void __launch_bounds__(kThreads) k_archive_count(W w) {
+// thaw_contacts.wgsl's and freeze_contacts.wgsl:13-45's marks (the resting manifolds that stay, the
+// contacts that join them) with each kScanBlock's counts, the archive's length
+// (contact_archive.wgsl keeps the step's contacts for the next step's relay: here the contact and
+// archive buffers trade places at the end of the step, swap_contact_buffers, instead of copying) and
+// static_wake_clear.wgsl.
+__global__ void __launch_bounds__(kThreads) k_archive(W w, uint32_t* freeze_flags, ScanSums kept, ScanSums frozen) {
+    __shared__ uint32_t s_scan[kThreads / kWave];
+    const uint32_t old = *w.nresting, contacts = *w.ncontacts;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *w.narchive = *w.ncontacts;
-        *cw(w.counters, DYN_COUNTER_ARCHIVED) = *w.ncontacts;
+        *w.narchive = contacts;
+        *cw(w.counters, DYN_COUNTER_ARCHIVED) = contacts;
     }
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= w.d && i < w.n) w.wake[i] = 0u;  // static_wake_clear.wgsl
+    for (uint32_t row = w.d + blockIdx.x * kThreads + threadIdx.x; row < w.n; row += gridDim.x * kThreads) w.wake[row] = 0u;
+    const uint32_t first = blockIdx.x * kScanBlock;
+    uint32_t stay = 0, join = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kScanItems; ++j) {
+        const uint32_t i = first + j * kThreads + threadIdx.x;
+        if (i < old) {
+            const bool keep = keeps_resting(w, i);
+            w.rest_flags[i] = keep ? 1u : 0u;
+            stay += keep ? 1u : 0u;
+        }
+        if (i < contacts) {
+            const uint2 ab = w.ckeys[i];
+            const uint32_t f = w.owner[ab.x], s = w.owner[ab.y];
+            const bool freeze = !body_is_active(w.st[f], w.de[f]) && !body_is_active(w.st[s], w.de[s]);
+            freeze_flags[i] = freeze ? 1u : 0u;
+            join += freeze ? 1u : 0u;
+        }
+    }
+    uint32_t total = 0;
+    block_exclusive_sum<kThreads>(stay, s_scan, &total);
+    if (threadIdx.x == 0) kept.sums[blockIdx.x] = total;
+    block_exclusive_sum<kThreads>(join, s_scan, &total);
+    if (threadIdx.x == 0) frozen.sums[blockIdx.x] = total;
 }
 
 // New resting list = kept manifolds then frozen manifolds, keyed by (min id, max id).
-__global__ void __launch_bounds__(kThreads) k_rest_gather(W w, const uint32_t* keep_dest,
-                                                          const uint32_t* keep_total,
-                                                          const uint32_t* freeze_dest,
-                                                          uint32_t* out_count) {
+__global__ void __launch_bounds__(kThreads) k_rest_gather(W w, const uint32_t* freeze_flags, ScanSums kept_sums,
+                                                          ScanSums frozen_sums, uint32_t* out_count) {
     // the workgroup lists its records (source, destination) and copies them together, its lanes
     // on consecutive 16-byte pieces
     constexpr uint32_t kPieces = sizeof(dyn_contact) / sizeof(float4);
     __shared__ const dyn_contact* from[2 * kThreads];
     __shared__ uint32_t to[2 * kThreads];
-    __shared__ uint32_t jobs;
-    if (threadIdx.x == 0) jobs = 0u;
-    __syncthreads();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t kept = *keep_total;
+    __shared__ uint32_t s_scan[kThreads / kWave];
+    const uint32_t first = blockIdx.x * kThreads, i = first + threadIdx.x;
     const uint32_t old = *w.nresting;
     const uint32_t ncont = *w.ncontacts;
+    if (first >= old && first >= ncont && blockIdx.x != 0) return;
+    uint32_t kept = 0, frozen = 0;
+    const uint32_t keep_base = scan_before(kept_sums, w.rest_flags, old, first, s_scan, &kept);
+    const uint32_t freeze_base = scan_before(frozen_sums, freeze_flags, ncont, first, s_scan, &frozen);
     if (i == 0) {
-        // freeze_dest totals are written after the map by k_scan_blocks into scan_total[1]
-        const uint32_t total = kept + w.scan_total[1];
+        const uint32_t total = kept + frozen;
         const uint32_t capped = min(total, w.contact_cap);
         *out_count = capped;
         *cw(w.counters, DYN_COUNTER_REFUSED_RESTING) = total - capped;
         *cw(w.counters, DYN_COUNTER_RESTING) = capped;
     }
-    if (i < old && keep_dest[i] != kNoSlot) {
-        const uint32_t at = keep_dest[i];
-        if (at < w.contact_cap) {
-            const dyn_contact& c = w.resting[i];
-            const uint32_t k = atomicAdd(&jobs, 1u);
-            from[k] = &c;
-            to[k] = at;
+    uint32_t jobs = 0;
+    auto list = [&](bool mine, uint32_t base, const dyn_contact* records) {
+        uint32_t found = 0;
+        const uint32_t rank = block_exclusive_sum<kThreads>(mine ? 1u : 0u, s_scan, &found);
+        const uint32_t n = base < w.contact_cap ? min(found, w.contact_cap - base) : 0u;
+        if (mine && rank < n) {
+            const uint32_t at = base + rank;
+            const dyn_contact& c = records[i];
+            from[jobs + rank] = &c;
+            to[jobs + rank] = at;
             w.rest_major[at] = min(c.first_body_id, c.second_body_id);
             w.rest_minor[at] = max(c.first_body_id, c.second_body_id);
             w.rest_slot[at] = at;
         }
-    }
-    if (i < ncont && freeze_dest[i] != kNoSlot) {
-        const uint32_t at = kept + freeze_dest[i];
-        if (at < w.contact_cap) {
-            const dyn_contact& c = w.contacts[i];
-            const uint32_t k = atomicAdd(&jobs, 1u);
-            from[k] = &c;
-            to[k] = at;
-            w.rest_major[at] = min(c.first_body_id, c.second_body_id);
-            w.rest_minor[at] = max(c.first_body_id, c.second_body_id);
-            w.rest_slot[at] = at;
-        }
-    }
+        jobs += n;
+    };
+    list(i < old && w.rest_flags[i] != 0u, keep_base, w.resting);
+    list(i < ncont && freeze_flags[i] != 0u, kept + freeze_base, w.contacts);
     __syncthreads();
-    const uint32_t n = jobs;
-    for (uint32_t item = threadIdx.x; item < n * kPieces; item += blockDim.x) {
+    for (uint32_t item = threadIdx.x; item < jobs * kPieces; item += kThreads) {
         const uint32_t k = item / kPieces, piece = item - k * kPieces;
         reinterpret_cast<float4*>(w.rest_tmp + to[k])[piece] = reinterpret_cast<const float4*>(from[k])[piece];
     }
 }
 
 // resting[i] = rest_tmp[rest_slot[i]], a workgroup's records copied together (lanes on
-// consecutive 16-byte pieces).
+// consecutive 16-byte pieces). The step's last kernel: it counts the step and drops its edits.
 __global__ void __launch_bounds__(kThreads) k_rest_place(W w, const uint32_t* count) {
     constexpr uint32_t kPieces = sizeof(dyn_contact) / sizeof(float4);
     __shared__ uint32_t from[kThreads];
     const uint32_t base = blockIdx.x * blockDim.x;
     const uint32_t i = base + threadIdx.x;
     const uint32_t n = *count;
-    if (i == 0) *w.nresting = n;
+    if (i == 0) {
+        *w.nresting = n;
+        *cw(w.counters, DYN_COUNTER_STEP) += 1u;
+        *w.edit_runs_count = 0u;  // the step applied the queued edits
+    }
     if (i < n) from[threadIdx.x] = w.rest_slot[i];
     __syncthreads();
     const uint32_t m = base < n ? min(n - base, static_cast<uint32_t>(kThreads)) : 0u;
@@ -2902,13 +2953,6 @@ __global__ void __launch_bounds__(kThreads) k_rest_place(W w, const uint32_t* co
         const uint32_t k = item / kPieces, piece = item - k * kPieces;
         reinterpret_cast<float4*>(w.resting + base + k)[piece] =
             reinterpret_cast<const float4*>(w.rest_tmp + from[k])[piece];
-    }
-}
-
-__global__ void k_consume(W w) {
-    if (threadIdx.x == 0) {
-        *cw(w.counters, DYN_COUNTER_STEP) += 1u;
-        *w.edit_runs_count = 0u;  // the step applied the queued edits
     }
 }
 
@@ -2942,8 +2986,7 @@ struct dyn_world {
     dyn_grid_entry* entries = nullptr;
     uint32_t* words = nullptr;        // small device words (counts)
     uint32_t* freeze_flags = nullptr;
-    uint32_t* keep_dest = nullptr;
-    uint32_t* freeze_dest = nullptr;
+    uint32_t* rest_blocks = nullptr;  // block sums of the resting manifolds that stay, then of those that join
     void* bp_scratch = nullptr;
     size_t bp_scratch_bytes = 0;
     void* sort_scratch = nullptr;
@@ -3036,7 +3079,6 @@ int alloc_streams(dyn_world* world, uint32_t pair_capacity, uint32_t contact_cap
     using namespace dyn;
     W& w = world->w;
     std::vector<void*>& g = world->streams;
-    const uint32_t body_count = w.n;
     int rc = DYN_OK;
 #define A(ptr, count) if (rc == DYN_OK) rc = alloc_in(g, &(ptr), (count))
     A(w.pmaj, pair_capacity);
@@ -3047,7 +3089,6 @@ int alloc_streams(dyn_world* world, uint32_t pair_capacity, uint32_t contact_cap
     A(w.worklist, pair_capacity);
     A(w.class_hist, kClasses * (static_cast<size_t>(ceil_div(pair_capacity ? pair_capacity : 1u, kClassBlock)) + 1u));
     A(w.work_minor, pair_capacity);
-    A(w.dest, pair_capacity);
     A(w.contacts, contact_capacity);
     A(w.ckeys, contact_capacity);
     A(w.matched, contact_capacity);
@@ -3069,12 +3110,9 @@ int alloc_streams(dyn_world* world, uint32_t pair_capacity, uint32_t contact_cap
     A(w.vwords, 12u * static_cast<size_t>(contact_capacity));
     A(w.pwords, 2u * static_cast<size_t>(contact_capacity));
     A(w.iedges, contact_capacity);
-    uint32_t scan_limit = pair_capacity > contact_capacity ? pair_capacity : contact_capacity;
-    if (body_count > scan_limit) scan_limit = body_count;  // the rows' list offsets
-    A(w.scan_blocks, ceil_div(scan_limit ? scan_limit : 1u, kScanBlock) + 1u);
+    A(w.scan_blocks, ceil_div(pair_capacity ? pair_capacity : 1u, kScanBlock));
     A(world->freeze_flags, contact_capacity);
-    A(world->keep_dest, contact_capacity);
-    A(world->freeze_dest, contact_capacity);
+    A(world->rest_blocks, 2u * static_cast<size_t>(ceil_div(contact_capacity ? contact_capacity : 1u, kScanBlock)));
 #undef A
     if (rc != DYN_OK) return rc;
     w.pair_cap = pair_capacity;
@@ -3153,33 +3191,16 @@ uint32_t blocks_for(uint32_t n) { return dyn::ceil_div(n ? n : 1u, dyn::kThreads
 // The grid of a row kernel that counts into a counter word (kCountBlocks).
 uint32_t count_blocks(uint32_t n) { return std::min(blocks_for(n), dyn::kCountBlocks); }
 
-int scan(const dyn::W& w, hipStream_t st, const uint32_t* flags, const uint32_t* count, uint32_t limit,
-         uint32_t* dest, uint32_t* total, bool counts = false) {
+// The scan of one or two lists' block sums, where they are too many to be added up in place.
+int scan_sums(hipStream_t st, const dyn::ScanSums& a, const dyn::ScanSums* b = nullptr) {
     using namespace dyn;
-    const uint32_t blocks = ceil_div(limit ? limit : 1u, kScanBlock);
-    {
-        ProfileScope scope("k_scan_count", st);
-        if (counts) k_scan_count<true><<<blocks, kThreads, 0, st>>>(flags, count, limit, w.scan_blocks);
-        else k_scan_count<false><<<blocks, kThreads, 0, st>>>(flags, count, limit, w.scan_blocks);
-    }
-    DYN_LAUNCHED("k_scan_count");
+    if (!a.scanned()) return DYN_OK;
     {
         ProfileScope scope("k_scan_blocks", st);
-        k_scan_blocks<<<1, 1024, 0, st>>>(w.scan_blocks, blocks, total);
+        k_scan_blocks<<<b ? 2 : 1, 1024, 0, st>>>(a, b ? *b : a);
     }
     DYN_LAUNCHED("k_scan_blocks");
-    {
-        ProfileScope scope("k_scan_dest", st);
-        if (counts) k_scan_dest<true><<<blocks, kThreads, 0, st>>>(flags, count, limit, w.scan_blocks, dest);
-        else k_scan_dest<false><<<blocks, kThreads, 0, st>>>(flags, count, limit, w.scan_blocks, dest);
-    }
-    DYN_LAUNCHED("k_scan_dest");
     return DYN_OK;
-}
-
-int scan(dyn_world* world, const uint32_t* flags, const uint32_t* count, uint32_t limit, uint32_t* dest,
-         uint32_t* total, bool counts = false) {
-    return scan(world->w, world->stream, flags, count, limit, dest, total, counts);
 }
 
 // Every candidate pair on the worklist, grouped by kind class: block histograms, their per-class
@@ -3326,8 +3347,7 @@ int solver_prepare(const dyn::W& w, hipStream_t st) {
     const uint32_t cb = blocks_for(w.contact_cap);
     LAUNCH_ON(st, k_solver_reset, count_blocks(w.n), w);
     LAUNCH_ON(st, k_blocks, cb, w);
-    LAUNCH_ON(st, k_rows_count, count_blocks(w.n), w);
-    DYN_TRY(scan(w, st, w.list_counts, nullptr, w.n, w.row_start, &w.scan_total[3], true));
+    LAUNCH_ON(st, k_rows_count, count_blocks(ceil_div(w.n, kRowItems)), w);
     LAUNCH_ON(st, k_fill_lists, cb, w);
     return DYN_OK;
 }
@@ -3400,27 +3420,29 @@ int solver_substeps(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint
     // the GPU's memory pipes busy otherwise; eight were slower), two above (one was slower)
     const uint32_t lanes_log2 = w.n <= (1u << 18) ? 2u : 1u;
     for (uint32_t sub = 0; sub < w.p.substeps; ++sub) {
-        LAUNCH_TH(st, k_integrate, w.d, threads, w);
-        LAUNCH_TH(st, k_solver_bodies, w.n, threads, w);
+        LAUNCH_TH(st, k_integrate, w.n, threads, w);
         LAUNCH_TH(st, k_solve_prep, w.contact_cap, threads, w, sub == 0 ? 1u : 0u);
-        // the substep's last apply writes the velocities back to the body states
+        // the substep's last apply writes the velocities back to the body states and advances the
+        // rows (which k_group_position does where it runs)
+        const uint32_t advance = plan.count ? 0u : 1u;
         if (sub == 0) {
-            LAUNCH_TH(st, k_warm, w.contact_cap, threads, w);
-            LAUNCH_TH(st, k_apply, w.n << lanes_log2, threads, w, w.p.solve_iterations == 0u ? 1u : 0u, lanes_log2);
+            const uint32_t last = w.p.solve_iterations == 0u ? 1u : 0u;
+            LAUNCH_TH(st, k_apply, w.n << lanes_log2, threads, w, last, last & advance, lanes_log2);
+        } else if (w.p.solve_iterations == 0u && advance) {
+            LAUNCH_TH(st, k_advance, w.d, threads, w);
         }
         for (uint32_t it = 0; it < w.p.solve_iterations; ++it) {
             // solver_block_solve.wgsl:85-87: the residual round is the one where the round
             // counter (reset by integrate, bumped by every apply) equals the iteration count,
             // which only the warm-started first substep reaches.
-            LAUNCH_TH(st, k_solve, w.contact_cap, threads, w, (sub == 0 && it + 1u == w.p.solve_iterations) ? 1u : 0u);
-            LAUNCH_TH(st, k_apply, w.n << lanes_log2, threads, w, it + 1u == w.p.solve_iterations ? 1u : 0u,
-                      lanes_log2);
+            const uint32_t last = it + 1u == w.p.solve_iterations ? 1u : 0u;
+            LAUNCH_TH(st, k_solve, w.contact_cap, threads, w, sub == 0 ? last : 0u);
+            LAUNCH_TH(st, k_apply, w.n << lanes_log2, threads, w, last, last & advance, lanes_log2);
         }
         if (plan.count) {
             DYN_TRY(group_position(w, st, plan, sub == 0u ? 1u : 0u, sub + 1u == w.p.substeps ? 1u : 0u));
             continue;
         }
-        LAUNCH_TH(st, k_advance, w.d, threads, w);
         for (uint32_t it = 0; it < w.p.position_iterations; ++it) {
             LAUNCH_TH(st, k_position_block, w.contact_cap, threads, w);
             LAUNCH_TH(st, k_position_apply, w.n << lanes_log2, threads, w, it == 0u ? 1u : 0u,
@@ -3560,7 +3582,7 @@ int world_step(dyn_world* world, float dt) {
     W& w = world->w;
     w.p.dt = dt;
     w.p.substep_dt = dt / static_cast<float>(w.p.substeps);
-    const uint32_t nb = blocks_for(w.n), db = blocks_for(w.d), kb = blocks_for(w.k);
+    const uint32_t nb = blocks_for(w.n), kb = blocks_for(w.k);
     const uint32_t pb = blocks_for(w.pair_cap), cb = blocks_for(w.contact_cap);
     hipStream_t st = world->stream;
     {
@@ -3591,19 +3613,14 @@ int world_step(dyn_world* world, float dt) {
     DYN_TRY(dyn_broadphase(st, &io));
     DYN_TRY(narrowphase(w, st, world->convex_colliders, &world->side));
     const uint32_t* pair_count = w.counters + DYN_COUNTER_PAIRS * DYN_COUNTER_STRIDE_WORDS;
-    DYN_TRY(scan(world, w.valid, pair_count, w.pair_cap, w.dest, &w.scan_total[0]));
-    LAUNCH(k_contacts_scatter, pb, w);
-    {
-        ProfileScope scope("k_contacts_total", st);
-        k_contacts_total<<<1, 64, 0, st>>>(w);
-    }
-    DYN_LAUNCHED("k_contacts_total");
+    const ScanSums found{w.scan_blocks, ceil_div(w.pair_cap ? w.pair_cap : 1u, kScanBlock), &w.scan_total[0]};
+    LAUNCH(k_scan_count, found.groups, w.valid, pair_count, w.pair_cap, found.sums);
+    DYN_TRY(scan_sums(st, found));
+    LAUNCH(k_contacts_scatter, pb, w, found);
     if (world->tape_states) LAUNCH(k_tape_sources, blocks_for(4u * w.contact_cap), w);
     LAUNCH(k_relay, cb, w);
     LAUNCH(k_contact_begin, cb, w, w.p.slop);
-    LAUNCH(k_island_init, db, w);
     DYN_TRY(island_components(w, st, w.p.slop));
-    LAUNCH(k_island_link_resting, cb, w);
     DYN_TRY(island_flatten(w, st, kFlattenPasses - 1u));
     LAUNCH(k_island_aggregate, count_blocks(w.d), w);
     LAUNCH(k_island_wake, count_blocks(w.d), w);
@@ -3613,22 +3630,17 @@ int world_step(dyn_world* world, float dt) {
     }
     DYN_TRY(solver(w, st, world->groups, world->solver_threads));
     LAUNCH(k_sleep, count_blocks(w.d), w);
-    LAUNCH(k_thaw, cb, w);
-    LAUNCH(k_archive, cb, w, world->freeze_flags);
-    DYN_TRY(scan(world, w.rest_flags, w.nresting, w.contact_cap, world->keep_dest, &w.scan_total[2]));
-    DYN_TRY(scan(world, world->freeze_flags, w.ncontacts, w.contact_cap, world->freeze_dest, &w.scan_total[1]));
-    LAUNCH(k_archive_count, nb, w);
-    LAUNCH(k_rest_gather, cb, w, world->keep_dest, &w.scan_total[2], world->freeze_dest, &world->words[0]);
+    const uint32_t rest_groups = ceil_div(w.contact_cap ? w.contact_cap : 1u, kScanBlock);
+    const ScanSums kept{world->rest_blocks, rest_groups, &w.scan_total[1]};
+    const ScanSums frozen{world->rest_blocks + rest_groups, rest_groups, &w.scan_total[2]};
+    LAUNCH(k_archive, rest_groups, w, world->freeze_flags, kept, frozen);
+    DYN_TRY(scan_sums(st, kept, &frozen));
+    LAUNCH(k_rest_gather, cb, w, world->freeze_flags, kept, frozen, &world->words[0]);
     // Sort the new resting list by (min id, max id); payload = its slot.
     const uint32_t words = dyn_sort_key_words(w.id_cap ? w.id_cap : 1u);
     DYN_TRY(dyn_sort_pairs(st, w.rest_major, w.rest_minor, w.rest_slot, w.contact_cap, &world->words[0],
                            nullptr, 1u, words, words, world->sort_scratch, world->sort_scratch_bytes));
     LAUNCH(k_rest_place, cb, w, &world->words[0]);
-    {
-        ProfileScope scope("k_consume", st);
-        k_consume<<<1, 64, 0, st>>>(w);
-    }
-    DYN_LAUNCHED("k_consume");
     swap_contact_buffers(world);
     return DYN_OK;
 }
@@ -3742,6 +3754,7 @@ int dyn_world_create(dyn_world** out, void* stream, const dyn_step_params* param
     A(w.row_start, body_count);
     A(w.contrib, body_count);
     A(w.scan_total, 4);
+    A(w.list_cursor, 1);
     A(w.work_total, kTotalWords);
     A(world->snap_header, 4);
     A(world->words, 8);
@@ -4292,9 +4305,7 @@ SolveLayout solve_layout(uint32_t bodies, uint32_t contact_capacity, void* base)
     w.vwords = reinterpret_cast<uint32_t*>(take(4u * 12u * c));
     w.pwords = reinterpret_cast<uint4*>(take(sizeof(uint4) * 2u * c));
     w.contrib = reinterpret_cast<uint32_t*>(take(4u * n));
-    const size_t limit = n > c ? n : c;
-    w.scan_blocks = reinterpret_cast<uint32_t*>(take(4u * (ceil_div(static_cast<uint32_t>(limit), kScanBlock) + 1u)));
-    w.scan_total = reinterpret_cast<uint32_t*>(take(4u * 4u));
+    w.list_cursor = reinterpret_cast<uint32_t*>(take(4u));
     w.ncontacts = reinterpret_cast<uint32_t*>(take(4u * 2u));  // the clamped count, the check word
     l.bytes = at;
     return l;
@@ -4377,7 +4388,7 @@ int dyn_islands(void* stream, const dyn_islands_io* io) {
     w.motion = reinterpret_cast<uint32_t*>(base + part);
     w.istate = reinterpret_cast<uint32_t*>(base + 2u * part);
     w.flat_flags = reinterpret_cast<uint32_t*>(base + 3u * part);
-    const uint32_t nb = blocks_for(w.n), db = blocks_for(w.d), cb = blocks_for(w.contact_cap);
+    const uint32_t nb = blocks_for(w.n), db = blocks_for(w.d);
     LAUNCH_ON(st, k_islands_stage_reset, nb, w);
     if (w.d == 0u) return DYN_OK;
     LAUNCH_ON(st, k_island_init, db, w);
