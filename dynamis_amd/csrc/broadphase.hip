@@ -216,6 +216,94 @@ __global__ void __launch_bounds__(1024) bp_scan_kernel(const uint32_t* __restric
     if (threadIdx.x >= 2 && threadIdx.x < kCtlWords) sort_ctl[threadIdx.x] = 0;
 }
 
+// The passes above (reset, resolution, fold, count, scan) in one workgroup, for up to kFrontColliders
+// colliders: four launches saved, and each of them was a few hundred colliders' work.
+constexpr uint32_t kFrontThreads = 1024;
+constexpr uint32_t kFrontColliders = 4u * kFrontThreads;
+
+__global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb* __restrict__ aabbs,
+                                                                 const dyn_aabb* __restrict__ resolution,
+                                                                 const uint32_t* __restrict__ flags, uint32_t n,
+                                                                 uint32_t* counters, uint32_t* level_keys,
+                                                                 uint32_t* cnt_level, uint32_t* block_offsets,
+                                                                 uint32_t* sort_hist, uint32_t* sort_ctl,
+                                                                 uint32_t entry_capacity) {
+    constexpr uint32_t kWaves = kFrontThreads / kWave;
+    constexpr uint32_t kBlocks = kFrontColliders / kBpThreads;
+    __shared__ uint32_t s_stats[5];          // scale, extent, levels, faults, coarse
+    __shared__ uint32_t s_blocks[kBlocks];   // entries of each emission workgroup's colliders
+    const uint32_t t = threadIdx.x;
+    if (t < 5u) s_stats[t] = 0u;
+    if (t < kBlocks) s_blocks[t] = 0u;
+    if (t < kGridLevels) level_keys[t] = 0u;
+    for (uint32_t k = t; k < kSortMaxPasses * kSortBins; k += kFrontThreads) sort_hist[k] = 0u;
+    __syncthreads();
+    uint32_t scale = 0, extent = 0;
+    for (uint32_t i = t; i < n; i += kFrontThreads) {
+        const float4 lo = reinterpret_cast<const float4*>(resolution)[2 * i];
+        const float4 hi = reinterpret_cast<const float4*>(resolution)[2 * i + 1];
+        const float3 mn = make_float3(lo.x, lo.y, lo.z), mx = make_float3(hi.x, hi.y, hi.z);
+        scale = max(scale, __float_as_uint(grid_scale_of(mn, mx)));
+        extent = max(extent, __float_as_uint(fmaxf(grid_extent_of(mn, mx), 0.0f)));
+    }
+    scale = wave_max(scale);
+    extent = wave_max(extent);
+    if (lane_id() == 0) {
+        atomicMax(&s_stats[0], scale);
+        atomicMax(&s_stats[1], extent);
+    }
+    __syncthreads();
+    const float base = grid_cell_size(s_stats[0], s_stats[1]);
+    uint32_t levels = 0, faults = 0, coarse = 0;
+    for (uint32_t first = 0; first < n; first += kFrontThreads) {
+        const uint32_t i = first + t;
+        uint32_t emitted = 0;
+        if (i < n) {
+            const float4 lo = reinterpret_cast<const float4*>(aabbs)[2 * i];
+            const float4 hi = reinterpret_cast<const float4*>(aabbs)[2 * i + 1];
+            const float3 mn = make_float3(lo.x, lo.y, lo.z), mx = make_float3(hi.x, hi.y, hi.z);
+            const uint32_t f = flags ? flags[i] : (DYN_BP_MOBILE | DYN_BP_AWAKE);
+            const uint32_t level = shape_levels(mn, mx, base);
+            const uint32_t count = cell_count(grid_cells(mn, mx, level_cell_size(level, base)));
+            emitted = min(count, DYN_MAX_CELLS_PER_COLLIDER);
+            faults += count - emitted;
+            levels |= 1u << level;
+            coarse += (level > 0u && (f & DYN_BP_AWAKE)) ? 1u : 0u;
+            cnt_level[i] = emitted | (level << 8);
+        }
+        emitted = wave_sum(emitted);
+        if (lane_id() == 0 && emitted) atomicAdd(&s_blocks[(first + t) / kBpThreads], emitted);
+    }
+    levels = wave_or(levels);
+    faults = wave_sum(faults);
+    coarse = wave_sum(coarse);
+    if (lane_id() == 0) {
+        atomicOr(&s_stats[2], levels);
+        atomicAdd(&s_stats[3], faults);
+        atomicAdd(&s_stats[4], coarse);
+    }
+    __syncthreads();
+    if (t < kWave) {
+        static_assert(kBlocks <= kWave && kWaves >= 1u, "one wave scans the blocks");
+        const uint32_t v = t < kBlocks ? s_blocks[t] : 0u;
+        const uint32_t inclusive = wave_inclusive_sum(v);
+        if (t * kBpThreads < n) block_offsets[t] = inclusive - v;
+        if (t == kWave - 1u) {
+            *ctr(counters, DYN_COUNTER_ENTRIES) = inclusive;
+            *ctr(counters, DYN_COUNTER_PAIRS) = 0u;
+            *ctr(counters, DYN_COUNTER_REFUSED_PAIRS) = 0u;
+            *ctr(counters, DYN_COUNTER_GRID_SCALE) = s_stats[0];
+            *ctr(counters, DYN_COUNTER_GRID_EXTENT) = s_stats[1];
+            *ctr(counters, DYN_COUNTER_GRID_LEVELS) = s_stats[2];
+            *ctr(counters, DYN_COUNTER_ENTRY_FAULTS) = s_stats[3];
+            *ctr(counters, DYN_COUNTER_COARSE_ACTIVE) = s_stats[4];
+            sort_ctl[kCtlLen] = min(inclusive, entry_capacity);
+            sort_ctl[kCtlBase] = 0u;
+        }
+        if (t >= 2u && t < kCtlWords) sort_ctl[t] = 0u;
+    }
+}
+
 // Workgroups up to which the emission also counts the sort's digits, saving a launch and a read of the
 // keys. Every workgroup adds its counts to the same 1,024 words, one atomic after another: at 2^20
 // boxes that made the emission 111 us, against 43 us and a 12 us pass over the keys without it.
@@ -312,15 +400,14 @@ __device__ __forceinline__ bool gather_pays(const uint32_t* __restrict__ dir, ui
 }
 
 // Distinct keys of every level, one count per run start.
-__global__ void __launch_bounds__(kBpThreads) bp_level_keys_kernel(const uint32_t* __restrict__ keys,
-                                                                   const uint32_t* sort_ctl,
-                                                                   uint32_t* level_keys) {
+__device__ __forceinline__ void count_level_keys(const uint32_t* __restrict__ keys, const uint32_t* sort_ctl,
+                                                 uint32_t* level_keys, uint32_t block, uint32_t blocks) {
     __shared__ uint32_t s_levels[kGridLevels];
     if (threadIdx.x < kGridLevels) s_levels[threadIdx.x] = 0u;
     __syncthreads();
     const uint32_t len = sort_ctl[kCtlLen];
     // A few blocks stride over the keys, so few adds reach each level's global word.
-    for (uint32_t first = blockIdx.x * kBpThreads; first < len; first += gridDim.x * kBpThreads) {
+    for (uint32_t first = block * kBpThreads; first < len; first += blocks * kBpThreads) {
         const uint32_t e = first + threadIdx.x;
         const bool start = e < len && (e == 0u || keys[e - 1] != keys[e]);
         const uint32_t level = start ? keys[e] >> DYN_LEVEL_KEY_SHIFT : 0u;
@@ -363,9 +450,15 @@ __global__ void __launch_bounds__(kBpThreads) bp_gather_kernel(const uint32_t* _
 
 // First sorted index of each 2^16-bucket of every occupied level (lower bound of the bucket's
 // smallest key); bucket kDirBuckets of a level holds the level's end.
-__global__ void __launch_bounds__(256) bp_directory_kernel(const uint32_t* __restrict__ keys,
-                                                          const uint32_t* counters,
-                                                          const uint32_t* sort_ctl, uint32_t* dir) {
+// The workgroups past the directory's count the levels' distinct keys beside it.
+constexpr uint32_t kDirBlocks = (kGridLevels * kDirStride + kBpThreads - 1u) / kBpThreads;
+__global__ void __launch_bounds__(kBpThreads) bp_directory_kernel(const uint32_t* __restrict__ keys,
+                                                                  const uint32_t* counters, const uint32_t* sort_ctl,
+                                                                  uint32_t* dir, uint32_t* level_keys) {
+    if (blockIdx.x >= kDirBlocks) {
+        count_level_keys(keys, sort_ctl, level_keys, blockIdx.x - kDirBlocks, gridDim.x - kDirBlocks);
+        return;
+    }
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= kGridLevels * kDirStride) return;
     const uint32_t level = g / kDirStride;
@@ -580,38 +673,36 @@ __device__ __forceinline__ void cell_mates(uint32_t index, uint32_t len,
     }
 }
 
-// Cell mates, counting pass: one thread per sorted entry.
-__global__ void __launch_bounds__(kBpThreads) bp_mates_count_kernel(
-    const uint32_t* __restrict__ keys, EntryRecords rec, const uint32_t* __restrict__ dir, const uint32_t* counters,
-    const uint32_t* sort_ctl, const uint32_t* __restrict__ worlds, uint32_t* mate_counts,
-    uint32_t* mate_blocks) {
-    __shared__ uint32_t s_scan[kBpThreads / kWave];
+// Cell mates, counting pass: one thread per sorted entry of block `block`.
+__device__ __forceinline__ void count_mates(
+    uint32_t block, const uint32_t* __restrict__ keys, EntryRecords rec, const uint32_t* __restrict__ dir,
+    const uint32_t* counters, const uint32_t* sort_ctl, const uint32_t* __restrict__ worlds, uint32_t* mate_counts,
+    uint32_t* mate_blocks, uint32_t* s_scan) {
     const uint32_t len = sort_ctl[kCtlLen];
     const float grid = grid_cell_size(counters[DYN_COUNTER_GRID_SCALE * DYN_COUNTER_STRIDE_WORDS],
                                       counters[DYN_COUNTER_GRID_EXTENT * DYN_COUNTER_STRIDE_WORDS]);
-    const uint32_t index = blockIdx.x * kBpThreads + threadIdx.x;
+    const uint32_t index = block * kBpThreads + threadIdx.x;
     PairCounter counter;
     rec.gathered = gather_pays(dir, counters[DYN_COUNTER_GRID_LEVELS * DYN_COUNTER_STRIDE_WORDS], rec.level_keys);
     if (index < len) cell_mates(index, len, keys, rec, grid, worlds, counter);
     if (index < len) mate_counts[index] = counter.n;
     uint32_t total = 0;
     block_exclusive_sum<kBpThreads>(counter.n, s_scan, &total);
-    if (threadIdx.x == 0) mate_blocks[blockIdx.x] = total;
+    if (threadIdx.x == 0) mate_blocks[block] = total;
 }
 
 // Cell mates, emitting pass: the same walk, pairs written at their scanned offsets.
-__global__ void __launch_bounds__(kBpThreads) bp_mates_emit_kernel(
-    const uint32_t* __restrict__ keys, EntryRecords rec, const uint32_t* __restrict__ dir, const uint32_t* counters,
-    const uint32_t* sort_ctl, const uint32_t* __restrict__ worlds,
-    const uint32_t* __restrict__ mate_counts, const uint32_t* __restrict__ mate_offsets,
-    uint32_t* pair_major, uint32_t* pair_minor, uint32_t pair_capacity) {
-    __shared__ uint32_t s_scan[kBpThreads / kWave];
+__device__ __forceinline__ void emit_mates(
+    uint32_t block, const uint32_t* __restrict__ keys, EntryRecords rec, const uint32_t* __restrict__ dir,
+    const uint32_t* counters, const uint32_t* sort_ctl, const uint32_t* __restrict__ worlds,
+    const uint32_t* __restrict__ mate_counts, const uint32_t* __restrict__ mate_offsets, uint32_t* pair_major,
+    uint32_t* pair_minor, uint32_t pair_capacity, uint32_t* s_scan) {
     const uint32_t len = sort_ctl[kCtlLen];
     const float grid = grid_cell_size(counters[DYN_COUNTER_GRID_SCALE * DYN_COUNTER_STRIDE_WORDS],
                                       counters[DYN_COUNTER_GRID_EXTENT * DYN_COUNTER_STRIDE_WORDS]);
-    const uint32_t index = blockIdx.x * kBpThreads + threadIdx.x;
+    const uint32_t index = block * kBpThreads + threadIdx.x;
     const uint32_t mine = index < len ? mate_counts[index] : 0u;
-    const uint32_t at = mate_offsets[blockIdx.x] + block_exclusive_sum<kBpThreads>(mine, s_scan, nullptr);
+    const uint32_t at = mate_offsets[block] + block_exclusive_sum<kBpThreads>(mine, s_scan, nullptr);
     if (mine == 0u || at >= pair_capacity) return;
     PairWriter writer{at, pair_capacity, pair_major, pair_minor};
     rec.gathered = gather_pays(dir, counters[DYN_COUNTER_GRID_LEVELS * DYN_COUNTER_STRIDE_WORDS], rec.level_keys);
@@ -720,8 +811,8 @@ __device__ __forceinline__ void level_links(uint32_t i, uint32_t packed, uint32_
 // finer collider probing that level reads, or where the colliders are too few to fill the GPU one
 // lane each; otherwise the lanes would mostly wait, and one lane walks a collider's probes.
 // bp_gather_kernel writes the choice and the gather decision to one word (kLinkModeLanes,
-// kLinkModeGathered), which both link passes and the offsets read. Each pass is launched in both
-// shapes, a workgroup per chunk; the workgroups of the shape not chosen read the word and return.
+// kLinkModeGathered), which both link passes and the offsets read. A pass has a workgroup per chunk for
+// each shape that the mode may choose; the workgroups of the shape not chosen read the word and return.
 
 template <uint32_t kLanes>
 __device__ __forceinline__ uint32_t link_chunk_colliders() { return kBpThreads / kLanes; }
@@ -761,81 +852,101 @@ __device__ __forceinline__ LinkArgs link_args(const dyn_aabb* aabbs, const uint3
                     capacity, worlds};
 }
 
+// Both pair walks of a pass in one launch: the level links in the shapes the mode may choose (shape 1
+// one lane a collider, shape 8 eight), then the cell mates; each workgroup knows its part from its
+// index. Both are bound by the latency of their dependent reads, and run beside each other so.
+struct PairArgs {
+    const dyn_aabb* aabbs;
+    const uint32_t *groups, *flags;
+    uint32_t n;
+    const uint32_t *cnt_level, *first_slot, *keys;
+    EntryRecords rec;
+    const uint32_t *dir, *counters;
+    uint32_t entry_capacity;
+    const uint32_t *worlds, *link_mode, *sort_ctl;
+    uint32_t *link_counts, *link_blocks;
+    uint2* link_stage;
+    uint32_t *mate_counts, *mate_blocks;
+    uint32_t *pair_major, *pair_minor, pair_capacity;
+    uint32_t thread_groups, lane_groups;  // workgroups of the two shapes
+};
+
 // Level links, counting pass: chunks of kBpThreads / kLanes consecutive colliders, a chunk per
 // workgroup, kLanes lanes per collider; link_blocks holds each chunk's pair total.
 template <uint32_t kLanes>
+__device__ __forceinline__ void count_links(uint32_t chunk, const PairArgs& p, uint32_t* s_scan) {
+    const uint32_t mode = *p.link_mode;
+    if (((mode & kLinkModeLanes) != 0u) != (kLanes > 1u)) return;
+    const LinkArgs a = link_args(p.aabbs, p.groups, p.flags, p.n, p.cnt_level, p.first_slot, p.keys, p.rec, p.dir,
+                                 p.counters, p.entry_capacity, p.worlds, mode);
+    const uint32_t i = chunk * link_chunk_colliders<kLanes>() + threadIdx.x / kLanes;
+    const bool leader = threadIdx.x % kLanes == 0u && i < p.n;
+    GroupStage<kLanes> counter{0u, p.link_stage + static_cast<size_t>(i < p.n ? i : 0u) * kLinkStage};
+    if (i < p.n) {
+        level_links<kLanes>(i, p.cnt_level[i], p.first_slot[i], a.aabbs, a.groups, a.flags, a.keys, a.rec, a.dir,
+                            a.coarse_active, a.occupied, a.grid, a.capacity, a.worlds, counter);
+        if (leader) p.link_counts[i] = counter.n;
+    }
+    uint32_t total = 0;
+    block_exclusive_sum<kBpThreads>(leader ? counter.n : 0u, s_scan, &total);
+    if (threadIdx.x == 0) p.link_blocks[chunk] = total;
+}
+
 // Eight waves a SIMD (64 registers, a few spilled): the walks are latency-bound (the batch's
 // count 1.63 -> 1.42 ms; the emit pass, which writes, was slower so).
-__global__ void __launch_bounds__(kBpThreads, 8) bp_links_count_kernel(
-    const dyn_aabb* __restrict__ aabbs, const uint32_t* __restrict__ groups,
-    const uint32_t* __restrict__ flags, uint32_t n, const uint32_t* __restrict__ cnt_level,
-    const uint32_t* __restrict__ first_slot, const uint32_t* __restrict__ keys,
-    EntryRecords rec,
-    const uint32_t* __restrict__ dir, const uint32_t* counters, uint32_t capacity,
-    const uint32_t* __restrict__ worlds, const uint32_t* link_mode, uint32_t* link_counts,
-    uint32_t* link_blocks, uint2* link_stage) {
+__global__ void __launch_bounds__(kBpThreads, 8) bp_pairs_count_kernel(PairArgs p) {
     __shared__ uint32_t s_scan[kBpThreads / kWave];
-    const uint32_t mode = *link_mode;
-    if (((mode & kLinkModeLanes) != 0u) != (kLanes > 1u)) return;
-    const LinkArgs a = link_args(aabbs, groups, flags, n, cnt_level, first_slot, keys, rec, dir, counters,
-                                 capacity, worlds, mode);
-    const uint32_t chunks = link_chunks(n, kLanes);
-    for (uint32_t chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
-        const uint32_t i = chunk * link_chunk_colliders<kLanes>() + threadIdx.x / kLanes;
-        const bool leader = threadIdx.x % kLanes == 0u && i < n;
-        GroupStage<kLanes> counter{0u, link_stage + static_cast<size_t>(i < n ? i : 0u) * kLinkStage};
-        if (i < n) {
-            level_links<kLanes>(i, cnt_level[i], first_slot[i], a.aabbs, a.groups, a.flags, a.keys, a.rec, a.dir,
-                                a.coarse_active, a.occupied, a.grid, a.capacity, a.worlds, counter);
-            if (leader) link_counts[i] = counter.n;
-        }
-        uint32_t total = 0;
-        block_exclusive_sum<kBpThreads>(leader ? counter.n : 0u, s_scan, &total);
-        if (threadIdx.x == 0) link_blocks[chunk] = total;
+    const uint32_t b = blockIdx.x;
+    if (b < p.thread_groups) {
+        count_links<1>(b, p, s_scan);
+    } else if (b < p.thread_groups + p.lane_groups) {
+        count_links<kLinkLanes>(b - p.thread_groups, p, s_scan);
+    } else {
+        count_mates(b - p.thread_groups - p.lane_groups, p.keys, p.rec, p.dir, p.counters, p.sort_ctl, p.worlds,
+                    p.mate_counts, p.mate_blocks, s_scan);
     }
 }
 
 // Level links, emitting pass: the counting pass's chunks and lanes.
 template <uint32_t kLanes>
-__global__ void __launch_bounds__(kBpThreads) bp_links_emit_kernel(
-    const dyn_aabb* __restrict__ aabbs, const uint32_t* __restrict__ groups,
-    const uint32_t* __restrict__ flags, uint32_t n, const uint32_t* __restrict__ cnt_level,
-    const uint32_t* __restrict__ first_slot, const uint32_t* __restrict__ keys,
-    EntryRecords rec,
-    const uint32_t* __restrict__ dir, const uint32_t* counters, uint32_t capacity,
-    const uint32_t* __restrict__ worlds, const uint32_t* link_mode, const uint32_t* __restrict__ link_counts,
-    const uint32_t* __restrict__ link_offsets, const uint2* __restrict__ link_stage,
-    uint32_t* pair_major, uint32_t* pair_minor, uint32_t pair_capacity) {
-    __shared__ uint32_t s_scan[kBpThreads / kWave];
-    __shared__ uint32_t s_at[kBpThreads / kLanes];
-    const uint32_t mode = *link_mode;
+__device__ __forceinline__ void emit_links(uint32_t chunk, const PairArgs& p, uint32_t* s_scan, uint32_t* s_at) {
+    const uint32_t mode = *p.link_mode;
     if (((mode & kLinkModeLanes) != 0u) != (kLanes > 1u)) return;
-    const LinkArgs a = link_args(aabbs, groups, flags, n, cnt_level, first_slot, keys, rec, dir, counters,
-                                 capacity, worlds, mode);
-    const uint32_t chunks = link_chunks(n, kLanes);
+    const LinkArgs a = link_args(p.aabbs, p.groups, p.flags, p.n, p.cnt_level, p.first_slot, p.keys, p.rec, p.dir,
+                                 p.counters, p.entry_capacity, p.worlds, mode);
     const uint32_t g = threadIdx.x / kLanes, q = threadIdx.x % kLanes;
-    for (uint32_t chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
-        const uint32_t i = chunk * link_chunk_colliders<kLanes>() + g;
-        const uint32_t mine = i < n ? link_counts[i] : 0u;
-        const uint32_t excl = block_exclusive_sum<kBpThreads>(q == 0u ? mine : 0u, s_scan, nullptr);
-        if (q == 0u) s_at[g] = link_offsets[chunk] + excl;
-        __syncthreads();
-        const uint32_t at = s_at[g];
-        if (mine != 0u && at < pair_capacity) {
-            if (mine <= kLinkStage) {  // the counting pass kept them all
-                const uint2* kept = link_stage + static_cast<size_t>(i) * kLinkStage;
-                for (uint32_t j = q; j < mine && at + j < pair_capacity; j += kLanes) {
-                    const uint2 p = kept[j];
-                    pair_major[at + j] = p.x;
-                    pair_minor[at + j] = p.y;
-                }
-            } else {
-                GroupWriter<kLanes> writer{at, pair_capacity, pair_major, pair_minor};
-                level_links<kLanes>(i, cnt_level[i], first_slot[i], a.aabbs, a.groups, a.flags, a.keys, a.rec,
-                                    a.dir, a.coarse_active, a.occupied, a.grid, a.capacity, a.worlds, writer);
-            }
+    const uint32_t i = chunk * link_chunk_colliders<kLanes>() + g;
+    const uint32_t mine = i < p.n ? p.link_counts[i] : 0u;
+    const uint32_t excl = block_exclusive_sum<kBpThreads>(q == 0u ? mine : 0u, s_scan, nullptr);
+    if (q == 0u) s_at[g] = p.link_blocks[chunk] + excl;
+    __syncthreads();
+    const uint32_t at = s_at[g];
+    if (mine == 0u || at >= p.pair_capacity) return;
+    if (mine <= kLinkStage) {  // the counting pass kept them all
+        const uint2* kept = p.link_stage + static_cast<size_t>(i) * kLinkStage;
+        for (uint32_t j = q; j < mine && at + j < p.pair_capacity; j += kLanes) {
+            const uint2 pair = kept[j];
+            p.pair_major[at + j] = pair.x;
+            p.pair_minor[at + j] = pair.y;
         }
-        __syncthreads();  // s_at is reused by the next chunk
+    } else {
+        GroupWriter<kLanes> writer{at, p.pair_capacity, p.pair_major, p.pair_minor};
+        level_links<kLanes>(i, p.cnt_level[i], p.first_slot[i], a.aabbs, a.groups, a.flags, a.keys, a.rec, a.dir,
+                            a.coarse_active, a.occupied, a.grid, a.capacity, a.worlds, writer);
+    }
+}
+
+__global__ void __launch_bounds__(kBpThreads) bp_pairs_emit_kernel(PairArgs p) {
+    __shared__ uint32_t s_scan[kBpThreads / kWave];
+    __shared__ uint32_t s_at[kBpThreads];
+    const uint32_t b = blockIdx.x;
+    if (b < p.thread_groups) {
+        emit_links<1>(b, p, s_scan, s_at);
+    } else if (b < p.thread_groups + p.lane_groups) {
+        emit_links<kLinkLanes>(b - p.thread_groups, p, s_scan, s_at);
+    } else {
+        emit_mates(b - p.thread_groups - p.lane_groups, p.keys, p.rec, p.dir, p.counters, p.sort_ctl, p.worlds,
+                   p.mate_counts, p.mate_blocks, p.pair_major, p.pair_minor, p.pair_capacity, s_scan);
     }
 }
 
@@ -968,42 +1079,52 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint32_t* counters = io->d_counters;
-    {
-        ProfileScope scope("bp_reset_kernel", st);
-        bp_reset_kernel<<<1, 64, 0, st>>>(counters, l.level_keys);
-    }
-    DYN_LAUNCHED("bp_reset_kernel");
     const uint32_t blocks = ceil_div(n ? n : 1u, kBpThreads);
-    if (n) {
-        const dyn_aabb* res = io->d_resolution ? io->d_resolution : io->d_aabbs;
+    const dyn_aabb* res = io->d_resolution ? io->d_resolution : io->d_aabbs;
+    if (n && n <= kFrontColliders) {
         {
-            ProfileScope scope("bp_resolution_kernel", st);
-            bp_resolution_kernel<<<min(blocks, kResolutionBlocks), kBpThreads, 0, st>>>(
-                res, n, l.res_partials);
+            ProfileScope scope("bp_front_kernel", st);
+            bp_front_kernel<<<1, kFrontThreads, 0, st>>>(io->d_aabbs, res, io->d_flags, n, counters, l.level_keys,
+                                                         l.cnt_level, l.block_offsets, l.entry_sort.hist,
+                                                         l.entry_sort.ctl, io->entry_capacity);
         }
-        DYN_LAUNCHED("bp_resolution_kernel");
+        DYN_LAUNCHED("bp_front_kernel");
+    } else {
         {
-            ProfileScope scope("bp_resolution_fold_kernel", st);
-            bp_resolution_fold_kernel<<<1, 1024, 0, st>>>(l.res_partials,
-                                                          min(blocks, kResolutionBlocks), counters);
+            ProfileScope scope("bp_reset_kernel", st);
+            bp_reset_kernel<<<1, 64, 0, st>>>(counters, l.level_keys);
         }
-        DYN_LAUNCHED("bp_resolution_fold_kernel");
+        DYN_LAUNCHED("bp_reset_kernel");
+        if (n) {
+            {
+                ProfileScope scope("bp_resolution_kernel", st);
+                bp_resolution_kernel<<<min(blocks, kResolutionBlocks), kBpThreads, 0, st>>>(
+                    res, n, l.res_partials);
+            }
+            DYN_LAUNCHED("bp_resolution_kernel");
+            {
+                ProfileScope scope("bp_resolution_fold_kernel", st);
+                bp_resolution_fold_kernel<<<1, 1024, 0, st>>>(l.res_partials,
+                                                              min(blocks, kResolutionBlocks), counters);
+            }
+            DYN_LAUNCHED("bp_resolution_fold_kernel");
+            {
+                ProfileScope scope("bp_count_kernel", st);
+                bp_count_kernel<<<blocks, kBpThreads, 0, st>>>(io->d_aabbs, io->d_flags, n, counters,
+                                                               l.cnt_level, l.block_totals,
+                                                               l.block_stats);
+            }
+            DYN_LAUNCHED("bp_count_kernel");
+        }
         {
-            ProfileScope scope("bp_count_kernel", st);
-            bp_count_kernel<<<blocks, kBpThreads, 0, st>>>(io->d_aabbs, io->d_flags, n, counters,
-                                                           l.cnt_level, l.block_totals,
-                                                           l.block_stats);
+            ProfileScope scope("bp_scan_kernel", st);
+            bp_scan_kernel<<<1, 1024, 0, st>>>(l.block_totals, l.block_stats, n ? blocks : 0u,
+                                               l.block_offsets,
+                                               counters, l.entry_sort.hist, l.entry_sort.ctl,
+                                               io->entry_capacity);
         }
-        DYN_LAUNCHED("bp_count_kernel");
+        DYN_LAUNCHED("bp_scan_kernel");
     }
-    {
-        ProfileScope scope("bp_scan_kernel", st);
-        bp_scan_kernel<<<1, 1024, 0, st>>>(l.block_totals, l.block_stats, n ? blocks : 0u,
-                                           l.block_offsets,
-                                           counters, l.entry_sort.hist, l.entry_sort.ctl,
-                                           io->entry_capacity);
-    }
-    DYN_LAUNCHED("bp_scan_kernel");
     if (n == 0 || io->entry_capacity == 0) return DYN_OK;
     const bool small_entries = io->entry_capacity <= kSortSmall;
     const bool emit_histogram = !small_entries && blocks <= kEmitHistogramBlocks;
@@ -1033,19 +1154,12 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
                             io->entry_capacity, kEntrySortNames));
     }
     const uint32_t entry_blocks = ceil_div(io->entry_capacity, kBpThreads);
-    const uint32_t dir_threads = kGridLevels * kDirStride;
     {
         ProfileScope scope("bp_directory_kernel", st);
-        bp_directory_kernel<<<ceil_div(dir_threads, 256), 256, 0, st>>>(io->d_entry_keys, counters,
-                                                                        l.entry_sort.ctl, l.dir);
+        bp_directory_kernel<<<kDirBlocks + min(entry_blocks, 1024u), kBpThreads, 0, st>>>(
+            io->d_entry_keys, counters, l.entry_sort.ctl, l.dir, l.level_keys);
     }
     DYN_LAUNCHED("bp_directory_kernel");
-    {
-        ProfileScope scope("bp_level_keys_kernel", st);
-        bp_level_keys_kernel<<<min(entry_blocks, 1024u), kBpThreads, 0, st>>>(io->d_entry_keys, l.entry_sort.ctl,
-                                                                  l.level_keys);
-    }
-    DYN_LAUNCHED("bp_level_keys_kernel");
     {
         ProfileScope scope("bp_gather_kernel", st);
         bp_gather_kernel<<<min(entry_blocks, 2048u), kBpThreads, 0, st>>>(io->d_entry_order, io->d_entries,
@@ -1054,27 +1168,18 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
     }
     DYN_LAUNCHED("bp_gather_kernel");
     const EntryRecords rec{l.sorted, io->d_entries, io->d_entry_order, l.level_keys, false};
-    const uint32_t thread_groups = link_chunks(n, 1u);
-    const uint32_t lane_groups = link_chunks(n, kLinkLanes);
+    // up to kLinkLanesBelow colliders the mode is eight lanes whatever the grid holds
+    const PairArgs pairs{io->d_aabbs, io->d_groups, io->d_flags, n, l.cnt_level, l.first_slot, io->d_entry_keys, rec,
+                         l.dir, counters, io->entry_capacity, io->d_worlds, l.link_mode, l.entry_sort.ctl,
+                         l.link_counts, l.link_blocks, l.link_stage, l.mate_counts, l.mate_blocks, io->d_pair_major,
+                         io->d_pair_minor, io->pair_capacity, n <= kLinkLanesBelow ? 0u : link_chunks(n, 1u),
+                         link_chunks(n, kLinkLanes)};
+    const uint32_t pair_groups = pairs.thread_groups + pairs.lane_groups + entry_blocks;
     {
-        ProfileScope scope("bp_links_count_kernel", st);
-        bp_links_count_kernel<1><<<thread_groups, kBpThreads, 0, st>>>(
-            io->d_aabbs, io->d_groups, io->d_flags, n, l.cnt_level, l.first_slot,
-            io->d_entry_keys, rec, l.dir, counters,
-            io->entry_capacity, io->d_worlds, l.link_mode, l.link_counts, l.link_blocks, l.link_stage);
-        bp_links_count_kernel<kLinkLanes><<<lane_groups, kBpThreads, 0, st>>>(
-            io->d_aabbs, io->d_groups, io->d_flags, n, l.cnt_level, l.first_slot,
-            io->d_entry_keys, rec, l.dir, counters,
-            io->entry_capacity, io->d_worlds, l.link_mode, l.link_counts, l.link_blocks, l.link_stage);
+        ProfileScope scope("bp_pairs_count_kernel", st);
+        bp_pairs_count_kernel<<<pair_groups, kBpThreads, 0, st>>>(pairs);
     }
-    DYN_LAUNCHED("bp_links_count_kernel");
-    {
-        ProfileScope scope("bp_mates_count_kernel", st);
-        bp_mates_count_kernel<<<entry_blocks, kBpThreads, 0, st>>>(
-            io->d_entry_keys, rec, l.dir, counters, l.entry_sort.ctl,
-            io->d_worlds, l.mate_counts, l.mate_blocks);
-    }
-    DYN_LAUNCHED("bp_mates_count_kernel");
+    DYN_LAUNCHED("bp_pairs_count_kernel");
     {
         ProfileScope scope("bp_pair_offsets_kernel", st);
         bp_pair_offsets_kernel<<<1, 1024, 0, st>>>(l.link_blocks, n, l.link_mode, l.mate_blocks, entry_blocks,
@@ -1083,38 +1188,21 @@ int dyn_broadphase(void* stream, const dyn_broadphase_io* io) {
     DYN_LAUNCHED("bp_pair_offsets_kernel");
     if (io->pair_capacity) {
         {
-            ProfileScope scope("bp_links_emit_kernel", st);
-            bp_links_emit_kernel<1><<<thread_groups, kBpThreads, 0, st>>>(
-                io->d_aabbs, io->d_groups, io->d_flags, n, l.cnt_level, l.first_slot,
-                io->d_entry_keys, rec, l.dir, counters,
-                io->entry_capacity, io->d_worlds, l.link_mode, l.link_counts, l.link_blocks, l.link_stage,
-                io->d_pair_major, io->d_pair_minor, io->pair_capacity);
-            bp_links_emit_kernel<kLinkLanes><<<lane_groups, kBpThreads, 0, st>>>(
-                io->d_aabbs, io->d_groups, io->d_flags, n, l.cnt_level, l.first_slot,
-                io->d_entry_keys, rec, l.dir, counters,
-                io->entry_capacity, io->d_worlds, l.link_mode, l.link_counts, l.link_blocks, l.link_stage,
-                io->d_pair_major, io->d_pair_minor, io->pair_capacity);
+            ProfileScope scope("bp_pairs_emit_kernel", st);
+            bp_pairs_emit_kernel<<<pair_groups, kBpThreads, 0, st>>>(pairs);
         }
-        DYN_LAUNCHED("bp_links_emit_kernel");
-        {
-            ProfileScope scope("bp_mates_emit_kernel", st);
-            bp_mates_emit_kernel<<<entry_blocks, kBpThreads, 0, st>>>(
-                io->d_entry_keys, rec, l.dir, counters, l.entry_sort.ctl,
-                io->d_worlds, l.mate_counts, l.mate_blocks, io->d_pair_major, io->d_pair_minor,
-                io->pair_capacity);
-        }
-        DYN_LAUNCHED("bp_mates_emit_kernel");
+        DYN_LAUNCHED("bp_pairs_emit_kernel");
     }
     if (io->sort_pairs && io->pair_capacity) {
         const uint32_t words = dyn_sort_key_words(n);
         sort_digits(words, words, digits);
-        const uint32_t* pairs = counters + DYN_COUNTER_PAIRS * DYN_COUNTER_STRIDE_WORDS;
+        const uint32_t* pair_count = counters + DYN_COUNTER_PAIRS * DYN_COUNTER_STRIDE_WORDS;
         // the pairs are their own keys: no payload is moved
         if (io->pair_capacity <= kSortSmall) {
-            return sort_small(st, io->d_pair_major, io->d_pair_minor, nullptr, pairs, nullptr, io->pair_capacity, digits,
+            return sort_small(st, io->d_pair_major, io->d_pair_minor, nullptr, pair_count, nullptr, io->pair_capacity, digits,
                               2u * words, kPairSortNames);
         }
-        DYN_TRY(sort_prepare(st, l.pair_sort, pairs, nullptr, io->pair_capacity, kPairSortNames));
+        DYN_TRY(sort_prepare(st, l.pair_sort, pair_count, nullptr, io->pair_capacity, kPairSortNames));
         DYN_TRY(sort_histogram(st, io->d_pair_major, io->d_pair_minor, l.pair_sort, digits,
                                2u * words, io->pair_capacity, kPairSortNames));
         DYN_TRY(sort_passes(st, io->d_pair_major, io->d_pair_minor, nullptr, l.pair_sort, digits, 2u * words,
