@@ -110,10 +110,22 @@ __device__ __forceinline__ uint32_t cell_offset(const Cells& c, const int32_t co
 }
 
 // grid_index.wgsl:79-89: the finest level at which the box spans at most 2 cells per axis.
+// A level whose cells are far too small is passed over without its six divisions, which a plane's box
+// took some 20 times in a row on one lane of every pass: with every coordinate within 2^22
+// cells a quotient is off by at most 1/4 and none saturates, so a side of more than 8 cells spans at
+// least 7.
 __device__ __forceinline__ uint32_t shape_levels(float3 mn, float3 mx, float base) {
+    const float side = fmaxf(fmaxf(mx.x - mn.x, mx.y - mn.y), mx.z - mn.z);
+    const float reach = fmaxf(fmaxf(fmaxf(fabsf(mn.x), fabsf(mn.y)), fabsf(mn.z)),
+                              fmaxf(fmaxf(fabsf(mx.x), fabsf(mx.y)), fabsf(mx.z)));
     uint32_t level = 0;
     for (;;) {
-        const Cells c = grid_cells(mn, mx, level_cell_size(level, base));
+        const float cell = level_cell_size(level, base);
+        if (level < DYN_GRID_LEVEL_LIMIT && reach <= 4194304.0f * cell && side > 8.0f * cell) {
+            ++level;
+            continue;
+        }
+        const Cells c = grid_cells(mn, mx, cell);
         const uint32_t m = max(max(span_of(c, 0), span_of(c, 1)), span_of(c, 2));
         if (m <= DYN_MAX_CELLS_PER_AXIS || level >= DYN_GRID_LEVEL_LIMIT) break;
         ++level;

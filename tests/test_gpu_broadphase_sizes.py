@@ -57,3 +57,26 @@ def test_short_streams_count_what_they_refuse(device, count):
     cut = few.read()
     assert abi.counter(cut.counters, "ENTRIES") == entries
     assert abi.counter(cut.counters, "ENTRY_FAULTS") == (abi.counter(whole.counters, "ENTRY_FAULTS") + entries - entries // 2)
+
+
+@pytest.mark.parametrize("count", [700, 4500])
+@pytest.mark.parametrize("reach", [40.0, 3.0e4, 5.0e6])
+def test_levels_of_boxes_of_every_side(device, oracle, count, reach):
+    """Sides on both sides of 1 to 16 cells of every level, one long axis or all three, near the origin,
+    and where a coordinate is past 2^22 of the finest cells."""
+    rng = np.random.default_rng(int(reach) + count)
+    boxes = uniform_boxes(count, reach, 0.2, 0.4, 3)
+    centre = rng.uniform(-reach, reach, (count, 3))
+    ratio = rng.choice([1.0, 1.99, 2.0, 2.01, 4.0, 7.99, 8.0, 8.01, 16.0], (count, 1))
+    half = 0.1 * ratio * 2.0 ** rng.integers(0, 14, (count, 1)) * np.where(rng.random((count, 1)) < 0.5, 1.0,
+                                                                          rng.uniform(0.01, 1.0, (count, 3)))
+    few = rng.random((count, 1)) < 0.03  # most boxes stay small: large ones pair with everything
+    half = np.where(few, half, 0.1)
+    boxes["min"][:, :3] = (centre - half).astype(np.float32)
+    boxes["max"][:, :3] = (centre + half).astype(np.float32)
+    bp = Broadphase(count, pair_capacity=256 * count)
+    bp.upload(boxes)
+    bp.run()
+    got, want = bp.read(), oracle.broadphase(boxes, pair_capacity=256 * count)
+    assert np.array_equal(got.entry_keys, want["entry_keys"])
+    assert np.array_equal(got.pairs, want["pairs"]) and len(got.pairs) < 256 * count
