@@ -2336,11 +2336,6 @@ __device__ __forceinline__ void solve_block(const W& w, uint32_t ci, const Bodie
     const v3 normal = mk(h1.x, h1.y, h1.z);
     const float relaxation = h1.w, damping_ratio = h2.x;
     const SolverBody bf = bodies(fb), bs = bodies(sb);
-    float split_f[6], split_s[6];
-    for (int k = 0; k < 6; ++k) {
-        split_f[k] = bf.inertia[k] * bf.count;
-        split_s[k] = bs.inertia[k] * bs.count;
-    }
     const v3 vf = bf.v, wf = bf.w, vs = bs.v, ws = bs.w;
     v3 first_v = vf, first_w = wf, second_v = vs, second_w = ws;
     v3 t1, t2;
@@ -2390,29 +2385,39 @@ __device__ __forceinline__ void solve_block(const W& w, uint32_t ci, const Bodie
         second_v = add(second_v, mul(impulse, bs.inverse_mass));
         second_w = add(second_w, inverse_inertia_at(bs.q, bs.inertia, cross3(rb, impulse)));
     }
+    // Rolling and spin friction. Their limits are zero for bodies without either (the default): the
+    // impulse is then clamped to zero and would add zeros to finite velocities, so it is left out.
+    const float roll = h2.y * normal_total, spin_limit = h2.z * normal_total;
     const v3 rel_spin = sub(second_w, first_w);
-    const v3 planar = sub(rel_spin, mul(normal, dot3(rel_spin, normal)));
-    const float planar_len = len3(planar);
-    if (planar_len > 1e-6f) {
-        const v3 axis = dv(planar, planar_len);
-        const float mass = dot3(axis, inverse_inertia_at(bf.q, split_f, axis)) +
-                           dot3(axis, inverse_inertia_at(bs.q, split_s, axis));
-        if (mass > 0.0f) {
-            const float lim = h2.y * normal_total;
-            const float applied = clampf(-planar_len / mass, -lim, lim);
-            first_w = sub(first_w, inverse_inertia_at(bf.q, bf.inertia, mul(axis, applied)));
-            second_w = add(second_w, inverse_inertia_at(bs.q, bs.inertia, mul(axis, applied)));
-        }
-    }
     const float twist = dot3(rel_spin, normal);
-    if (fabsf(twist) > 1e-6f) {
-        const float mass = dot3(normal, inverse_inertia_at(bf.q, split_f, normal)) +
-                           dot3(normal, inverse_inertia_at(bs.q, split_s, normal));
-        if (mass > 0.0f) {
-            const float lim = h2.z * normal_total;
-            const float applied = clampf(-twist / mass, -lim, lim);
-            first_w = sub(first_w, inverse_inertia_at(bf.q, bf.inertia, mul(normal, applied)));
-            second_w = add(second_w, inverse_inertia_at(bs.q, bs.inertia, mul(normal, applied)));
+    const v3 planar = sub(rel_spin, mul(normal, twist));
+    const float planar_len = len3(planar);
+    const bool rolls = planar_len > 1e-6f && !(roll == 0.0f && planar_len <= kBig);
+    const bool spins = fabsf(twist) > 1e-6f && !(spin_limit == 0.0f && fabsf(twist) <= kBig);
+    if (rolls || spins) {
+        float split_f[6], split_s[6];
+        for (int k = 0; k < 6; ++k) {
+            split_f[k] = bf.inertia[k] * bf.count;
+            split_s[k] = bs.inertia[k] * bs.count;
+        }
+        if (rolls) {
+            const v3 axis = dv(planar, planar_len);
+            const float mass = dot3(axis, inverse_inertia_at(bf.q, split_f, axis)) +
+                               dot3(axis, inverse_inertia_at(bs.q, split_s, axis));
+            if (mass > 0.0f) {
+                const float applied = clampf(-planar_len / mass, -roll, roll);
+                first_w = sub(first_w, inverse_inertia_at(bf.q, bf.inertia, mul(axis, applied)));
+                second_w = add(second_w, inverse_inertia_at(bs.q, bs.inertia, mul(axis, applied)));
+            }
+        }
+        if (spins) {
+            const float mass = dot3(normal, inverse_inertia_at(bf.q, split_f, normal)) +
+                               dot3(normal, inverse_inertia_at(bs.q, split_s, normal));
+            if (mass > 0.0f) {
+                const float applied = clampf(-twist / mass, -spin_limit, spin_limit);
+                first_w = sub(first_w, inverse_inertia_at(bf.q, bf.inertia, mul(normal, applied)));
+                second_w = add(second_w, inverse_inertia_at(bs.q, bs.inertia, mul(normal, applied)));
+            }
         }
     }
     imp[0] = make_float4(acc_n[0], acc_n[1], acc_n[2], acc_n[3]);
