@@ -1459,10 +1459,38 @@ __global__ void __launch_bounds__(kThreads) k_relay(W w) {
     cur.events |= kContactAnnounced;
 }
 
+// The rows a contact links in the island pass (island_link.wgsl:47-60): a touching, non-sensor
+// contact between colliders and bodies inside the records; kNoSlot twice otherwise.
+__device__ __forceinline__ uint2 island_edge(const W& w, uint32_t i, float slop) {
+    const uint2 none = make_uint2(kNoSlot, kNoSlot);
+    const dyn_contact& c = w.contacts[i];
+    if (c.point_count == 0u || c.sensor == 1u || !touches(c, slop)) return none;
+    // colliders or bodies outside the records (possible only for contacts handed to dyn_islands)
+    // link nothing
+    if (c.a >= w.k || c.b >= w.k) return none;
+    const uint32_t fb = w.owner[c.a], sb = w.owner[c.b];
+    if (fb >= w.n || sb >= w.n) return none;
+    return make_uint2(fb, sb);
+}
+
+// The island pass's first part: each contact's linking rows go to iedges (when present), and
+// every linking contact between two simulated rows points the higher row's parent at the lower
+// row (an atomic minimum, so each row ends at its lowest linked neighbour below it, or itself).
+// Parents still point only at lower rows of the same component, so the hooks and the flatten
+// rounds end at the same minimum-row roots; most rows then start a few hops from their root.
+// (A row's contacts sit together in the list but mostly as its lower side: one atomic a lane.)
+__device__ __forceinline__ void island_seed_at(const W& w, uint32_t i, float slop) {
+    const uint2 e = island_edge(w, i, slop);
+    if (w.iedges) w.iedges[i] = e;
+    if (e.x < w.d && e.y < w.d && e.x != e.y) atomicMin(&w.parents[max(e.x, e.y)], min(e.x, e.y));
+}
+
 // contact_begin.wgsl:41-71 over the resting archive sorted by (min id, max id)
 __global__ void __launch_bounds__(kThreads) k_contact_begin(W w, float slop) {
     const uint32_t index = blockIdx.x * blockDim.x + threadIdx.x;
-    if (index >= *w.ncontacts || w.matched[index]) return;
+    if (index >= *w.ncontacts) return;
+    island_seed_at(w, index, slop);  // reads nothing that this pass changes
+    if (w.matched[index]) return;
     // changed in place: the fields below are the only ones a copy written back would change
     dyn_contact& c = w.contacts[index];
     const uint32_t kmaj = min(c.first_body_id, c.second_body_id);
@@ -1611,20 +1639,6 @@ __device__ inline void island_couple(const W& w, uint32_t a, uint32_t b) {
     atomicAdd(cw(w.counters, DYN_COUNTER_ISLAND_FAULTS), 1u);
 }
 
-// The rows a contact links in the island pass (island_link.wgsl:47-60): a touching, non-sensor
-// contact between colliders and bodies inside the records; kNoSlot twice otherwise.
-__device__ __forceinline__ uint2 island_edge(const W& w, uint32_t i, float slop) {
-    const uint2 none = make_uint2(kNoSlot, kNoSlot);
-    const dyn_contact& c = w.contacts[i];
-    if (c.point_count == 0u || c.sensor == 1u || !touches(c, slop)) return none;
-    // colliders or bodies outside the records (possible only for contacts handed to dyn_islands)
-    // link nothing
-    if (c.a >= w.k || c.b >= w.k) return none;
-    const uint32_t fb = w.owner[c.a], sb = w.owner[c.b];
-    if (fb >= w.n || sb >= w.n) return none;
-    return make_uint2(fb, sb);
-}
-
 __device__ __forceinline__ uint2 island_edge_at(const W& w, uint32_t i, float slop) {
     return w.iedges ? w.iedges[i] : island_edge(w, i, slop);
 }
@@ -1712,24 +1726,10 @@ __global__ void __launch_bounds__(kThreads) k_solve_stage_check(W w, uint32_t* w
     if (c.a >= w.k || c.b >= w.k || w.owner[c.a] >= w.n || w.owner[c.b] >= w.n) atomicOr(&words[1], 1u);
 }
 
-// The island pass's first kernel: each contact's linking rows go to iedges (when present), and
-// every linking contact between two simulated rows points the higher row's parent at the lower
-// row (an atomic minimum, so each row ends at its lowest linked neighbour below it, or itself).
-// Parents still point only at lower rows of the same component, so the hooks and the flatten
-// rounds end at the same minimum-row roots; most rows then start a few hops from their root.
+// island_seed_at alone, for dyn_islands (a step's k_contact_begin seeds).
 __global__ void __launch_bounds__(kThreads) k_island_seed(W w, float slop) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool take = false;
-    uint32_t hi = 0, lo = 0;
-    if (i < min(*w.ncontacts, w.contact_cap)) {
-        const uint2 e = island_edge(w, i, slop);
-        if (w.iedges) w.iedges[i] = e;
-        take = e.x < w.d && e.y < w.d && e.x != e.y;
-        hi = max(e.x, e.y);
-        lo = min(e.x, e.y);
-    }
-    // a row's contacts sit together in the list but mostly as its lower side: one atomic a lane
-    if (take) atomicMin(&w.parents[hi], lo);
+    if (i < min(*w.ncontacts, w.contact_cap)) island_seed_at(w, i, slop);
 }
 
 // dyn_islands' set-up: no wake or motion flags, the island counters at zero.
@@ -1838,20 +1838,131 @@ __global__ void __launch_bounds__(kThreads) k_island_aggregate(W w) {
     block_count(cw(w.counters, DYN_COUNTER_ISLANDS), roots);
 }
 
-// island_wake.wgsl
+// island_wake.wgsl; `woken`: the row's island wakes.
+__device__ __forceinline__ uint32_t island_wake_at(const W& w, uint32_t i, bool woken) {
+    w.wake[i] = 0u;
+    if (!woken || w.st[i].sleeping == 0u) return 0u;
+    w.st[i].sleeping = 0u;
+    w.st[i].sleep_timer = 0.0f;
+    return 1u;
+}
+
 __global__ void __launch_bounds__(kThreads) k_island_wake(W w) {
     uint32_t woke = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < w.d; i += gridDim.x * blockDim.x) {
-        const uint32_t root = w.parents[i];
-        if (w.st[i].sleeping != 0u && (w.istate[root] & kIslandWake)) {
-            ++woke;
-            w.st[i].sleeping = 0u;
-            w.st[i].sleep_timer = 0.0f;
-        }
-        w.wake[i] = 0u;
+        woke += island_wake_at(w, i, (w.istate[w.parents[i]] & kIslandWake) != 0u);
     }
     block_count(cw(w.counters, DYN_COUNTER_WOKE), woke);
     block_count(cw(w.counters, DYN_COUNTER_WOKE_DEFERRED), woke);
+}
+
+// The island pass of a small world after its seeding, in one workgroup with the rows' parents and flags
+// in LDS: flatten, link every contact and resting contact, flatten, aggregate, wake (k_island_flatten,
+// k_island_link, k_island_aggregate, k_island_wake; the hooking rounds only shorten the link's walks,
+// which are cheap here). Ten launches of 6 to 10 us each became one of 9 us at 25 rows and 13 us at
+// 1,001; larger worlds have the work to fill the launches, and their rows do not fit.
+constexpr uint32_t kIslandGroupRows = 4096;
+constexpr uint32_t kRowWoken = 1u, kRowIslandWakes = 2u;
+struct IslandLds {
+    uint32_t parents[kIslandGroupRows];
+    uint32_t flags[kIslandGroupRows];
+    uint32_t roots, woke;
+    __device__ __forceinline__ uint32_t parent(uint32_t row) const {
+        return __hip_atomic_load(&parents[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ uint32_t find(uint32_t row) const {
+        uint32_t up = parent(row);
+        while (up != row) {
+            row = up;
+            up = parent(row);
+        }
+        return row;
+    }
+};
+
+// Rounds of bounded walks, as k_island_flatten_rounds, until every row points at its root.
+__device__ inline void island_group_flatten(const W& w, IslandLds& l) {
+    int short_of_root;
+    do {
+        short_of_root = 0;
+        for (uint32_t i = threadIdx.x; i < w.d; i += 1024u) {
+            uint32_t at = l.parent(i), up = l.parent(at);
+            for (uint32_t hop = 0; up != at && hop < 16u; ++hop) {
+                at = up;
+                up = l.parent(at);
+            }
+            __hip_atomic_store(&l.parents[i], at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (up != at) short_of_root = 1;
+        }
+    } while (__syncthreads_or(short_of_root));
+}
+
+// island_couple on the rows in LDS.
+__device__ inline void island_group_couple(const W& w, IslandLds& l, uint32_t a, uint32_t b) {
+    if (b >= w.d && (l.flags[b] & kRowWoken)) atomicOr(&l.flags[a], kRowWoken);
+    if (a >= w.d && (l.flags[a] & kRowWoken)) atomicOr(&l.flags[b], kRowWoken);
+    if (a >= w.d || b >= w.d || a == b) return;
+    uint32_t ra = l.find(a), rb = l.find(b);
+    for (uint32_t attempt = 0; attempt < 256u; ++attempt) {
+        if (ra == rb) return;
+        const uint32_t lower = min(ra, rb), higher = max(ra, rb);
+        const uint32_t was = atomicMin(&l.parents[higher], lower);
+        if (was == higher) return;  // it was a root
+        ra = l.find(lower);
+        rb = l.find(was);
+    }
+    atomicAdd(cw(w.counters, DYN_COUNTER_ISLAND_FAULTS), 1u);
+}
+
+__global__ void __launch_bounds__(1024) k_island_group(W w) {
+    __shared__ IslandLds l;
+    const uint32_t t = threadIdx.x;
+    if (t == 0u) l.roots = l.woke = 0u;
+    for (uint32_t i = t; i < w.n; i += 1024u) {
+        if (i < w.d) l.parents[i] = w.parents[i];
+        l.flags[i] = w.wake[i] != 0u ? kRowWoken : 0u;
+    }
+    __syncthreads();
+    island_group_flatten(w, l);
+    const uint32_t count = min(*w.ncontacts, w.contact_cap), resting = *w.nresting;
+    for (uint32_t i = t; i < count; i += 1024u) {
+        const uint2 e = w.iedges[i];
+        if (e.x != kNoSlot) island_group_couple(w, l, e.x, e.y);
+    }
+    for (uint32_t i = t; i < resting; i += 1024u) {
+        const dyn_contact& c = w.resting[i];
+        const uint32_t r1 = resolve_row(w, c.first_body_id, c.first_generation);
+        const uint32_t r2 = resolve_row(w, c.second_body_id, c.second_generation);
+        if (r1 != DYN_NO_BODY && r2 != DYN_NO_BODY) island_group_couple(w, l, r1, r2);
+    }
+    __syncthreads();
+    island_group_flatten(w, l);
+    uint32_t roots = 0, woke = 0;
+    for (uint32_t i = t; i < w.d; i += 1024u) {
+        const uint32_t root = l.parents[i];
+        roots += root == i ? 1u : 0u;
+        if ((l.flags[i] & kRowWoken) || w.motion[i] != 0u) atomicOr(&l.flags[root], kRowIslandWakes);
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < w.d; i += 1024u) {
+        const uint32_t root = l.parents[i];
+        w.parents[i] = root;
+        w.istate[i] = l.flags[i] & kRowIslandWakes ? kIslandWake : 0u;
+        woke += island_wake_at(w, i, (l.flags[root] & kRowIslandWakes) != 0u);
+    }
+    roots = wave_sum(roots);
+    woke = wave_sum(woke);
+    if (lane_id() == 0u) {
+        if (roots) atomicAdd(&l.roots, roots);
+        if (woke) atomicAdd(&l.woke, woke);
+    }
+    __syncthreads();
+    if (t != 0u) return;
+    if (l.roots) atomicAdd(cw(w.counters, DYN_COUNTER_ISLANDS), l.roots);
+    if (l.woke) {
+        atomicAdd(cw(w.counters, DYN_COUNTER_WOKE), l.woke);
+        atomicAdd(cw(w.counters, DYN_COUNTER_WOKE_DEFERRED), l.woke);
+    }
 }
 
 // what k_blocks reads of a block's body, in one 48-byte record
@@ -3445,21 +3556,38 @@ int island_flatten(const dyn::W& w, hipStream_t st, uint32_t pass, uint32_t roun
     return DYN_OK;
 }
 
-// The contact part of the island pass, before the resting archive's links and the last flatten:
-// the seeding pass (which also lists each contact's linking rows), then kHookRounds hooking
-// rounds, a flatten round (walks of up to 64 hops) before each and after the last, then the
-// retrying hooks over every contact. The rounds only shorten the hooks' work: neither needs a
-// flat forest, and k_island_link alone would end at the same components.
+// The contact part of the island pass after the seeding (which also lists each contact's linking
+// rows) and before the last flatten: kHookRounds hooking rounds, a flatten round (walks of up to 64
+// hops) before each and after the last, then the retrying hooks over every contact, a resting
+// archive's among them. The rounds only shorten the hooks' work: neither needs a flat forest, and
+// k_island_link alone would end at the same components.
 int island_components(const dyn::W& w, hipStream_t st, float slop) {
     using namespace dyn;
     const uint32_t cb = blocks_for(w.contact_cap);
-    LAUNCH_ON(st, k_island_seed, cb, w, slop);
     DYN_TRY(island_flatten(w, st, 0u, 1u));
     for (uint32_t h = 0; h < kHookRounds; ++h) {
         LAUNCH_ON(st, k_island_hook, cb, w, slop);
         DYN_TRY(island_flatten(w, st, 1u + h, 1u));
     }
     LAUNCH_ON(st, k_island_link, cb, w, slop);
+    return DYN_OK;
+}
+
+// A step's island pass after k_contact_begin.
+int islands(const dyn::W& w, hipStream_t st) {
+    using namespace dyn;
+    if (w.n <= kIslandGroupRows) {
+        {
+            ProfileScope scope("k_island_group", st);
+            k_island_group<<<1, 1024, 0, st>>>(w);
+        }
+        DYN_LAUNCHED("k_island_group");
+        return DYN_OK;
+    }
+    DYN_TRY(island_components(w, st, w.p.slop));
+    DYN_TRY(island_flatten(w, st, kFlattenPasses - 1u));
+    LAUNCH_ON(st, k_island_aggregate, count_blocks(w.d), w);
+    LAUNCH_ON(st, k_island_wake, count_blocks(w.d), w);
     return DYN_OK;
 }
 
@@ -3744,10 +3872,7 @@ int world_step(dyn_world* world, float dt) {
     if (world->tape_states) LAUNCH(k_tape_sources, blocks_for(4u * w.contact_cap), w);
     LAUNCH(k_relay, cb, w);
     LAUNCH(k_contact_begin, cb, w, w.p.slop);
-    DYN_TRY(island_components(w, st, w.p.slop));
-    DYN_TRY(island_flatten(w, st, kFlattenPasses - 1u));
-    LAUNCH(k_island_aggregate, count_blocks(w.d), w);
-    LAUNCH(k_island_wake, count_blocks(w.d), w);
+    DYN_TRY(islands(w, st));
     if (world->tape_states) {
         LAUNCH(k_tape_record, blocks_for(std::max(w.n, w.contact_cap)), w, world->tape_states, world->tape_contacts,
                world->tape_count, world->tape_error);
@@ -4517,6 +4642,7 @@ int dyn_islands(void* stream, const dyn_islands_io* io) {
     if (w.d == 0u) return DYN_OK;
     LAUNCH_ON(st, k_island_init, db, w);
     if (w.contact_cap) {
+        LAUNCH_ON(st, k_island_seed, blocks_for(w.contact_cap), w, io->slop);
         DYN_TRY(island_components(w, st, io->slop));
     }
     DYN_TRY(island_flatten(w, st, kFlattenPasses - 1u));
