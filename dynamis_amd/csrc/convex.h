@@ -1265,19 +1265,16 @@ __device__ inline bool convex_hit_after_gjk(const Pair& p, const ShapeSet& ss, c
 __device__ inline Hit convex_hit_finish(const Shape& first, const Shape& second, const ShapeSet& ss,
                                         const SimplexPoint* simplex, uint32_t count, const Epa& epa) {
     const v3 centers = sub(second.center, first.center);
-    Hit result;
-    if (epa.valid && epa.depth > 0.0f && epa.depth < kBig && len3(epa.normal) > 0.5f &&
-        epa.depth < support_projection_depth(first, second, ss, epa.normal) +
-                        0.1f * fmn(shape_scale(first), shape_scale(second))) {
-        result = make_hit(-epa.depth,
-                          mul(add(support(first, ss, epa.normal), support(second, ss, neg(epa.normal))), 0.5f),
-                          epa.normal);
-    } else {
+    v3 normal = epa.normal;
+    float depth = epa.depth;
+    if (!(epa.valid && epa.depth > 0.0f && epa.depth < kBig && len3(epa.normal) > 0.5f &&
+          epa.depth < support_projection_depth(first, second, ss, epa.normal) +
+                          0.1f * fmn(shape_scale(first), shape_scale(second)))) {
         const Probe probe = penetration_probe(first, second, ss, simplex, count, false);
-        result = make_hit(-probe.depth,
-                          mul(add(support(first, ss, probe.normal), support(second, ss, neg(probe.normal))), 0.5f),
-                          probe.normal);
+        normal = probe.normal;
+        depth = probe.depth;
     }
+    Hit result = make_hit(-depth, mul(add(support(first, ss, normal), support(second, ss, neg(normal))), 0.5f), normal);
     if (dot3(result.normal, centers) < 0.0f) result.normal = neg(result.normal);
     return result;
 }
@@ -1382,10 +1379,17 @@ __device__ inline void hull_feature_ring(const Shape& w, const ShapeSet& ss, v3 
     uint32_t ids[16];
     ids[0] = 0u;
     uint32_t count = 0, first_id = kEmptyRingFace;
-    for (uint32_t i = 0; i < src.vertex_count && count < 16u; ++i) {
-        const v3 v = hull_vertex(ss, src, i);
-        if (dot3(v, d) >= best_dot - eps) {
-            points[count] = add(w.center, qrot(w.rotation, mulv(v, w.scale)));
+    // eight vertices in flight at a time: one after another, a lane waited for each of up to 64 loads
+    for (uint32_t base = 0; base < src.vertex_count && count < 16u; base += 8u) {
+        uint32_t on = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const v3 v = hull_vertex(ss, src, min(base + k, src.vertex_count - 1u));
+            if (base + k < src.vertex_count && dot3(v, d) >= best_dot - eps) on |= 1u << k;
+        }
+        for (; on != 0u && count < 16u; on &= on - 1u) {
+            const uint32_t i = base + static_cast<uint32_t>(__ffs(static_cast<int>(on))) - 1u;
+            points[count] = add(w.center, qrot(w.rotation, mulv(hull_vertex(ss, src, i), w.scale)));
             ids[count] = i;
             first_id = first_id < i ? first_id : i;
             ++count;
@@ -1552,11 +1556,11 @@ __device__ inline uint32_t clip_feature_to_ring(const Feature& inc, const Featur
 }
 
 // convex.wgsl:984-1071
-__device__ inline bool convex_pair_manifold(const Shape& first, const Shape& second, const ShapeSet& ss,
-                                            v3 direction, Manifold& m) {
-    Feature fa, fb;
-    shape_feature(first, ss, direction, &fa);
-    shape_feature(second, ss, neg(direction), &fb);
+// The candidates of the two shapes' features across `direction`; false when the hit's own point
+// is the manifold (`hit`), or when the deepest point of the incident feature, which is pushed.
+__device__ inline bool convex_pair_candidates(const Feature& fa, const Feature& fb, v3 direction, Manifold& m,
+                                              Candidates& cand, bool* hit) {
+    *hit = true;
     if (!fa.ring && !fb.ring) return false;
     bool first_reference = fa.ring;
     if (fa.ring && fb.ring) first_reference = feature_radius(fa) >= feature_radius(fb);
@@ -1578,8 +1582,6 @@ __device__ inline bool convex_pair_manifold(const Shape& first, const Shape& sec
     v3 clipped[kCandidates];
     uint32_t clipped_ids[kCandidates];
     const uint32_t clipped_count = clip_feature_to_ring(inc, ref, ref_dir, clipped, clipped_ids);
-    Candidates cand;
-    cand.count = 0;
     for (uint32_t i = 0; i < clipped_count && cand.count < kCandidates; ++i) {
         const float depth = dot3(sub(center, clipped[i]), ref_dir);
         if (depth > 0.0f) {
@@ -1590,13 +1592,11 @@ __device__ inline bool convex_pair_manifold(const Shape& first, const Shape& sec
             ++cand.count;
         }
     }
-    if (cand.count == 0u) {
-        if (deepest_depth <= 0.0f) return false;
-        push(m, sub(deepest, mul(ref_dir, deepest_depth * 0.5f)), deepest_depth, kFeaturePoint);
-        return true;
-    }
-    keep(m, cand);
-    return true;
+    if (cand.count == 0u && deepest_depth <= 0.0f) return false;
+    *hit = false;
+    if (cand.count != 0u) return true;
+    push(m, sub(deepest, mul(ref_dir, deepest_depth * 0.5f)), deepest_depth, kFeaturePoint);
+    return false;
 }
 
 // narrowphase.wgsl:479-483
@@ -1604,29 +1604,19 @@ __device__ __forceinline__ void manifold_from_hit(Manifold& m, const Hit& hit, f
     if (hit.distance <= margin) push(m, hit.point, -hit.distance, kFeaturePoint);
 }
 
-// narrowphase.wgsl:485-512
-__device__ inline void plane_convex(Manifold& m, const Shape& plane, const Shape& convex, const ShapeSet& ss,
-                                    float margin) {
-    const v3 n = qrot(plane.rotation, mk(0.0f, 1.0f, 0.0f));
-    const float center_side = dot3(sub(convex.center, plane.center), n);
-    const v3 facing = center_side < 0.0f ? neg(n) : n;
-    emit(m, facing);
-    Feature f;
-    shape_feature(convex, ss, neg(facing), &f);
-    Candidates cand;
-    cand.count = 0;
+// narrowphase.wgsl:485-512 from a shape's feature: the candidates within the margin of the plane.
+__device__ inline void plane_candidates(const Feature& f, v3 plane_center, v3 facing, float margin, Candidates& cand) {
     for (uint32_t i = 0; i < f.count; ++i) {
-        const float depth = dot3(sub(plane.center, f.p[i]), facing);
+        const float depth = dot3(sub(plane_center, f.p[i]), facing);
         if (depth <= -margin) continue;
         cand.pos[cand.count] = add(f.p[i], mul(facing, depth * 0.5f));
         cand.depth[cand.count] = depth;
         cand.feature[cand.count] = feature_pair(kFeatureVertex, kFeatureFaceBit | 0u, f.id[i]);
         ++cand.count;
     }
-    keep(m, cand);
 }
 
-// plane_convex for the shapes k_narrow gives it (sphere, box, capsule): the same feature
+// A plane against the shapes k_narrow gives it (sphere, box, capsule): the same feature
 // (shape_feature's branches for those kinds), candidates and selection, with every array
 // addressed at compile-time indices so that none sits in scratch memory.
 __device__ inline void plane_analytic(Manifold& m, const Shape& plane, const Shape& convex, const ShapeSet& ss,
@@ -1657,7 +1647,7 @@ __device__ inline void plane_analytic(Manifold& m, const Shape& plane, const Sha
     for (uint32_t i = 0; i < 4; ++i) {  // a box face, a capsule side or one point
         if (i < f.count) {
             const float depth = dot3(sub(plane.center, f.p[i]), facing);
-            if (!(depth <= -margin)) {  // plane_convex's test, NaN included
+            if (!(depth <= -margin)) {  // plane_candidates' test, NaN included
                 cand_push(cand, add(f.p[i], mul(facing, depth * 0.5f)), depth,
                           feature_pair(kFeatureVertex, kFeatureFaceBit | 0u, f.id[i]));
             }

@@ -1066,20 +1066,18 @@ __device__ __forceinline__ void finish_pair(const W& w, uint32_t index, uint32_t
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     const Shape wf = world_collider(first.s, fc), wsd = world_collider(second.s, sc);
     const float* park = parked(w, index);
+    const bool plane = mark == kPairPlane, plane_first = plane && fc.kind == DYN_SHAPE_PLANE;
     Manifold m;
-    m.count = 0;
-    m.normal = zero3v();
-    bool mirrored_features = false;
-    if (mark == kPairPlane) {
-        if (fc.kind == DYN_SHAPE_PLANE) {
-            plane_convex(m, wf, wsd, shapes, margin);
-        } else {
-            plane_convex(m, wsd, wf, shapes, margin);
-            mirror(m);
-            mirrored_features = true;
-        }
+    Hit hit;
+    v3 direction;  // from the first shape to the second
+    if (plane) {   // narrowphase.wgsl:485-512
+        const Shape& ground = plane_first ? wf : wsd;
+        const v3 n = qrot(ground.rotation, mk(0.0f, 1.0f, 0.0f));
+        const float center_side = dot3(sub((plane_first ? wsd : wf).center, ground.center), n);
+        const v3 facing = center_side < 0.0f ? neg(n) : n;
+        emit(m, facing);
+        direction = plane_first ? facing : neg(facing);
     } else {
-        Hit hit;
         if (mark == kPairHit) {
             hit = make_hit(park[0], mk(park[1], park[2], park[3]), mk(park[4], park[5], park[6]));
         } else {
@@ -1095,8 +1093,29 @@ __device__ __forceinline__ void finish_pair(const W& w, uint32_t index, uint32_t
             if (!(hit.distance <= margin)) return;
         }
         emit(m, hit.normal);
-        if (!convex_pair_manifold(wf, wsd, shapes, hit.normal, m)) manifold_from_hit(m, hit, margin);
+        direction = hit.normal;
     }
+    // One copy of the features' code for both shapes and both kinds of pair, and one of the selection's:
+    // a few pairs wait for every new line of code to be fetched, and four copies made it 21,400
+    // instructions (now 12,400; 77 us to 65 for 24 bodies, the same at 20,000).
+    Feature features[2];
+#pragma unroll 1
+    for (uint32_t k = plane_first ? 1u : 0u; k < (plane && !plane_first ? 1u : 2u); ++k) {
+        shape_feature(k ? wsd : wf, shapes, k ? neg(direction) : direction, &features[k]);
+    }
+    Candidates cand;
+    cand.count = 0;
+    bool chosen = true;
+    if (plane) {
+        plane_candidates(features[plane_first ? 1 : 0], (plane_first ? wf : wsd).center, m.normal, margin, cand);
+    } else {
+        bool alone;
+        chosen = convex_pair_candidates(features[0], features[1], direction, m, cand, &alone);
+        if (alone) manifold_from_hit(m, hit, margin);
+    }
+    if (chosen) keep(m, cand);
+    const bool mirrored_features = plane && !plane_first;
+    if (mirrored_features) mirror(m);
     if (m.count == 0u) return;
     write_contact(w, index, fs, ss, first, second, fc, sc, m, mirrored_features);
 }
