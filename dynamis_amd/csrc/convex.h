@@ -1348,17 +1348,24 @@ __device__ inline void ring_of(const Shape& w, const ShapeSet& ss, v3 direction,
     const v3 u = fabsf(n.x) > 0.9f ? norm3(cross3(n, mk(0.0f, 1.0f, 0.0f))) : norm3(cross3(n, mk(1.0f, 0.0f, 0.0f)));
     const v3 v = cross3(n, u);
     for (uint32_t i = 0; i < count; ++i) {
+        v3 first = points[i];
+        uint32_t first_id = ids[i];
+        float x = dot3(sub(first, center), u), y = dot3(sub(first, center), v);
         for (uint32_t j = i + 1; j < count; ++j) {
-            const v3 pa = sub(points[i], center), pb = sub(points[j], center);
-            if (angle_before(dot3(pb, u), dot3(pb, v), dot3(pa, u), dot3(pa, v))) {
-                const v3 tp = points[i];
-                points[i] = points[j];
-                points[j] = tp;
-                const uint32_t ti = ids[i];
-                ids[i] = ids[j];
-                ids[j] = ti;
+            const v3 other = points[j];
+            const float ox = dot3(sub(other, center), u), oy = dot3(sub(other, center), v);
+            if (angle_before(ox, oy, x, y)) {
+                const uint32_t other_id = ids[j];
+                points[j] = first;
+                ids[j] = first_id;
+                first = other;
+                first_id = other_id;
+                x = ox;
+                y = oy;
             }
         }
+        points[i] = first;
+        ids[i] = first_id;
     }
     const uint32_t keep = count < kFeatureMax ? count : kFeatureMax;
     for (uint32_t i = 0; i < keep; ++i) {
@@ -1498,7 +1505,7 @@ __device__ inline uint32_t clip_feature_to_ring(const Feature& inc, const Featur
     uint32_t* kept_ids = spare_ids;
     uint32_t live = inc.count;
     for (uint32_t side = 0; side < ref.count; ++side) {
-        const v3 current = ref.p[side], next = ref.p[(side + 1u) % ref.count];
+        const v3 current = ref.p[side], next = ref.p[side + 1u == ref.count ? 0u : side + 1u];
         const v3 plane_normal = norm3(cross3(sub(next, current), ref_dir));
         uint32_t written = 0;
         if (live == 2u) {
@@ -1521,10 +1528,19 @@ __device__ inline uint32_t clip_feature_to_ring(const Feature& inc, const Featur
                 ++written;
             }
         } else {
+            // each point is read and measured once, as the next one of its predecessor
+            v3 cp = live ? from[0] : zero3v();
+            float cs = dot3(sub(cp, current), plane_normal) - kClipMargin;
+            const v3 p0 = cp;
+            const float s0 = cs;
             for (uint32_t i = 0; i < live; ++i) {
-                const v3 cp = from[i], np = from[(i + 1u) % live];
-                const float cs = dot3(sub(cp, current), plane_normal) - kClipMargin;
-                const float ns = dot3(sub(np, current), plane_normal) - kClipMargin;
+                const bool last = i + 1u == live;
+                v3 np = p0;
+                float ns = s0;
+                if (!last) {
+                    np = from[i + 1u];
+                    ns = dot3(sub(np, current), plane_normal) - kClipMargin;
+                }
                 if (cs <= 0.0f && written < kCandidates) {
                     kept[written] = cp;
                     kept_ids[written] = from_ids[i];
@@ -1535,6 +1551,8 @@ __device__ inline uint32_t clip_feature_to_ring(const Feature& inc, const Featur
                     kept_ids[written] = kFeatureClip | (side * kCandidates + i);
                     ++written;
                 }
+                cp = np;
+                cs = ns;
             }
         }
         live = written;

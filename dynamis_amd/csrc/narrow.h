@@ -194,12 +194,6 @@ __device__ __forceinline__ void swap_candidates(Candidates& c, uint32_t i, uint3
     c.feature[j] = f;
 }
 
-__device__ __forceinline__ float gap_of(const Candidates& c, uint32_t kept, uint32_t index) {
-    float gap = 3.402823466e38f;
-    for (uint32_t h = 0; h < kept; ++h) gap = fmn(gap, len3(sub(c.pos[index], c.pos[h])));
-    return gap;
-}
-
 // core.wgsl:720-760: deepest first (ties by feature), then farthest from the kept ones.
 __device__ __forceinline__ void keep(Manifold& m, Candidates& c) {
     const uint32_t n = c.count;
@@ -212,17 +206,24 @@ __device__ __forceinline__ void keep(Manifold& m, Candidates& c) {
     // Round k only reorders places k and above, and at most four places are pushed, so the
     // rounds past the fourth place change nothing that is read.
     const uint32_t placed = min(n, static_cast<uint32_t>(DYN_CONTACT_MAX_POINTS));
+    float gap[kCandidates];  // to the nearest kept place
+    for (uint32_t i = 1; i < n; ++i) gap[i] = 3.402823466e38f;
     for (uint32_t kept = 1; kept < placed; ++kept) {
+        const v3 latest = c.pos[kept - 1u];
         uint32_t best = kept;
-        float best_gap = gap_of(c, kept, kept);
-        for (uint32_t i = kept + 1; i < n; ++i) {
-            const float g = gap_of(c, kept, i);
-            if (g > best_gap) {
+        float best_gap = 0.0f;
+        for (uint32_t i = kept; i < n; ++i) {
+            const float g = fmn(gap[i], len3(sub(c.pos[i], latest)));
+            gap[i] = g;
+            if (i == kept || g > best_gap) {
                 best_gap = g;
                 best = i;
             }
         }
-        if (best != kept) swap_candidates(c, kept, best);
+        if (best != kept) {
+            swap_candidates(c, kept, best);
+            gap[best] = gap[kept];
+        }
     }
     for (uint32_t i = 0; i < n && m.count < DYN_CONTACT_MAX_POINTS; ++i) {
         push(m, c.pos[i], c.depth[i], c.feature[i]);
