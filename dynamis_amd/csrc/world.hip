@@ -2913,7 +2913,9 @@ __device__ __forceinline__ bool position_correction(const W& w, const PositionRo
         ++contributing;
     }
     if (contributing == 0u) return false;
-    const v3 correction = dv(total, static_cast<float>(contributing));
+    // over the contributing points; a half and a quarter are the divisions by two and four, bit for bit
+    v3 correction = mul(total, contributing == 4u ? 0.25f : (contributing == 2u ? 0.5f : 1.0f));
+    if (contributing == 3u) correction = dv(total, 3.0f);
     const v3 la = mul(neg(correction), imf), lb = mul(correction, ims);
     if (!(dot3(la, la) > 0.0f || dot3(lb, lb) > 0.0f)) return false;
     *la_out = la;
@@ -2961,11 +2963,9 @@ __device__ __forceinline__ void position_move(v3 p0, float4 q0, uint32_t x, uint
                                               v3* p1, float4* q1, v3* moved) {
     const v3 lin = mk(solver_value(x, DYN_SOLVER_POSITION_SCALE), solver_value(y, DYN_SOLVER_POSITION_SCALE),
                       solver_value(z, DYN_SOLVER_POSITION_SCALE));
-    const float none = solver_value(0u, DYN_SOLVER_POSITION_SCALE);
-    const float cf = static_cast<float>(contributing);
-    const v3 al = dv(lin, cf), aa = dv(mk(none, none, none), cf);
+    const v3 al = dv(lin, static_cast<float>(contributing));
     *p1 = add(p0, al);
-    *q1 = qnorm(qmul(make_float4(aa.x * 0.5f, aa.y * 0.5f, aa.z * 0.5f, 1.0f), q0));
+    *q1 = qnorm(qmul(make_float4(0.0f, 0.0f, 0.0f, 1.0f), q0));  // no angle, of however many blocks
     *moved = al;
 }
 
