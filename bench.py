@@ -85,18 +85,18 @@ def broadphase_bytes(name: str, k: int, entries: int, pairs: int) -> float:
     record 32 bytes; box = 24 bytes of min/max; pair = 8 bytes)."""
     if name == "entry_sort_pass":        # read key+slot, write key+slot
         return 16.0 * entries
-    if name in ("bp_mates_count_kernel", "bp_mates_emit_kernel"):  # every sorted key read once;
-        return 4.0 * entries + 8.0 * pairs                             # a pair's record each
-    if name in ("bp_links_count_kernel", "bp_links_emit_kernel"):  # box + packed count per collider;
-        return 28.0 * k + 8.0 * pairs                                  # a pair's record each
+    if name == "bp_pairs_count_kernel":  # box + packed count per collider, every sorted key read once,
+        return 28.0 * k + 4.0 * entries + 8.0 * pairs  # a pair's record each
+    if name == "bp_pairs_emit_kernel":   # each collider's and entry's count in, a pair's record in and out
+        return 4.0 * k + 4.0 * entries + 16.0 * pairs
     if name == "bp_emit_kernel":         # box + packed count in; key, slot, record out
         return 28.0 * k + 40.0 * entries
     if name == "bp_count_kernel":        # box in, packed count out
         return 28.0 * k
     if name == "bp_resolution_kernel":   # box in
         return 24.0 * k
-    if name == "pair_sort_pass":         # 3 lanes in and out
-        return 24.0 * pairs
+    if name == "pair_sort_pass":         # both key lanes in and out
+        return 16.0 * pairs
     if name == "pair_sort_histogram":
         return 8.0 * pairs
     return 0.0
@@ -127,7 +127,7 @@ def step_bytes(name: str, n: int, k: int, entries: int, pairs: int, contacts: in
         return contacts * 16.0
     if name == "k_narrow":              # worklist entry, two bodies and colliders per pair, manifold out
         return pairs * 320.0 + contacts * manifold
-    if name == "k_pair_class":          # the pair, both colliders' kinds, the class out
+    if name == "k_class_count":         # the pair, both colliders' kinds, the class out
         return pairs * 17.0
     if name == "k_narrow_convex":       # the GJK worklist: pair record + index, parked results
         return gjk * 320.0 + manifold_pairs * 68.0 + gjk_resumed * 208.0  # and parked GJK states
@@ -139,10 +139,14 @@ def step_bytes(name: str, n: int, k: int, entries: int, pairs: int, contacts: in
         return epa_wave * (4.0 + 316.0 + 48.0 + 20.0)
     if name == "k_narrow_finish":       # pair record, parked result, contact out
         return manifold_pairs * (316.0 + 68.0 + 352.0)
-    if name in ("k_integrate", "k_advance"):
+    if name == "k_integrate":           # pose, velocity and constants; the claimed rows' solver records out
+        return n * 126.0 + rows * 112.0
+    if name == "k_advance":
         return n * 126.0
-    if name in ("k_relay", "k_contact_begin", "k_contacts_scatter"):
+    if name in ("k_relay", "k_contacts_scatter"):
         return 2.0 * contacts * manifold
+    if name == "k_contact_begin":       # and the island pass's linking rows out
+        return contacts * (2.0 * manifold + 16.0)
     if name == "k_archive":             # the archive is the swapped contact buffer: freeze marks only
         return contacts * 40.0
     return broadphase_bytes(name, k, entries, pairs)

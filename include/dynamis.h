@@ -459,7 +459,7 @@ int dyn_world_set_graphs(dyn_world* world, int enabled);
 /* Blocks until every enqueued step has finished. */
 int dyn_world_wait(dyn_world* world);
 /* The workgroup size of the solver substeps' per-contact and per-row kernels (k_integrate,
- * k_solver_bodies, k_solve_prep, k_warm, k_solve, k_apply, k_advance, k_position_block,
+ * k_solve_prep, k_solve, k_apply, k_advance, k_position_block,
  * k_position_apply, k_impulses_store): 64, 128 or 256 (default). Each of them indexes its contact
  * or row by the global thread index alone, so every size gives the same result. No counterpart in
  * the reference, whose programs have a fixed workgroup size. dyn_world_tune_solver times `steps`
