@@ -90,10 +90,10 @@ struct W {
     uint8_t* pkind;        // per convex pair: the unordered class of its two shape kinds
     uint32_t* worklist;    // pair lists (WorkList): every candidate pair by kind class, then GJK's open
                            // pairs, then the penetrating pairs (front) and the hits (from the end)
-    uint32_t* class_hist;  // per kind class and block of pairs: count, then offset in the class;
-                           // then the classes' totals
     uint32_t* work_total;  // device words: the lists' lengths (WorkTotal)
-    uint32_t* work_minor;  // pair lists: GJK's pairs, then the wave EPA's (front), the plane pairs (from the end)
+    uint32_t* work_minor;  // pair lists: GJK's pairs, then the wave EPA's (front), the plane pairs (from the end);
+                           // before them, per kind class and block of pairs its count, then its offset in
+                           // the class, and the classes' totals
     dyn_contact* contacts;
     uint2* ckeys;          // per contact: its collider pair (a, b), the key the relay searches
     uint32_t* matched;
@@ -569,8 +569,8 @@ struct BlockLists {
 
 constexpr uint32_t kClasses = 32;       // unordered pairs of 7 kind slots (28) and spare
 constexpr uint32_t kHullClasses = 21;   // the classes of pairs with a hull come last, from here
-constexpr uint32_t kClassItems = 16;
-constexpr uint32_t kClassBlock = kThreads * kClassItems;  // 4096 pairs per block
+constexpr uint32_t kClassItems = 4;
+constexpr uint32_t kClassBlock = kThreads * kClassItems;  // 1024 pairs per block
 
 __device__ __forceinline__ uint32_t kind_slot(uint32_t kind) {
     switch (kind) {
@@ -614,8 +614,9 @@ __global__ void __launch_bounds__(kThreads) k_class_count(W w) {
     __syncthreads();
     const uint32_t live = min(*cw(w.counters, DYN_COUNTER_PAIRS), w.pair_cap);
     const uint32_t base = blockIdx.x * kClassBlock;
-    // a block is few waves and its pairs' kinds two dependent reads away: all its reads in flight at once
-    // (114,000 pairs are 28 blocks; 21 us one pair after another)
+    // A pair's kinds are two dependent reads away, on lines of their own: what bounds a block is the lines
+    // that its CU can take in, so blocks are small (4,096 pairs a block took 22 us at 114,000 pairs, which
+    // then are 28 blocks; 1,024 take 9).
     uint32_t kinds[kClassItems];
 #pragma unroll
     for (uint32_t j = 0; j < kClassItems; ++j) {
@@ -630,7 +631,7 @@ __global__ void __launch_bounds__(kThreads) k_class_count(W w) {
         atomicAdd(&hist[kinds[j]], 1u);
     }
     __syncthreads();
-    if (threadIdx.x < kClasses) w.class_hist[threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
+    if (threadIdx.x < kClasses) w.work_minor[threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
 }
 
 // One workgroup per kind class: the class's block counts become offsets within the class, and
@@ -662,9 +663,9 @@ __global__ void __launch_bounds__(kThreads) k_class_scatter(W w) {
     __shared__ uint32_t cursor[kClasses];
     if (threadIdx.x < kWave) {
         const uint32_t c = threadIdx.x;
-        const uint32_t total = c < kClasses ? w.class_hist[static_cast<size_t>(kClasses) * gridDim.x + c] : 0u;
+        const uint32_t total = c < kClasses ? w.work_minor[static_cast<size_t>(kClasses) * gridDim.x + c] : 0u;
         const uint32_t inclusive = wave_inclusive_sum(total);
-        if (c < kClasses) cursor[c] = inclusive - total + w.class_hist[c * gridDim.x + blockIdx.x];
+        if (c < kClasses) cursor[c] = inclusive - total + w.work_minor[c * gridDim.x + blockIdx.x];
         if (blockIdx.x == 0u && c == kWave - 1u) w.work_total[kTotalAll] = inclusive;
     }
     __syncthreads();
@@ -3340,7 +3341,6 @@ int alloc_streams(dyn_world* world, uint32_t pair_capacity, uint32_t contact_cap
     A(w.valid, pair_capacity);
     A(w.pkind, pair_capacity);
     A(w.worklist, pair_capacity);
-    A(w.class_hist, kClasses * (static_cast<size_t>(ceil_div(pair_capacity ? pair_capacity : 1u, kClassBlock)) + 1u));
     A(w.work_minor, pair_capacity);
     A(w.contacts, contact_capacity);
     A(w.ckeys, contact_capacity);
@@ -3468,6 +3468,8 @@ int class_worklist(const dyn::W& w, hipStream_t st) {
         DYN_LAUNCHED("k_class_small");
         return DYN_OK;
     }
+    // the blocks' counts take 32 / 1,024 of a word per pair, and 64 words, of a list of a word per pair
+    static_assert(kClasses * (kClassSmall / kClassBlock + 2u) <= kClassSmall, "the counts fit the list");
     const uint32_t blocks = ceil_div(w.pair_cap, kClassBlock);
     {
         ProfileScope scope("k_class_count", st);
@@ -3476,7 +3478,7 @@ int class_worklist(const dyn::W& w, hipStream_t st) {
     DYN_LAUNCHED("k_class_count");
     {
         ProfileScope scope("k_class_scan", st);
-        k_class_scan<<<kClasses, 1024, 0, st>>>(w.class_hist, blocks, w.work_total);
+        k_class_scan<<<kClasses, 1024, 0, st>>>(w.work_minor, blocks, w.work_total);
     }
     DYN_LAUNCHED("k_class_scan");
     {
@@ -4450,7 +4452,7 @@ namespace {
 // dyn_narrowphase's scratch: the kind classes and the worklists.
 struct NarrowLayout {
     uint8_t* pkind;
-    uint32_t *worklist, *class_hist, *work_total, *work_minor;
+    uint32_t *worklist, *work_total, *work_minor;
     size_t bytes;
 };
 
@@ -4466,8 +4468,6 @@ NarrowLayout narrow_layout(uint32_t pair_capacity, void* base) {
     const size_t cap = pair_capacity ? pair_capacity : 1u;
     l.pkind = reinterpret_cast<uint8_t*>(take(cap));
     l.worklist = reinterpret_cast<uint32_t*>(take(4u * cap));
-    l.class_hist = reinterpret_cast<uint32_t*>(take(4u * kClasses * (static_cast<size_t>(ceil_div(
-                                                                          static_cast<uint32_t>(cap), kClassBlock)) + 1u)));
     l.work_total = reinterpret_cast<uint32_t*>(take(4u * kTotalWords));
     l.work_minor = reinterpret_cast<uint32_t*>(take(4u * cap));
     l.bytes = at;
@@ -4529,7 +4529,6 @@ int dyn_narrowphase(void* stream, const dyn_narrowphase_io* io) {
     w.valid = io->d_valid;
     w.pkind = l.pkind;
     w.worklist = l.worklist;
-    w.class_hist = l.class_hist;
     w.work_total = l.work_total;
     w.work_minor = l.work_minor;
     return narrowphase(w, static_cast<hipStream_t>(stream), true);
