@@ -1880,13 +1880,18 @@ __global__ void __launch_bounds__(kThreads) k_island_wake(W w) {
 // in LDS: flatten, link every contact and resting contact, flatten, aggregate, wake (k_island_flatten,
 // k_island_link, k_island_aggregate, k_island_wake; the hooking rounds only shorten the link's walks,
 // which are cheap here). Ten launches of 6 to 10 us each became one of 9 us at 25 rows and 13 us at
-// 1,001; larger worlds have the work to fill the launches, and their rows do not fit.
-constexpr uint32_t kIslandGroupRows = 4096;
-constexpr uint32_t kRowWoken = 1u, kRowIslandWakes = 2u;
+// 1,001. A step of 5,000 cubes takes 687 us so and 717 by launches, one of 8,000 756 and 792; the parents
+// of more rows than this do not fit the LDS that a kernel declares.
+constexpr uint32_t kIslandGroupRows = 8192;
 struct IslandLds {
     uint32_t parents[kIslandGroupRows];
-    uint32_t flags[kIslandGroupRows];
+    uint32_t woken[kIslandGroupRows / 32u];   // a bit per row: woken
+    uint32_t wakes[kIslandGroupRows / 32u];   // a bit per root: its island wakes
     uint32_t roots, woke;
+    static __device__ __forceinline__ bool get(const uint32_t* bits, uint32_t row) {
+        return (__hip_atomic_load(&bits[row / 32u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> (row % 32u)) & 1u;
+    }
+    static __device__ __forceinline__ void set(uint32_t* bits, uint32_t row) { atomicOr(&bits[row / 32u], 1u << (row % 32u)); }
     __device__ __forceinline__ uint32_t parent(uint32_t row) const {
         return __hip_atomic_load(&parents[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -1919,8 +1924,8 @@ __device__ inline void island_group_flatten(const W& w, IslandLds& l) {
 
 // island_couple on the rows in LDS.
 __device__ inline void island_group_couple(const W& w, IslandLds& l, uint32_t a, uint32_t b) {
-    if (b >= w.d && (l.flags[b] & kRowWoken)) atomicOr(&l.flags[a], kRowWoken);
-    if (a >= w.d && (l.flags[a] & kRowWoken)) atomicOr(&l.flags[b], kRowWoken);
+    if (b >= w.d && l.get(l.woken, b)) l.set(l.woken, a);
+    if (a >= w.d && l.get(l.woken, a)) l.set(l.woken, b);
     if (a >= w.d || b >= w.d || a == b) return;
     uint32_t ra = l.find(a), rb = l.find(b);
     for (uint32_t attempt = 0; attempt < 256u; ++attempt) {
@@ -1938,9 +1943,11 @@ __global__ void __launch_bounds__(1024) k_island_group(W w) {
     __shared__ IslandLds l;
     const uint32_t t = threadIdx.x;
     if (t == 0u) l.roots = l.woke = 0u;
+    for (uint32_t i = t; i < kIslandGroupRows / 32u; i += 1024u) l.woken[i] = l.wakes[i] = 0u;
+    __syncthreads();
     for (uint32_t i = t; i < w.n; i += 1024u) {
         if (i < w.d) l.parents[i] = w.parents[i];
-        l.flags[i] = w.wake[i] != 0u ? kRowWoken : 0u;
+        if (w.wake[i] != 0u) l.set(l.woken, i);
     }
     __syncthreads();
     island_group_flatten(w, l);
@@ -1961,14 +1968,14 @@ __global__ void __launch_bounds__(1024) k_island_group(W w) {
     for (uint32_t i = t; i < w.d; i += 1024u) {
         const uint32_t root = l.parents[i];
         roots += root == i ? 1u : 0u;
-        if ((l.flags[i] & kRowWoken) || w.motion[i] != 0u) atomicOr(&l.flags[root], kRowIslandWakes);
+        if ((l.get(l.woken, i) || w.motion[i] != 0u) && !l.get(l.wakes, root)) l.set(l.wakes, root);
     }
     __syncthreads();
     for (uint32_t i = t; i < w.d; i += 1024u) {
         const uint32_t root = l.parents[i];
         w.parents[i] = root;
-        w.istate[i] = l.flags[i] & kRowIslandWakes ? kIslandWake : 0u;
-        woke += island_wake_at(w, i, (l.flags[root] & kRowIslandWakes) != 0u);
+        w.istate[i] = l.get(l.wakes, i) ? kIslandWake : 0u;
+        woke += island_wake_at(w, i, l.get(l.wakes, root));
     }
     roots = wave_sum(roots);
     woke = wave_sum(woke);

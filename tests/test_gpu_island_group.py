@@ -1,4 +1,4 @@
-"""The step's island pass at the edge of its one-workgroup form (4,096 rows): chains of touching balls in
+"""The step's island pass at the edge of its one-workgroup form (8,192 rows): chains of touching balls in
 shuffled row order that fall asleep, and are woken at one end by a ball and by each other. Each step's
 islands, sleeps, wakes and resting contacts against the oracle's step."""
 
@@ -26,7 +26,7 @@ def chains(rows):
     return [BodyDesc.sphere(0.5, position=place[0]).fixed()] + [bodies[i] for i in order]
 
 
-@pytest.mark.parametrize("rows", [9, 1023, 4096, 4097])
+@pytest.mark.parametrize("rows", [9, 1023, 8192, 8193])
 def test_chains(device, oracle, rows):
     scene = encode(chains(rows), static_config())
     world, ref = World(), oracle.world(scene)
