@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb*
 
 // Workgroups up to which the emission also counts the sort's digits, saving a launch and a read of the
 // keys. Every workgroup adds its counts to the same 1,024 words, one atomic after another: at 2^20
-// boxes that made the emission 111 us, against 43 us and a 12 us pass over the keys without it.
+// boxes that made the emission 111 us, against 74 us and a 20 us pass over the keys without it.
 constexpr uint32_t kEmitHistogramBlocks = 128;
 
 // collider_emit.wgsl:6-63 with slots from the scan.
@@ -960,7 +960,9 @@ __global__ void __launch_bounds__(1024) bp_pair_offsets_kernel(uint32_t* link_bl
     const uint32_t mate_n = ceil_div(sort_ctl[kCtlLen], kBpThreads);  // blocks past the entries count nothing
     // Block totals per thread and round, moved sixteen bytes at a time: what one CU can do here is
     // bounded by the lines that its accesses touch (at 2^20 boxes 39 us with a word an access, now 12).
-    constexpr uint32_t kItems = 16;
+    // The arrays are padded to 256 bytes, so the last access needs no path of its own, whose code a
+    // small scene would wait for.
+    constexpr uint32_t kItems = 8;
     __shared__ uint32_t s_scan[1024 / kWave];
     __shared__ uint32_t s_carry;
     if (threadIdx.x == 0) s_carry = 0;
@@ -970,39 +972,27 @@ __global__ void __launch_bounds__(1024) bp_pair_offsets_kernel(uint32_t* link_bl
         for (uint32_t first = 0; first < count; first += 1024u * kItems) {
             __syncthreads();
             const uint32_t base = first + threadIdx.x * kItems;
-            uint32_t v[kItems];
+            uint32_t v[kItems] = {};
             uint32_t sum = 0;
-            const bool whole = base + kItems <= count;
             uint4* quads = reinterpret_cast<uint4*>(blocks + base);
 #pragma unroll
             for (uint32_t j = 0; j < kItems; j += 4u) {
-                uint4 q = make_uint4(0u, 0u, 0u, 0u);
-                if (whole) {
-                    q = quads[j / 4u];
-                } else {
-                    if (base + j < count) q.x = blocks[base + j];
-                    if (base + j + 1u < count) q.y = blocks[base + j + 1u];
-                    if (base + j + 2u < count) q.z = blocks[base + j + 2u];
-                    if (base + j + 3u < count) q.w = blocks[base + j + 3u];
-                }
+                if (base + j >= count) continue;
+                const uint4 q = quads[j / 4u];
                 v[j] = q.x;
-                v[j + 1u] = q.y;
-                v[j + 2u] = q.z;
-                v[j + 3u] = q.w;
-                sum += q.x + q.y + q.z + q.w;
+                v[j + 1u] = base + j + 1u < count ? q.y : 0u;
+                v[j + 2u] = base + j + 2u < count ? q.z : 0u;
+                v[j + 3u] = base + j + 3u < count ? q.w : 0u;
             }
+#pragma unroll
+            for (uint32_t j = 0; j < kItems; ++j) sum += v[j];
             uint32_t total = 0;
             uint32_t run = s_carry + block_exclusive_sum<1024>(sum, s_scan, &total);
 #pragma unroll
-            for (uint32_t j = 0; j < kItems; ++j) {
-                const uint32_t mine = v[j];
-                v[j] = run;
-                if (!whole && base + j < count) blocks[base + j] = run;
-                run += mine;
-            }
-            if (whole) {
-#pragma unroll
-                for (uint32_t j = 0; j < kItems; j += 4u) quads[j / 4u] = make_uint4(v[j], v[j + 1u], v[j + 2u], v[j + 3u]);
+            for (uint32_t j = 0; j < kItems; j += 4u) {
+                const uint4 at = make_uint4(run, run + v[j], run + v[j] + v[j + 1u], run + v[j] + v[j + 1u] + v[j + 2u]);
+                run = at.w + v[j + 3u];
+                if (base + j < count) quads[j / 4u] = at;
             }
             __syncthreads();
             if (threadIdx.x == 0) s_carry += total;

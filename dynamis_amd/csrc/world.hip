@@ -1786,7 +1786,8 @@ __global__ void __launch_bounds__(kThreads) k_island_flatten(W w, uint32_t* flag
     if (up != at) flags[round] = 1u;  // stopped short of the root
 }
 
-// All the flatten rounds of a small world in one workgroup, a barrier after each round (within a
+// All the flatten rounds of a few rows in one workgroup (dyn_islands: a step of as many rows takes
+// k_island_group), a barrier after each round (within a
 // round, as across the launched rounds, a row may read a parent another row has already moved
 // up, which only shortens its walk); it stops after the first round whose walks all reached
 // their roots.
