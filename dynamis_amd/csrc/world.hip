@@ -836,6 +836,10 @@ constexpr uint32_t kQuadPairs = kThreads / kQuad;  // pairs of a workgroup
 // GJK lists longer than this are run one thread a pair (convex.h says why): four lanes a pair then fill
 // the GPU many times over (2^17 pairs are 8,192 waves of quads, 8 a SIMD).
 constexpr uint32_t kLongGjk = 1u << 17;
+// The same for the lists of resumed pairs, whose quads stay longer below the vector units' bound: 70,560
+// pairs take 175 us by quads and 209 by threads, 94,080 210 and 217, 141,120 282 and 247 (a settled
+// 100k pile's 157,257: 398 and 283).
+constexpr uint32_t kLongResume = 3u << 15;
 
 template <typename Pair>
 struct ConvexPair {
@@ -955,19 +959,28 @@ __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w) {
     lists.finish(open ? 0u : kNoList, index, false, nullptr, {{&w.work_total[kTotalResume], w.worklist, 0u}});
 }
 
-// The remaining GJK iterations of the pairs k_narrow_convex parked, a quad per pair, from their parked
-// state, then the rest of convex_hit as in k_narrow_convex.
-__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
-    const uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) / kQuad, q = threadIdx.x % kQuad;
-    if (t >= w.work_total[kTotalResume]) return;
-    const uint32_t index = w.worklist[t];
-    const ConvexPair<QuadPair> c = load_quad_pair(w, index, q);
+// A pair's remaining GJK iterations from its parked state, then the rest of convex_hit.
+template <typename Pair>
+__device__ inline void resume_convex_pair(const W& w, const ConvexPair<Pair>& c, uint32_t q) {
     const ShapeSet shapes{w.sources, w.vertices, w.support_cells, w.support_cands};
     GjkState g;
-    unpark_gjk(parked(w, index), &g);
+    unpark_gjk(parked(w, c.index), &g);
     Closest closest;
     gjk_run(c.shapes, shapes, &g, kGjkIterations, &closest);
     convex_pair_after_gjk(w, c, q, shapes, closest, g);
+}
+
+// The remaining GJK iterations of the pairs k_narrow_convex parked, then the rest of convex_hit as in
+// k_narrow_convex: a quad per pair or (in a list longer than kLongResume) a thread.
+__global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
+    const uint32_t total = w.work_total[kTotalResume];
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (total > kLongResume) {
+        if (t < total) resume_convex_pair(w, load_thread_pair(w, w.worklist[t]), kWholePair);
+        return;
+    }
+    const uint32_t pair = t / kQuad, q = t % kQuad;
+    if (pair < total) resume_convex_pair(w, load_quad_pair(w, w.worklist[pair], q), q);
 }
 
 // After GJK: its penetrating pairs to the front of worklist, its hits to the end.

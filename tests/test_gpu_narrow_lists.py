@@ -1,7 +1,7 @@
 """The narrowphase's pair lists and its two kinds of GJK at their edges: pair capacities on both sides of
-the one-workgroup grouping, and a list long enough for one thread a pair (above 131,072 GJK pairs). The
-same pairs repeated give the same contacts in every copy, and the first copy is held to the oracle by
-the stage's own tests."""
+the one-workgroup grouping, and lists long enough for one thread a pair (above 131,072 GJK pairs, above
+98,304 resumed ones). The same pairs repeated give the same contacts in every copy, and the first copy is
+held to the oracle by the stage's own tests."""
 
 from __future__ import annotations
 
@@ -16,13 +16,23 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
-def pile(device):
+def settled(device):
     scene = pile_scene(3000, seed=5, hull_sources=64, spacing=1.5)
     with World() as world:
         world.create(scene)
         for _ in range(60):
             world.step(DT)
-        return with_states(scene, world.states()), world.pairs()
+        return with_states(scene, world.states()), world.pairs(), world.convex_work()
+
+
+@pytest.fixture(scope="module")
+def pile(settled):
+    return settled[:2]
+
+
+@pytest.fixture(scope="module")
+def work(settled):
+    return settled[2]
 
 
 def run(scene, pairs, capacity):
@@ -44,12 +54,21 @@ def test_capacities(pile, count, capacity):
     assert raw[hit].tobytes() == want_raw[hit].tobytes()
 
 
-def test_long_list(pile):
+# the lists' limits, and a quarter more for what moved since the step whose lists are counted
+LONG_GJK, LONG_RESUME, MARGIN = 1 << 17, 3 << 15, 1.25
+
+
+@pytest.mark.parametrize("long_resume", [False, True])
+def test_long_list(pile, work, long_resume):
+    """GJK by a thread a pair, its open pairs resumed by quads, and both by threads."""
     scene, pairs = pile
+    copies = 1 + int(MARGIN * max(LONG_GJK / work["gjk"], long_resume * LONG_RESUME / work["gjk_resumed"]))
+    assert MARGIN * work["gjk"] < LONG_GJK < copies * work["gjk"] / MARGIN * 1.01
+    assert (copies * work["gjk_resumed"] > LONG_RESUME * MARGIN) == long_resume
+    assert long_resume or copies * work["gjk_resumed"] * MARGIN < LONG_RESUME
     want_raw, want_valid = run(scene, pairs, len(pairs))
     hit = want_valid == 1
     assert hit.sum() > 1000
-    copies = 1 + 700000 // len(pairs)  # about a third of the pairs go to GJK
     raw, valid = run(scene, np.tile(pairs, (copies, 1)), copies * len(pairs))
     for c in range(copies):
         part = slice(c * len(pairs), (c + 1) * len(pairs))
