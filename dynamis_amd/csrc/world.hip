@@ -499,18 +499,19 @@ __device__ __forceinline__ bool bounds_apart(const Shape& a, const Shape& b, con
 // of a 755 us pass over 114,000 pairs). Two arrays of pair_cap words hold them all: no pair is on two
 // lists that share an array at one time.
 
-// Words of work_total. kTotalGjk to kTotalEpaWave are also what dyn_world_read_work reports (the
-// second as all manifold pairs).
+// Words of work_total, on two cache lines: a line takes in one atomic after another, about 12 ns each, so
+// the counters that a kernel's workgroups add to together lie on both (k_work_split of 919,000 pairs 28 us
+// with one line, 22 with two; a line for each counter 20).
 enum WorkTotal : uint32_t {
     kTotalGjk = 0,      // work_minor, front
-    kTotalPlane = 1,    // work_minor, from the end
-    kTotalEpa = 2,      // worklist, front
-    kTotalHull = 3,     // GJK pairs of the hull classes
-    kTotalResume = 4,   // worklist, front (until k_work_split)
-    kTotalEpaWave = 5,  // work_minor, front (after k_work_split)
-    kTotalAll = 6,      // worklist (until k_narrow has read it)
-    kTotalHit = 7,      // worklist, from the end
-    kTotalWords = 8
+    kTotalEpa = 1,      // worklist, front
+    kTotalResume = 2,   // worklist, front (until k_work_split)
+    kTotalEpaWave = 3,  // work_minor, front (after k_work_split)
+    kTotalAll = 4,      // worklist (until k_narrow has read it)
+    kTotalPlane = 32,   // work_minor, from the end
+    kTotalHull = 33,    // GJK pairs of the hull classes
+    kTotalHit = 34,     // worklist, from the end
+    kTotalWords = 64
 };
 constexpr uint32_t kNoList = 0xFFFFFFFFu;
 
@@ -520,11 +521,12 @@ struct ListTarget {
     uint32_t end;  // non-zero: entries go down from list[end - 1]
 };
 
-// A workgroup's takers for kLists lists, appended by the last of its waves to arrive (no wave waits).
-template <uint32_t kLists>
+// The takers of a workgroup of kBlock lanes for kLists lists, appended by the last of its waves to
+// arrive (no wave waits).
+template <uint32_t kLists, uint32_t kBlock>
 struct BlockLists {
     uint32_t n[kLists], arrived, hull;
-    uint32_t item[kLists][kThreads];
+    uint32_t item[kLists][kBlock];
 
     __device__ __forceinline__ void begin() {
         if (threadIdx.x < kLists) n[threadIdx.x] = 0u;
@@ -549,7 +551,7 @@ struct BlockLists {
         __threadfence_block();
         uint32_t before = 0;
         if (lane == 0u) before = atomicAdd(&arrived, 1u);
-        if (__builtin_amdgcn_readfirstlane(before) + 1u != kThreads / kWave) return;
+        if (__builtin_amdgcn_readfirstlane(before) + 1u != kBlock / kWave) return;
         __threadfence_block();
 #pragma unroll
         for (uint32_t k = 0; k < kLists; ++k) {
@@ -753,7 +755,7 @@ __device__ __forceinline__ uint32_t narrow_pair(const W& w, uint32_t index) {
 // One thread per candidate pair of the kind-grouped list (every pair's result goes to its own slot,
 // so the order changes nothing).
 __global__ void __launch_bounds__(kThreads) k_narrow(W w) {
-    __shared__ BlockLists<2> lists;
+    __shared__ BlockLists<2, kThreads> lists;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t total = w.work_total[kTotalAll];
     if (blockIdx.x * blockDim.x >= total) return;
@@ -934,7 +936,7 @@ __device__ inline bool narrow_convex_pair(const W& w, const ConvexPair<Pair>& c,
 // wave hides more of its latency than the spills cost (708 -> 627 us on a settled 100k pile; four
 // waves, 128 registers, were slower).
 __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex(W w) {
-    __shared__ BlockLists<1> lists;
+    __shared__ BlockLists<1, kThreads> lists;
     const uint32_t total = w.work_total[kTotalGjk];
     const bool quads = total <= kLongGjk;
     if (blockIdx.x * (quads ? kQuadPairs : kThreads) >= total) return;
@@ -983,9 +985,12 @@ __global__ void __launch_bounds__(kThreads, 3) k_narrow_convex_resume(W w) {
     if (pair < total) resume_convex_pair(w, load_quad_pair(w, w.worklist[pair], q), q);
 }
 
-// After GJK: its penetrating pairs to the front of worklist, its hits to the end.
-__global__ void __launch_bounds__(kThreads) k_work_split(W w) {
-    __shared__ BlockLists<2> lists;
+// After GJK: its penetrating pairs to the front of worklist, its hits to the end. What bounds it is the
+// workgroups' atomics on the two lengths, so workgroups are the largest: 919,000 pairs take 67 us in
+// workgroups of 256 (89 with both lengths on one line) and 22 in those of 1,024.
+constexpr uint32_t kSplitThreads = 1024;
+__global__ void __launch_bounds__(kSplitThreads) k_work_split(W w) {
+    __shared__ BlockLists<2, kSplitThreads> lists;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t total = w.work_total[kTotalGjk];
     if (blockIdx.x * blockDim.x >= total) return;
@@ -3537,7 +3542,11 @@ int narrowphase(const dyn::W& w, hipStream_t st, bool convex, const SideStream* 
     const uint32_t qb = ceil_div(static_cast<uint64_t>(w.pair_cap ? w.pair_cap : 1u) * kQuad, kThreads);
     LAUNCH_ON(st, k_narrow_convex, qb, w);
     LAUNCH_ON(st, k_narrow_convex_resume, qb, w);
-    LAUNCH_ON(st, k_work_split, pb, w);
+    {
+        ProfileScope scope("k_work_split", st);
+        k_work_split<<<ceil_div(w.pair_cap ? w.pair_cap : 1u, kSplitThreads), kSplitThreads, 0, st>>>(w);
+    }
+    DYN_LAUNCHED("k_work_split");
     {
         constexpr uint32_t kPairsPerBlock = kEpaWaves * kWave / kEpaGroup;
         const uint32_t small_groups = min(ceil_div(w.pair_cap ? w.pair_cap : 1u, kPairsPerBlock), 2048u);
@@ -4312,9 +4321,13 @@ int dyn_world_read_work(dyn_world* world, uint32_t* out) {
     DYN_HIP(hipStreamSynchronize(world->stream));
     uint32_t totals[dyn::kTotalWords];
     DYN_HIP(hipMemcpy(totals, world->w.work_total, sizeof totals, hipMemcpyDeviceToHost));
-    std::copy(totals, totals + 6, out);
+    out[0] = totals[dyn::kTotalGjk];
     // the manifold kernel's pairs: the planes', the hits, and the polytopes not given a wave
     out[1] = totals[dyn::kTotalPlane] + totals[dyn::kTotalHit] + totals[dyn::kTotalEpa] - totals[dyn::kTotalEpaWave];
+    out[2] = totals[dyn::kTotalEpa];
+    out[3] = totals[dyn::kTotalHull];
+    out[4] = totals[dyn::kTotalResume];
+    out[5] = totals[dyn::kTotalEpaWave];
     return DYN_OK;
 }
 

@@ -8,6 +8,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from dynamis_amd import abi
 from dynamis_amd.narrowphase import Narrowphase
 from dynamis_amd.world import World
 from tests.narrow_cases import DT, pile_scene, with_states
@@ -52,6 +53,20 @@ def test_capacities(pile, count, capacity):
     assert np.array_equal(valid, want_valid)
     hit = valid == 1
     assert raw[hit].tobytes() == want_raw[hit].tobytes()
+
+
+@pytest.mark.parametrize("count", [1, 1023, 1024, 1025, 2049])
+def test_split_edges(pile, count):
+    """GJK lists of just as many pairs (touching ones with a hull or a cylinder and no plane) around the
+    workgroups of 1,024 that split them into the penetrating pairs and the hits."""
+    scene, pairs = pile
+    raw, valid = run(scene, pairs, len(pairs))
+    kinds = scene.colliders["kind"][pairs]
+    gjk = np.isin(kinds, (abi.SHAPE_HULL, abi.SHAPE_CYLINDER)).any(axis=1) & (kinds != abi.SHAPE_PLANE).all(axis=1)
+    chosen = np.resize(np.flatnonzero(gjk & (valid == 1)), count)
+    got_raw, got_valid = run(scene, pairs[chosen], 4096)
+    assert (got_valid == 1).all()
+    assert got_raw.tobytes() == raw[chosen].tobytes()
 
 
 # the lists' limits, and a quarter more for what moved since the step whose lists are counted
