@@ -3666,10 +3666,29 @@ int solver_prepare(const dyn::W& w, hipStream_t st) {
 // Rows a workgroup of k_group_solve and k_group_position can hold: 64 bytes of LDS each.
 constexpr uint32_t kGroupRowLimit = 2304;
 // Worlds of at most this many rows are solved whole by a workgroup: one CU's share of the velocity
-// iterations then takes no longer than launching them (a lane a block: 5 us an iteration at 33 contacts,
-// 35 us at 2,664, against about 12 us launched; quads cut both by some 40%). Larger ones, up to the limit above, run only their position
-// iterations so (103 us for 20 of them at 2,664 contacts, against 5 us a launch and two each).
+// iterations then takes no longer than launching them. A step of one world of 120 bodies (148 contacts, 8
+// iterations) takes 284 us so and 316 with launched velocity iterations, of 160 (221 contacts) 335 and 333,
+// of 200 370 and 360, of 300 528 and 395. Larger worlds, up to the limit above, run only their position
+// iterations so.
 constexpr uint32_t kGroupWholeRows = 160;
+// Up to this many worlds: 512 of the workgroups (256 of those above 64 rows) are resident at once, and
+// every further round of them adds its whole latency. A step of 1,024 worlds of 8 bodies takes 588 us whole
+// and 652 with launched velocity iterations, 2,048 767 and 714, 4,096 1,139 and 879; 1,024 worlds of 100
+// bodies 1,500 and 1,526, 4,096 4,641 and 4,309.
+constexpr uint32_t kGroupWholeWorlds = 1024;
+
+// Whether k_group_position, a workgroup a world, beats the launched position iterations: `count` worlds
+// of `rows` rows in all, the largest of `largest`. In ns a substep of ten iterations: the launched ones
+// take 50,000 and 0.72 a row; a workgroup takes 34 a row of its world, and its share of the chip is 21
+// where it has 256 lanes and 62 where it has 1,024 (one a CU), however few rows its world has. A step by
+// k_group_position and by launches, in us: one world of 1,400 bodies 602 and 618, of 1,600 635 and 627, of
+// 2,300 718 and 662, 16 of 2,300 1,318 and 1,324; 2,048 worlds of 8 715 and 747, 4,096 878 and 832, 10,000
+// 1,368 and 1,083; 4,096 of 32 1,662 and 1,728; 2,000 of 100 beside one of 2,300 2,722 and 2,825, 10,000 of 8
+// beside it 2,276 and 1,248; 4,096 of 8 to 2,048 12,060 and 13,523.
+bool group_position_pays(uint32_t count, uint32_t largest, uint32_t rows) {
+    const double group = std::max(34.0 * largest, count * (largest <= 256u ? 21.0 : 62.0));
+    return group <= 50000.0 + 0.72 * rows;
+}
 
 template <typename Kernel, typename... Args>
 int group_launch(const char* name, Kernel kernel, uint32_t threads, hipStream_t st, const GroupPlan& g, Args... args) {
@@ -3704,7 +3723,7 @@ int group_position(const dyn::W& w, hipStream_t st, const GroupPlan& g, uint32_t
 // The plan of one world of n rows.
 GroupPlan plan_group(uint32_t n) {
     GroupPlan plan;
-    if (n && n <= kGroupRowLimit) {
+    if (n && n <= kGroupRowLimit && group_position_pays(1u, n, n)) {
         plan.count = 1u;
         plan.rows = n;
         plan.whole = n <= kGroupWholeRows;
@@ -3765,8 +3784,8 @@ int solver(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint32_t thre
 }
 
 // The plan of a batch: every world's colliders, simulated rows and other rows must each be one run
-// (as merge_scenes lays them out) and every row must belong to a world of at most kGroupRowLimit
-// rows; otherwise no launches, and the batch is solved by the launched passes.
+// (as merge_scenes lays them out), every row must belong to a world of at most kGroupRowLimit rows, and
+// the worlds must be few or large enough (group_position_pays); otherwise the batch is solved by the launched passes.
 void plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t colliders,
                  const std::vector<uint32_t>& world_of_row, uint32_t worlds) {
     using namespace dyn;
@@ -3795,15 +3814,19 @@ void plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t col
     }
     auto rows = [](const GroupWorld& g) { return g.dynamic_count + g.static_count; };
     std::stable_sort(order.begin(), order.end(), [&](const GroupWorld& a, const GroupWorld& b) { return rows(a) > rows(b); });
+    if (order.empty()) return;
+    GroupPlan plan;
+    plan.count = static_cast<uint32_t>(order.size());
+    plan.rows = rows(order[0]);
+    plan.whole = plan.rows <= kGroupWholeRows && plan.count <= kGroupWholeWorlds;
+    if (!plan.whole && !group_position_pays(plan.count, plan.rows, w.n)) return;
     GroupWorld* device = nullptr;
-    if (order.empty() || alloc(world, &device, order.size()) != DYN_OK ||
+    if (alloc(world, &device, order.size()) != DYN_OK ||
         hipMemcpy(device, order.data(), sizeof(GroupWorld) * order.size(), hipMemcpyHostToDevice) != hipSuccess) {
         return;
     }
-    world->groups.worlds = device;
-    world->groups.count = static_cast<uint32_t>(order.size());
-    world->groups.rows = rows(order[0]);
-    world->groups.whole = rows(order[0]) <= kGroupWholeRows;
+    plan.worlds = device;
+    world->groups = plan;
 }
 
 void drop_graph(dyn_world* world) {
