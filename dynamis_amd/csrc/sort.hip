@@ -553,10 +553,11 @@ static int launch_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, u
 // ---- tiling: the autotuner's table ---------------------------------------------------------------
 //
 // A pass's tiling is keys per lane (8: 4096-key tiles; 16: 8192-key tiles, for streams with enough live
-// records) and the cap on its persistent workgroups. The tuner times every candidate on the device for a capacity bucket
-// (ceil(log2(capacity))) and keeps the fastest per (device, bucket); untuned buckets use the
-// default: narrow tiles up to 2^21 keys (more of the chip busy on shorter streams), 1024 groups
-// (about four per CU).
+// records) and the cap on its persistent workgroups. The tuner times the candidates on the device for a
+// capacity bucket (ceil(log2(capacity))) and keeps the fastest per (device, bucket); 16 keys a lane only
+// above kNarrowBelow, where they differ from 8, and nothing up to kSortSmall, where no pass runs. Untuned
+// buckets use the default: narrow tiles up to 2^21 keys (more of the chip busy on shorter streams), 1024
+// groups (about four per CU).
 
 struct SortTiling {
     uint32_t items, groups;
@@ -669,6 +670,12 @@ int dyn_sort_autotune(void* stream, uint32_t capacity, uint32_t digit_passes, ui
     if (digit_passes == 0u || digit_passes > kSortMaxPasses) {
         return fail(DYN_E_INVALID, "dyn_sort_autotune: digit_passes must be 1..8");
     }
+    if (capacity <= kSortSmall) {  // sorted by one workgroup, which has no tiling
+        const SortTiling t = default_tiling(capacity);
+        if (items_out) *items_out = t.items;
+        if (groups_out) *groups_out = t.groups;
+        return DYN_OK;
+    }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const size_t scratch_bytes = sort_scratch_layout(capacity, digit_passes, true, nullptr, nullptr);
     std::vector<void*> owned;
@@ -699,6 +706,7 @@ int dyn_sort_autotune(void* stream, uint32_t capacity, uint32_t digit_passes, ui
     int rc = DYN_OK;
     for (uint32_t round = 0; round < 4 && rc == DYN_OK; ++round) {  // round 0 warms every variant
         for (uint32_t c = 0; c < kTilingCount && rc == DYN_OK; ++c) {
+            if (kTilings[c].items > 8u && capacity <= kNarrowBelow) continue;  // it runs 8 keys a lane too
             sort_tune_fill<<<ceil_div(capacity, 256u), 256, 0, st>>>(lanes[0], lanes[1], lanes[2], capacity, round);
             rc = sort_prepare(st, s, nullptr, nullptr, capacity, names);
             if (rc == DYN_OK) rc = sort_histogram(st, lanes[0], lanes[1], s, digits, digit_passes, capacity, names);

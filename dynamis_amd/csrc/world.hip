@@ -4779,8 +4779,8 @@ int dyn_world_autotune(dyn_world* world, uint32_t* tilings) {
     using namespace dyn;
     if (!world) return fail(DYN_E_INVALID, "dyn_world_autotune: null world");
     const W& w = world->w;
-    // the step's sorts: entry regions (4 key digits), candidate pairs and GJK worklists (pair
-    // capacity), the resting index (contact capacity)
+    // the step's sorts: entry regions (4 key digits), candidate pairs (pair capacity), the resting
+    // index (contact capacity)
     const uint32_t caps[3] = {world->entry_cap, w.pair_cap, w.contact_cap};
     const uint32_t passes[3] = {4u, 2u * dyn_sort_key_words(w.k ? w.k : 1u), 2u * dyn_sort_key_words(w.id_cap ? w.id_cap : 1u)};
     DYN_HIP(hipStreamSynchronize(world->stream));

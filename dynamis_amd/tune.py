@@ -2,7 +2,7 @@
 
 The library chooses each sort pass's tiling (keys per lane, persistent workgroups) from a
 process-wide table keyed by device and capacity bucket (ceil(log2(capacity))); `dyn_sort_autotune`
-fills an entry by timing every tiling on the device. `autotune_world` tunes the capacities of a
+fills an entry by timing the tilings on the device. `autotune_world` tunes the capacities of a
 world's sorts and keeps the table in a JSON file per GPU name, so later runs on the same kind of
 GPU load it instead of timing again. Every tiling sorts to the same stable order: tuning changes
 time, never results.
@@ -21,6 +21,8 @@ import numpy as np
 from ._native import call
 
 MAX_CELLS_PER_COLLIDER = 8  # entries per collider: the world's entry-sort capacity factor
+SORT_SMALL = 8192  # capacities up to this are sorted by one workgroup: no tiling, none in the table
+DEFAULT_TILING = (8, 1024)  # what dyn_sort_autotune returns for them
 
 
 def device_name() -> str:
@@ -91,13 +93,14 @@ def autotune_world(world, directory: str | os.PathLike | None = None, retune: bo
         data = json.loads(path.read_text())
         if data.get("device") == device_name():
             cached = np.array(data["entries"], np.uint32).reshape(-1, 4)
-    if cached is not None and {bucket(c) for c in caps} <= set(int(b) for b in cached[:, 1]):
+    if cached is not None and {bucket(c) for c in caps if c > SORT_SMALL} <= set(int(b) for b in cached[:, 1]):
         rows = {(int(r[0]), int(r[1])): r for r in table()}
         for r in cached:
             rows[(int(r[0]), int(r[1]))] = r
         load(np.array(list(rows.values()), np.uint32))
         world.set_graphs(True)  # drops the captured step
-        chosen = {c: tuple(int(v) for v in cached[cached[:, 1] == bucket(c)][0, 2:4]) for c in caps}
+        chosen = {c: tuple(int(v) for v in cached[cached[:, 1] == bucket(c)][0, 2:4]) if c > SORT_SMALL
+                  else DEFAULT_TILING for c in caps}
         return {"tilings": chosen, "from_cache": True, "cache": str(path)}
     out = np.zeros(9, np.uint32)
     call("dyn_world_autotune", world._handle, out.ctypes.data)

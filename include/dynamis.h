@@ -505,13 +505,16 @@ int dyn_fixed_grid(void* stream, const dyn_aabb* d_boxes, uint32_t boxes, float 
 /* ---- autotuning (no reference counterpart: the reference's sort has one fixed tiling) ----
  * A sort pass's tiling (keys per lane 8 or 16, cap on persistent workgroups 512/1024/2048) is
  * chosen per (device, ceil(log2(capacity))) from a process-wide table; untuned buckets use the
- * default. dyn_sort_autotune times every tiling on the device for `capacity` keys and
+ * default. dyn_sort_autotune times the tilings on the device for `capacity` keys and
  * `digit_passes` digits (synthetic keys, minimum of three rounds after a warm round) and keeps the
- * fastest; dyn_world_autotune does so for the capacities of a world's sorts (entries, pairs and
- * worklists, the resting index) and drops its captured step; tilings (optional, 9 words) receives
- * capacity, keys per lane, groups for each. The table is exported and imported as 4 words per
- * entry (device, bucket, keys per lane, groups) so a caller can keep it per GPU. Every tiling
- * sorts to the same stable order. */
+ * fastest. Streams of up to 1,572,864 live records run 8 keys per lane whatever the table holds, so
+ * capacities up to that time only those; capacities up to 8,192 are sorted by one workgroup, which
+ * has no tiling: for them it times and records nothing and returns the default.
+ * dyn_world_autotune does so for the capacities of a world's sorts (entries, pairs, the resting
+ * index) and drops its captured step; tilings (optional, 9 words) receives capacity, keys per
+ * lane, groups for each. The table is exported and imported as 4 words per entry (device, bucket,
+ * keys per lane, groups) so a caller can keep it per GPU. Every tiling sorts to the same stable
+ * order. */
 int dyn_sort_autotune(void* stream, uint32_t capacity, uint32_t digit_passes, uint32_t* items_out,
                       uint32_t* groups_out);
 int dyn_sort_tuning_export(uint32_t* out, uint32_t capacity, uint32_t* count);

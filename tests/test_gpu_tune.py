@@ -3,10 +3,13 @@ world whose sorts were tuned steps bit for bit as an untuned one; the per-GPU ca
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 from dynamis_amd import scenes, tune
+from dynamis_amd._native import call
 from dynamis_amd.sort import RadixSort, SortChannels, units_for
 from dynamis_amd.world import World, encode
 from tests.sort_cases import expected_order, xorshift
@@ -50,6 +53,35 @@ def test_autotuned_world_steps_identically(device, tmp_path):
         again, info2 = run(True)
         assert info2["from_cache"] and info2["tilings"] == info["tilings"]
         assert again.tobytes() == plain.tobytes()
+    finally:
+        tune.load(np.zeros((0, 4), np.uint32))
+
+
+def autotune(capacity):
+    items, groups = ctypes.c_uint32(), ctypes.c_uint32()
+    call("dyn_sort_autotune", None, capacity, 2, ctypes.byref(items), ctypes.byref(groups))
+    return items.value, groups.value
+
+
+def test_tuner_times_what_is_run(device, tmp_path):
+    """Capacities that one workgroup sorts have no tiling and leave no entry; those whose streams are
+    always short enough for 8 keys a lane are not given 16; a world of such sorts only is cached."""
+    try:
+        tune.load(np.zeros((0, 4), np.uint32))
+        assert autotune(1) == autotune(tune.SORT_SMALL) == tune.DEFAULT_TILING
+        assert len(tune.table()) == 0
+        for capacity in (tune.SORT_SMALL + 1, 40_000, 150_000, 300_000, 600_000, 1_200_000, 1_572_864):
+            assert autotune(capacity)[0] == 8
+            assert tune.bucket(capacity) in tune.table()[:, 1]
+        tune.load(np.zeros((0, 4), np.uint32))
+        with World() as world:
+            world.create(encode(scenes.cube_drop(100, seed=3)))
+            assert world.pair_capacity <= tune.SORT_SMALL
+            first = tune.autotune_world(world, tmp_path)
+            again = tune.autotune_world(world, tmp_path)
+        assert set(first["tilings"].values()) == {tune.DEFAULT_TILING}
+        assert again["from_cache"] and again["tilings"] == first["tilings"]
+        assert len(tune.table()) == 0
     finally:
         tune.load(np.zeros((0, 4), np.uint32))
 
