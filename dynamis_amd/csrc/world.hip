@@ -4397,6 +4397,11 @@ int dyn_world_tune_solver(dyn_world* world, uint32_t steps, uint32_t* threads_ou
     if (world->hull_colliders && world->shape_sources == nullptr) {
         return fail(DYN_E_INVALID, "dyn_world_tune_solver: hull colliders need dyn_world_upload_shapes first");
     }
+    if (world->groups.whole) {  // k_group_solve: no workgroup size to choose
+        if (threads_out) *threads_out = world->solver_threads;
+        for (uint32_t i = 0; ms_out && i < 3u; ++i) ms_out[i] = 0.0f;
+        return DYN_OK;
+    }
     if (steps == 0u) steps = 3u;
     const float dt = world->last_dt > 0.0f ? world->last_dt : 1.0f / 60.0f;
     size_t bytes = 0;

@@ -58,7 +58,8 @@ def cache_path(directory: str | os.PathLike | None = None) -> pathlib.Path:
 def autotune_solver(world, directory: str | os.PathLike | None = None, retune: bool = False,
                     steps: int = 3) -> dict:
     """Tunes (or loads from the per-GPU cache, keyed by the contact capacity's bucket) the
-    workgroup size of a world's solver substeps; the world's state is left as it was."""
+    workgroup size of a world's solver substeps; the world's state is left as it was. A world
+    that is solved whole by a workgroup has no such size: nothing is timed or cached."""
     if hasattr(world, "_ensure"):
         world._ensure()
     path = cache_path(directory).with_name(cache_path(directory).name.replace("sort-tilings-", "solver-threads-"))
@@ -73,9 +74,10 @@ def autotune_solver(world, directory: str | os.PathLike | None = None, retune: b
         world.set_solver_threads(int(sizes[key]))
         return {"threads": int(sizes[key]), "from_cache": True, "cache": str(path)}
     threads, ms = world.tune_solver(steps)
-    sizes[key] = threads
-    path.parent.mkdir(parents=True, exist_ok=True)
-    path.write_text(json.dumps({"device": device_name(), "threads": sizes}))
+    if any(ms):
+        sizes[key] = threads
+        path.parent.mkdir(parents=True, exist_ok=True)
+        path.write_text(json.dumps({"device": device_name(), "threads": sizes}))
     return {"threads": threads, "ms_per_step": {"64": ms[0], "128": ms[1], "256": ms[2]}, "from_cache": False,
             "cache": str(path)}
 

@@ -388,7 +388,8 @@ class World(BodyCommands):
 
     def tune_solver(self, steps: int = 3) -> tuple[int, list[float]]:
         """Times the solver's workgroup sizes on this world's next steps (from a snapshot, then
-        restored) and keeps the fastest: (size, ms per step of 64, 128, 256)."""
+        restored) and keeps the fastest: (size, ms per step of 64, 128, 256). A world solved
+        whole by a workgroup has none to choose: (its size, zeros)."""
         self._ensure()
         threads = ctypes.c_uint32()
         ms = (ctypes.c_float * 3)()

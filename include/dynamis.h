@@ -466,7 +466,9 @@ int dyn_world_wait(dyn_world* world);
  * steps (3 when 0) of the world with each size from a snapshot of its current state (at the last
  * step's dt), keeps the fastest, restores the state, and returns the size and the three
  * milliseconds-per-step (either pointer may be NULL); it records no capacity demand, allocates a
- * snapshot buffer while it runs, and fails while edits are queued or a tape is recorded. */
+ * snapshot buffer while it runs, and fails while edits are queued or a tape is recorded. Worlds small
+ * enough to be solved whole by a workgroup launch none of these kernels: for them it times nothing,
+ * keeps the size and returns zeros for the milliseconds. */
 int dyn_world_set_solver_threads(dyn_world* world, uint32_t threads);
 int dyn_world_tune_solver(dyn_world* world, uint32_t steps, uint32_t* threads_out, float* ms_out);
 /* Capacity planning (World::apply_plan, crates/dynamis-world/src/backend/mod.rs:194-230, with the

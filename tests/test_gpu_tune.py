@@ -127,3 +127,18 @@ def test_solver_tuning_leaves_the_world_unchanged(device):
     assert tuned.inspect_contacts().tobytes() == plain.inspect_contacts().tobytes()
     plain.close()
     tuned.close()
+
+
+def test_solver_tuning_of_a_world_solved_whole(device, tmp_path):
+    """No workgroup size is used there: nothing is timed, and no size is cached for larger worlds."""
+    with World() as world:
+        world.create(encode(scenes.cube_drop(100, seed=5)))
+        for _ in range(40):
+            world.step(1 / 60)
+        world.set_solver_threads(128)
+        before = world.states().copy()
+        assert world.tune_solver(3) == (128, [0.0, 0.0, 0.0])
+        info = tune.autotune_solver(world, tmp_path)
+        assert info["threads"] == 128 and not info["from_cache"]
+        assert list(tmp_path.iterdir()) == []
+        assert world.states().tobytes() == before.tobytes()
