@@ -3694,9 +3694,9 @@ template <typename Kernel, typename... Args>
 int group_launch(const char* name, Kernel kernel, uint32_t threads, hipStream_t st, const GroupPlan& g, Args... args) {
     using namespace dyn;
     const uint32_t lds = g.rows * kGroupRowWords * 4u;
-    if (lds > 60u * 1024u) {
+    if (lds > 60u * 1024u) {  // the most that any world asks for: other threads launch other worlds
         DYN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    static_cast<int>(lds)));
+                                    static_cast<int>(kGroupRowLimit * kGroupRowWords * 4u)));
     }
     {
         ProfileScope scope(name, st);

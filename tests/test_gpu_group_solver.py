@@ -6,6 +6,7 @@ oracle's solver, and each world of a batch against itself alone."""
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -113,6 +114,29 @@ def test_many_worlds(device, parts, solve, position):
                 assert batch.world_states(at, states).tobytes() == alone.tobytes(), at
         first += count
     batch.close()
+
+
+def test_sizes_side_by_side(device):
+    """Worlds whose workgroups ask for different amounts of LDS, launched from two threads at once."""
+    scenes = [encode(cube_drop(n, seed=n, footprint=0.5 * n ** 0.5, low=1.0, high=3.0), config()) for n in (1000, 1500)]
+
+    def steps(scene, out, key):
+        with World() as world:
+            world.create(scene)
+            world.set_graphs(False)
+            for _ in range(60):
+                world.step(DT)
+            out[key] = world.states().tobytes()
+
+    alone, beside = {}, {}
+    for i, scene in enumerate(scenes):
+        steps(scene, alone, i)
+    threads = [threading.Thread(target=steps, args=(scene, beside, i)) for i, scene in enumerate(scenes)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert beside == alone
 
 
 def test_batch_of_scattered_colliders(device):
