@@ -3785,13 +3785,14 @@ int solver(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint32_t thre
 
 // The plan of a batch: every world's colliders, simulated rows and other rows must each be one run
 // (as merge_scenes lays them out), every row must belong to a world of at most kGroupRowLimit rows, and
-// the worlds must be few or large enough (group_position_pays); otherwise the batch is solved by the launched passes.
-void plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t colliders,
-                 const std::vector<uint32_t>& world_of_row, uint32_t worlds) {
+// the worlds must be few or large enough (group_position_pays); otherwise there is none, and the batch
+// is solved by the launched passes.
+int plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t colliders,
+                const std::vector<uint32_t>& world_of_row, uint32_t worlds) {
     using namespace dyn;
     const W& w = world->w;
     for (uint32_t i = 1; i < colliders; ++i) {
-        if (collider_worlds[i] < collider_worlds[i - 1]) return;
+        if (collider_worlds[i] < collider_worlds[i - 1]) return DYN_OK;
     }
     std::vector<GroupWorld> table(worlds, GroupWorld{});
     for (uint32_t i = 0; i < colliders; ++i) {
@@ -3799,34 +3800,35 @@ void plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t col
         if (g.collider_count++ == 0u) g.collider_base = i;
     }
     for (uint32_t row = 0; row < w.n; ++row) {
-        if (world_of_row[row] == DYN_NO_BODY) return;
+        if (world_of_row[row] == DYN_NO_BODY) return DYN_OK;
         GroupWorld& g = table[world_of_row[row]];
         uint32_t& base = row < w.d ? g.dynamic_base : g.static_base;
         uint32_t& count = row < w.d ? g.dynamic_count : g.static_count;
         if (count == 0u) base = row;
-        if (row != base + count) return;
+        if (row != base + count) return DYN_OK;
         ++count;
     }
     std::vector<GroupWorld> order;
     for (const GroupWorld& g : table) {
-        if (g.dynamic_count + g.static_count > kGroupRowLimit) return;
+        if (g.dynamic_count + g.static_count > kGroupRowLimit) return DYN_OK;
         if (g.dynamic_count + g.static_count) order.push_back(g);
     }
     auto rows = [](const GroupWorld& g) { return g.dynamic_count + g.static_count; };
     std::stable_sort(order.begin(), order.end(), [&](const GroupWorld& a, const GroupWorld& b) { return rows(a) > rows(b); });
-    if (order.empty()) return;
+    if (order.empty()) return DYN_OK;
     GroupPlan plan;
     plan.count = static_cast<uint32_t>(order.size());
     plan.rows = rows(order[0]);
     plan.whole = plan.rows <= kGroupWholeRows && plan.count <= kGroupWholeWorlds;
-    if (!plan.whole && !group_position_pays(plan.count, plan.rows, w.n)) return;
+    if (!plan.whole && !group_position_pays(plan.count, plan.rows, w.n)) return DYN_OK;
     GroupWorld* device = nullptr;
     if (alloc(world, &device, order.size()) != DYN_OK ||
         hipMemcpy(device, order.data(), sizeof(GroupWorld) * order.size(), hipMemcpyHostToDevice) != hipSuccess) {
-        return;
+        return fail(DYN_E_HIP, "dyn_batch_create: world table");
     }
     plan.worlds = device;
     world->groups = plan;
+    return DYN_OK;
 }
 
 void drop_graph(dyn_world* world) {
@@ -4171,7 +4173,11 @@ int dyn_batch_create(dyn_world** out, void* stream, const dyn_step_params* param
     }
     world->w.worlds = worlds;
     world->groups = GroupPlan{};
-    plan_groups(world, collider_worlds, collider_count, world_of_row, world_count);
+    const int rc = plan_groups(world, collider_worlds, collider_count, world_of_row, world_count);
+    if (rc != DYN_OK) {
+        dyn_world_destroy(world);
+        return rc;
+    }
     *out = world;
     return DYN_OK;
 }
