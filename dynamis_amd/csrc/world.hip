@@ -3788,20 +3788,25 @@ int solver(const dyn::W& w, hipStream_t st, const GroupPlan& plan, uint32_t thre
 // the worlds must be few or large enough (group_position_pays); otherwise there is none, and the batch
 // is solved by the launched passes.
 int plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t colliders,
-                const std::vector<uint32_t>& world_of_row, uint32_t worlds) {
+                const std::vector<uint32_t>& world_of_row) {
     using namespace dyn;
     const W& w = world->w;
     for (uint32_t i = 1; i < colliders; ++i) {
         if (collider_worlds[i] < collider_worlds[i - 1]) return DYN_OK;
     }
-    std::vector<GroupWorld> table(worlds, GroupWorld{});
+    std::vector<uint32_t> ids;  // the worlds that have colliders, which may be few of many ids
+    std::vector<GroupWorld> table;
     for (uint32_t i = 0; i < colliders; ++i) {
-        GroupWorld& g = table[collider_worlds[i]];
-        if (g.collider_count++ == 0u) g.collider_base = i;
+        if (i == 0u || collider_worlds[i] != collider_worlds[i - 1]) {
+            ids.push_back(collider_worlds[i]);
+            table.push_back(GroupWorld{});
+            table.back().collider_base = i;
+        }
+        ++table.back().collider_count;
     }
     for (uint32_t row = 0; row < w.n; ++row) {
         if (world_of_row[row] == DYN_NO_BODY) return DYN_OK;
-        GroupWorld& g = table[world_of_row[row]];
+        GroupWorld& g = table[std::lower_bound(ids.begin(), ids.end(), world_of_row[row]) - ids.begin()];
         uint32_t& base = row < w.d ? g.dynamic_base : g.static_base;
         uint32_t& count = row < w.d ? g.dynamic_count : g.static_count;
         if (count == 0u) base = row;
@@ -4173,7 +4178,7 @@ int dyn_batch_create(dyn_world** out, void* stream, const dyn_step_params* param
     }
     world->w.worlds = worlds;
     world->groups = GroupPlan{};
-    const int rc = plan_groups(world, collider_worlds, collider_count, world_of_row, world_count);
+    const int rc = plan_groups(world, collider_worlds, collider_count, world_of_row);
     if (rc != DYN_OK) {
         dyn_world_destroy(world);
         return rc;

@@ -139,20 +139,41 @@ def test_sizes_side_by_side(device):
     assert beside == alone
 
 
+def batch_of(scene, colliders, owners, worlds, world_count) -> World:
+    world = World()
+    world.scene = scene
+    colliders, owners, worlds = (np.ascontiguousarray(a) for a in (colliders, owners, worlds))
+    n, k = len(scene.states), len(colliders)
+    call("dyn_batch_create", ctypes.byref(world._handle), None, scene.params.ctypes.data, scene.states.ctypes.data,
+         scene.descs.ctypes.data, n, scene.dynamic_count, colliders.ctypes.data, owners.ctypes.data,
+         worlds.ctypes.data, k, world_count, 8 * n, 32 * n)
+    return world
+
+
+def test_batch_of_sparse_world_ids(device):
+    """Two worlds with the ids 7 and 2^32 - 2 of 2^32 - 1: creation keeps nothing for an id without colliders."""
+    scenes = [encode(cube_drop(30, seed=3 + i, footprint=4.0, low=1.0, high=3.0), config()) for i in range(2)]
+    batch = Batch(scenes)
+    merged, worlds = batch.scene, batch.layout.collider_worlds
+    ids = np.array([7, 0xFFFFFFFE], np.uint32)[worlds]
+    world = batch_of(merged, merged.colliders, merged.owners, ids, 0xFFFFFFFF)
+    for _ in range(40):
+        batch.step(DT)
+        world.step(DT)
+    assert "k_group_solve" in kernels_of_a_step(world)
+    batch.step(DT)
+    assert world.states().tobytes() == batch.states().tobytes()
+    batch.close()
+    world.close()
+
+
 def test_batch_of_scattered_colliders(device):
     """Colliders of two worlds interleaved: their contacts are no runs, and the launched passes run."""
     scenes = [encode(cube_drop(30, seed=3 + i, footprint=4.0, low=1.0, high=3.0), config()) for i in range(2)]
     batch = Batch(scenes)
     merged, worlds = batch.scene, batch.layout.collider_worlds
     mixed = np.argsort(np.concatenate([np.arange(31), np.arange(31)]), kind="stable")
-    world = World()
-    world.scene = merged
-    owners, order = merged.owners[mixed].copy(), worlds[mixed].copy()
-    colliders = merged.colliders[mixed].copy()
-    n, k = len(merged.states), len(colliders)
-    call("dyn_batch_create", ctypes.byref(world._handle), None, merged.params.ctypes.data, merged.states.ctypes.data,
-         merged.descs.ctypes.data, n, merged.dynamic_count, colliders.ctypes.data, owners.ctypes.data,
-         order.ctypes.data, k, 2, 8 * n, 32 * n)
+    world = batch_of(merged, merged.colliders[mixed], merged.owners[mixed], worlds[mixed], 2)
     for _ in range(40):
         batch.step(DT)
         world.step(DT)
