@@ -505,9 +505,8 @@ static int launch_passes(hipStream_t stream, uint32_t* major, uint32_t* minor, u
     // Persistent workgroups take tiles in order (any count makes progress: a tile's look-back only
     // waits on earlier tiles, which running groups hold). The tiles of 8 keys a lane: a stream with
     // few live records takes those whatever ITEMS is.
-    constexpr uint32_t kTile = kSortThreads * 8;
-    static_assert(kTile >= kSortMinTile, "the look-back words are laid out for the narrowest tiling");
-    const uint32_t tiles = ceil_div(capacity ? capacity : 1u, kTile);
+    static_assert(ITEMS * kSortThreads >= kSortMinTile, "the look-back words are laid out for the narrowest tiling");
+    const uint32_t tiles = ceil_div(capacity ? capacity : 1u, kSortMinTile);
     const uint32_t groups = tiles < group_cap ? tiles : group_cap;
     const size_t flag_stride = static_cast<size_t>(s.max_tiles) * kSortBins;
     uint32_t* src[3] = {major, minor, payload};

@@ -92,3 +92,11 @@ def test_scratch_sizes_grow_with_capacity():
     assert large >= 3 * 4 * 1_000_000
     assert lib.dyn_broadphase_scratch_bytes(1000, 8000, 8000) > 0
     assert np.uint64(lib.dyn_broadphase_scratch_bytes(0, 0, 0)) > 0
+
+
+def test_sort_scratch_holds_the_words_that_a_pass_indexes():
+    """A pass more costs a look-back word for each digit of each narrowest tile (512 lanes, 8 keys)."""
+    lib = _native.lib()
+    for capacity in (1, 4096, 4097, 100_000, 1 << 20):
+        tiles = -(-capacity // 4096)
+        assert lib.dyn_sort_scratch_bytes(capacity, 4) - lib.dyn_sort_scratch_bytes(capacity, 3) == tiles * 256 * 4
