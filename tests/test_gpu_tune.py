@@ -4,6 +4,8 @@ world whose sorts were tuned steps bit for bit as an untuned one; the per-GPU ca
 from __future__ import annotations
 
 import ctypes
+import pathlib
+import re
 
 import numpy as np
 import pytest
@@ -12,26 +14,39 @@ from dynamis_amd import scenes, tune
 from dynamis_amd._native import call
 from dynamis_amd.sort import RadixSort, SortChannels, units_for
 from dynamis_amd.world import World, encode
-from tests.sort_cases import expected_order, xorshift
+from tests.sort_cases import expected_order
 
 pytestmark = pytest.mark.gpu
 
 TILINGS = [(8, 512), (8, 1024), (8, 2048), (16, 512), (16, 1024), (16, 2048)]
 
 
-@pytest.mark.parametrize("items,groups", TILINGS)
-def test_every_tiling_sorts_the_same(device, items, groups):
-    n = 300_000
-    major, minor = xorshift(n, 11), xorshift(n, 12)
+SORT_THREADS = int(re.search(r"kSortThreads = (\d+);", (pathlib.Path(tune.__file__).parent / "csrc" / "sort.h").read_text())[1])
+NARROW_BELOW = 1572864  # live records up to which every tiling runs 8 keys a lane
+
+
+# 300,000 records; two tiles more than there are workgroups, so that some take a second ticket and the
+# others one past the last tile; the fewest records that run 16 keys a lane
+@pytest.mark.parametrize("items,groups,n", [(i, g, 300_000) for i, g in TILINGS] +
+                         [(i, g, SORT_THREADS * i * (g + 1) + 77) for i, g in TILINGS] + [(16, 2048, NARROW_BELOW + 1)])
+def test_every_tiling_sorts_the_same(device, items, groups, n):
+    rng = np.random.default_rng(n)
+    major, minor = (rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(2))
+    # all eight digits where numpy's sort is quick enough, else two of them
+    words = (4, 4) if n < 1 << 21 else (1, 1)
     payload = np.arange(n, dtype=np.uint32)
     try:
         tune.load(np.array([[0, tune.bucket(n), items, groups]], np.uint32))
         channels = SortChannels.upload(major, minor, payload)
-        RadixSort().sort(channels, units_for(n), 4, 4)
+        RadixSort().sort(channels, units_for(n), *words)
         m, k, p = channels.download(n)
     finally:
         tune.load(np.zeros((0, 4), np.uint32))
-    assert np.array_equal(p, expected_order(major, minor, 4, 4))
+    if words == (4, 4):
+        assert np.array_equal(p, expected_order(major, minor, *words))
+    else:
+        key = ((major & 0xFF) << 8 | (minor & 0xFF)).astype(np.uint16)
+        assert np.array_equal(p, np.argsort(key, kind="stable"))
     assert np.array_equal(m, major[p]) and np.array_equal(k, minor[p])
 
 
