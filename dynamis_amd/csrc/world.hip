@@ -1218,7 +1218,7 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(ScanSums a, ScanSums b) {
 __device__ inline uint32_t scan_before(const ScanSums& s, const uint32_t* __restrict__ flags, uint32_t live,
                                        uint32_t first, uint32_t* s_scan, uint32_t* all) {
     const uint32_t group = first / kScanBlock;
-    uint32_t before = 0, rest = 0;
+    uint32_t before = 0, every = 0;
     for (uint32_t i = group * kScanBlock + threadIdx.x; i < first; i += kThreads) {  // its group's flags before it
         if (i < live && flags[i]) ++before;
     }
@@ -1227,7 +1227,7 @@ __device__ inline uint32_t scan_before(const ScanSums& s, const uint32_t* __rest
         for (uint32_t g = threadIdx.x; g < end; g += kThreads) {
             const uint32_t v = s.sums[g];
             if (g < group) before += v;
-            else rest += v;
+            every += v;
         }
     }
     uint32_t total = 0;
@@ -1237,14 +1237,7 @@ __device__ inline uint32_t scan_before(const ScanSums& s, const uint32_t* __rest
         if (group < s.groups) base += s.sums[group];
         if (all) *all = *s.total;
     } else if (all) {
-        uint32_t partial = 0;
-        for (uint32_t i = group * kScanBlock + threadIdx.x; i < first; i += kThreads) {
-            if (i < live && flags[i]) ++partial;
-        }
-        uint32_t in_group = 0;
-        block_exclusive_sum<kThreads>(partial, s_scan, &in_group);
-        block_exclusive_sum<kThreads>(rest, s_scan, &total);
-        *all = base - in_group + total;
+        block_exclusive_sum<kThreads>(every, s_scan, all);
     }
     return base;
 }
