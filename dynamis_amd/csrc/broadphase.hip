@@ -228,7 +228,6 @@ __global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb*
                                                                  uint32_t* cnt_level, uint32_t* block_offsets,
                                                                  uint32_t* sort_hist, uint32_t* sort_ctl,
                                                                  uint32_t entry_capacity) {
-    constexpr uint32_t kWaves = kFrontThreads / kWave;
     constexpr uint32_t kBlocks = kFrontColliders / kBpThreads;
     __shared__ uint32_t s_stats[5];          // scale, extent, levels, faults, coarse
     __shared__ uint32_t s_blocks[kBlocks];   // entries of each emission workgroup's colliders
@@ -284,7 +283,7 @@ __global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb*
     }
     __syncthreads();
     if (t < kWave) {
-        static_assert(kBlocks <= kWave && kWaves >= 1u, "one wave scans the blocks");
+        static_assert(kBlocks <= kWave, "one wave scans the blocks");
         const uint32_t v = t < kBlocks ? s_blocks[t] : 0u;
         const uint32_t inclusive = wave_inclusive_sum(v);
         if (t * kBpThreads < n) block_offsets[t] = inclusive - v;
