@@ -87,6 +87,25 @@ def test_reserve_and_snapshot_capacities(device):
     again.close()
 
 
+@pytest.mark.parametrize("capacity", [4096 * 1024, 4096 * 1024 + 1])
+def test_compaction_of_long_streams(device, capacity):
+    """Streams of 4,096 blocks of 1,024 flags, whose sums the moving pass adds up by itself, and of one more,
+    which are scanned first: contacts, the resting archive and the states as in streams of the usual size."""
+    scene = encode(cube_drop(60, seed=3, footprint=8.0, high=4.0), default_config())
+    dev, usual = device_world(scene, None, None), device_world(scene, None, None)
+    dev.reserve(capacity, capacity)
+    for frame in range(240):
+        dev.step(DT)
+        usual.step(DT)
+        if frame % 60 == 59:
+            assert dev.states().tobytes() == usual.states().tobytes()
+            assert dev.inspect_contacts().tobytes() == usual.inspect_contacts().tobytes()
+            assert dev.measured() == usual.measured()
+    assert usual.measured()["RESTING"] > 0
+    dev.close()
+    usual.close()
+
+
 def test_differentiable_rollout_holds_capacities(device):
     sc, cfg, _ = scenes.adjoint_worlds(2, 8, seed=7)
     batch = Batch(sc, cfg)

@@ -13,16 +13,17 @@ import pytest
 
 from dynamis_amd._native import call
 from dynamis_amd.device import profile_collect, profile_enable
+from dynamis_amd.solver import Solver
 from dynamis_amd.world import Batch, World
-from tests.solve_cases import NO_SLEEP, drop_scene
+from tests.solve_cases import drop_scene, solver_inputs
 from tests.test_gpu_solve import check_parity
 from tests.worlds import DT, config, cube_drop, encode
 
 pytestmark = pytest.mark.gpu
 
 
-# bodies (a plane more): 64 | 65 rows (128 | 256 threads), 160 | 161 (whole | position only),
-# 256 | 257 (256 | 1,024 threads); 1502 | 1503 below (position only | launched)
+# bodies (a plane more): 64 | 65 rows (256 | 512 lanes), 160 | 161 (whole | position only),
+# 256 | 257 (256 | 1,024 lanes); 1502 | 1503 below (position only | launched)
 @pytest.mark.parametrize("count", [1, 63, 64, 159, 160, 255, 256])
 def test_row_edges(device, oracle, count):
     check_parity(oracle, drop_scene(count, footprint=1.2 + 0.35 * count ** 0.5), 60, 0 if count == 1 else count // 2)
@@ -35,11 +36,26 @@ def test_row_limit(device, oracle, count):
     check_parity(oracle, drop_scene(count, footprint=side), 4, 4000 if count > 2000 else 1500)
 
 
-@pytest.mark.parametrize("count,footprint", [(159, 1.5), (255, 1.0)])
-def test_more_contacts_than_registers_hold(device, oracle, count, footprint):
-    # cubes dropped onto one spot overlap one another many times over: above 4 x 256 contacts
-    scene = encode(cube_drop(count, seed=5, footprint=footprint, low=1.0, high=4.0), config(**NO_SLEEP))
-    check_parity(oracle, scene, 2, 1025)
+# Blocks that a workgroup of k_group_solve has a quad for each, kept in registers (64 of 256 lanes up to 64
+# rows, 128 of 512 up to 160), and contacts that the position iterations hold, four a lane (1,024, 2,048;
+# k_group_position 1,024 of 256 lanes up to 256 rows, 4,096 of 1,024 above): just as many and one more, and no contact.
+@pytest.mark.parametrize("bodies,contacts", [
+    (40, 0), (40, 64), (40, 65), (40, 1024), (40, 1025), (120, 128), (120, 129), (120, 2048), (120, 2049),
+    (200, 1024), (200, 1025), (400, 4096), (400, 4097)])
+def test_contacts_that_registers_hold(device, oracle, bodies, contacts):
+    scene = drop_scene(bodies, footprint=1.2 + 0.35 * bodies ** 0.5)
+    inputs, some, _, _ = solver_inputs(oracle, scene, 60)
+    assert len(some) > bodies // 2
+    given = np.resize(some, contacts) if contacts else some[:0]  # the list over and over
+    ref = oracle.world(inputs, contact_capacity=max(contacts, 1))
+    want_contacts = ref.solve(given, DT)
+    want_states = ref.states()
+    ref.close()
+    solver = Solver(inputs, max(contacts, 1))
+    solver.run(inputs.states, given, DT)
+    states, got_contacts, _ = solver.read()
+    assert states.tobytes() == want_states.tobytes()
+    assert got_contacts.tobytes() == want_contacts.tobytes()
 
 
 def test_sleeping_rows(device, oracle):
