@@ -151,8 +151,9 @@ struct PassArgs {
 
 // Passes of 8 keys a lane read the digits' counts beside the control words, and up to this many tiles draw
 // their first ticket before the counts' scan: a pass of few tiles is a chain of latencies, which are then
-// beside one another. A fixed grid of 8,043 boxes (25 launches) takes 120 us so and 122 without, a million
-// records of six digits 128.7 and 130.8; with 16 keys a lane it was 3 us slower at 3,000,017 records.
+// beside one another. A fixed grid of 8,043 boxes (25 launches) takes 120 us so and 123 without, a million
+// records of six digits 129 and 131; with 16 keys a lane, where registers are short, 3,000,017 records
+// took 209 us so and 206 without.
 constexpr uint32_t kFewTiles = 128;
 
 // One digit pass over tiles of kSortThreads * ITEMS keys. A workgroup with no tile leaves at once,
@@ -184,15 +185,16 @@ __device__ __forceinline__ void sort_pass(const PassArgs& a, uint32_t* s_stage) 
     const uint32_t ntiles = ceil_div(len, TILE);
     if (blockIdx.x >= ntiles) return;
 
-    // Global start of every digit: exclusive scan of this pass's histogram.
-    const bool few = ITEMS <= 8 && ntiles <= kFewTiles;
+    bool drawn = ITEMS <= 8 && ntiles <= kFewTiles;
     uint32_t ticket = 0;
-    if (few && t == 0) ticket = atomicAdd(&ctl[kCtlTiles + pass], 1u);
+    if (drawn && t == 0) ticket = atomicAdd(&ctl[kCtlTiles + pass], 1u);
+    // Global start of every digit: exclusive scan of this pass's histogram.
     if (ITEMS > 8 && t < kSortBins) digit_count = a.hist[t];
     const uint32_t digit_base = block_exclusive_sum<kSortThreads>(digit_count, s_scan, nullptr);
-    if (!few && t == 0) ticket = atomicAdd(&ctl[kCtlTiles + pass], 1u);
     for (;;) {
+        if (!drawn && t == 0) ticket = atomicAdd(&ctl[kCtlTiles + pass], 1u);
         if (t == 0) s_tile = ticket;
+        drawn = false;
         for (uint32_t k = t; k < WAVES * kSortBins; k += kSortThreads) (&s_wave[0][0])[k] = 0u;
         __syncthreads();
         const uint32_t tile = s_tile;
@@ -327,7 +329,6 @@ __device__ __forceinline__ void sort_pass(const PassArgs& a, uint32_t* s_stage) 
             }
         }
         if (gridDim.x >= ntiles) break;  // a workgroup per tile: this was its only one
-        if (t == 0) ticket = atomicAdd(&ctl[kCtlTiles + pass], 1u);
         __syncthreads();
     }
 }
