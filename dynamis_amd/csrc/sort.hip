@@ -878,8 +878,12 @@ int dyn_sort_pairs_static(void* stream, uint32_t* d_major, uint32_t* d_minor, ui
         return dyn_sort_pairs(stream, d_major, d_minor, d_payload, capacity, d_count, d_base, plan, major_words,
                               minor_words, nullptr, 0u);  // the same argument errors
     }
+    // The capacities refused are those whose look-back words would not fit for tiles of 2,048 keys, as when
+    // the array was sized, and not those that fit since tiles are larger: a caller's limit stays its limit.
+    const uint32_t passes = major_words + minor_words;
+    const size_t words = size_t{passes} * (ceil_div(capacity, 2048u) - ceil_div(capacity, kSortMinTile)) * kSortBins;
     if (capacity > kSortMaxCapacity ||
-        sort_scratch_layout(capacity, major_words + minor_words, true, nullptr, nullptr) > kStaticScratchBytes) {
+        sort_scratch_layout(capacity, passes, true, nullptr, nullptr) + 4u * words > kStaticScratchBytes) {
         return fail(DYN_E_CAPACITY, "dyn_sort_pairs_static: capacity beyond the static scratch (2^20 records)");
     }
     void* base = nullptr;

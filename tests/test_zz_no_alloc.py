@@ -66,5 +66,10 @@ def test_capacity_beyond_the_static_scratch_is_refused(device):
     big = SortChannels.upload(major, minor, payload, 1_400_000)
     with pytest.raises(DynamisError, match="beyond the static scratch"):
         sort_static(big, 4, 4)
+    # the limits at eight digits and at one, to the record
+    for words, most in (((4, 4), 1_113_408), ((1, 0), 1_425_344)):
+        sort_static(SortChannels.upload(major, minor, payload, most), *words)
+        with pytest.raises(DynamisError, match="beyond the static scratch"):
+            sort_static(SortChannels.upload(major, minor, payload, most + 1), *words)
     with pytest.raises(DynamisError):
         sort_static(SortChannels.upload(major, minor, payload), 0, 0)
