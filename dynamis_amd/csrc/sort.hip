@@ -151,7 +151,7 @@ struct PassArgs {
 
 // Passes of 8 keys a lane read the digits' counts beside the control words, and up to this many tiles draw
 // their first ticket before the counts' scan: a pass of few tiles is a chain of latencies, which are then
-// beside one another. A fixed grid of 8,043 boxes (25 launches) takes 120 us so and 123 without, a million
+// beside one another. A fixed grid of 8,043 boxes (10 passes) takes 120 us so and 123 without, a million
 // records of six digits 129 and 131; with 16 keys a lane, where registers are short, 3,000,017 records
 // took 209 us so and 206 without.
 constexpr uint32_t kFewTiles = 128;

@@ -838,10 +838,10 @@ constexpr uint32_t kQuadPairs = kThreads / kQuad;  // pairs of a workgroup
 // GJK lists longer than this are run one thread a pair (convex.h says why): four lanes a pair then fill
 // the GPU many times over (2^17 pairs are 8,192 waves of quads, 8 a SIMD).
 constexpr uint32_t kLongGjk = 1u << 17;
-// The same for the lists of resumed pairs, whose quads stay longer below the vector units' bound: 70,560
-// pairs take 175 us by quads and 209 by threads, 94,080 210 and 217, 141,120 282 and 247 (a settled
-// 100k pile's 157,257: 398 and 283).
-constexpr uint32_t kLongResume = 3u << 15;
+// The same for the lists of resumed pairs, whose quads stay longer below the vector units' bound: in
+// settling piles 53,475 pairs take 189 us by quads and 231 by threads, 74,843 228 and 243, 87,441 253 and
+// 246, 156,364 398 and 286.
+constexpr uint32_t kLongResume = 5u << 14;
 
 template <typename Pair>
 struct ConvexPair {
