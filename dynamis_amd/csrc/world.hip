@@ -835,9 +835,10 @@ constexpr uint32_t kGjkFirstIterations = 8;
 
 constexpr uint32_t kQuad = 4;                     // lanes per pair
 constexpr uint32_t kQuadPairs = kThreads / kQuad;  // pairs of a workgroup
-// GJK lists longer than this are run one thread a pair (convex.h says why): four lanes a pair then fill
-// the GPU many times over (2^17 pairs are 8,192 waves of quads, 8 a SIMD).
-constexpr uint32_t kLongGjk = 1u << 17;
+// GJK lists longer than this are run one thread a pair (convex.h says why). In settling piles 66,230 pairs
+// take 141 us by quads and 150 by threads, 79,518 148 and 161, 92,938 164 and 162, 106,469 183 and 160,
+// 123,288 209 and 164.
+constexpr uint32_t kLongGjk = 11u << 13;
 // The same for the lists of resumed pairs, whose quads stay longer below the vector units' bound: in
 // settling piles 53,475 pairs take 189 us by quads and 231 by threads, 74,843 228 and 243, 87,441 253 and
 // 246, 156,364 398 and 286.

@@ -1,5 +1,5 @@
 """The narrowphase's pair lists and its two kinds of GJK at their edges: pair capacities on both sides of
-the one-workgroup grouping, and lists long enough for one thread a pair (above 131,072 GJK pairs, above
+the one-workgroup grouping, and lists long enough for one thread a pair (above 90,112 GJK pairs, above
 81,920 resumed ones). The same pairs repeated give the same contacts in every copy, and the first copy is
 held to the oracle by the stage's own tests."""
 
@@ -70,7 +70,7 @@ def test_split_edges(pile, count):
 
 
 # the lists' limits, and a quarter more for what moved since the step whose lists are counted
-LONG_GJK, LONG_RESUME, MARGIN = 1 << 17, 5 << 14, 1.25
+LONG_GJK, LONG_RESUME, MARGIN = 11 << 13, 5 << 14, 1.25
 
 
 @pytest.mark.parametrize("long_resume", [False, True])
