@@ -2693,9 +2693,10 @@ __device__ __forceinline__ void solve_block_alone(const W& w, uint32_t ci, bool 
 }
 
 // Blocks above which an iteration gives each a single lane: enough waves to fill the chip, which quads
-// would only multiply. 228k blocks take 25.7 us by lanes and 33.9 by quads (where the memory is half of
-// it), 33k take 9.3 by quads and 10.9 by lanes.
-constexpr uint32_t kLongSolve = 1u << 17;
+// would only multiply. In settling piles 28,776 blocks take 10.1 us by quads and 11.3 by lanes, 39,902 11.8
+// and 11.6, 56,858 14.3 and 12.5, 115,968 20.6 and 17.0, 268,862 36.6 and 28.4 (where the memory is half of
+// it); of cubes 43,282 11.8 and 12.0, 61,693 14.5 and 13.5.
+constexpr uint32_t kLongSolve = 5u << 13;
 __global__ void __launch_bounds__(kThreads) k_solve(W w, uint32_t residual) {
     const uint32_t at = blockIdx.x * blockDim.x + threadIdx.x, count = *w.ncontacts;
     if (count > kLongSolve) {

@@ -1,4 +1,4 @@
-"""The solver's blocks by quads and by single lanes (above 2^17 blocks), with rolling and spin friction
+"""The solver's blocks by quads and by single lanes (above 40,960 blocks), with rolling and spin friction
 and compliance, which no scene of the other solver tests has: blocks of one to four points with zero,
 small and large limits, in worlds solved whole by a workgroup and by the launched passes. Bit
 for bit against the oracle's solver."""
@@ -16,7 +16,8 @@ from tests.worlds import config, ellipsoid_hulls, encode, mixed_pile
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("bodies,blocks", [(40, 0), (200, 0), (200, 1 << 17), (200, (1 << 17) + 1)])
+@pytest.mark.parametrize("bodies,blocks", [(40, 0), (200, 0), (200, 5 << 13), (200, (5 << 13) + 1),
+                                           (200, 1 << 17), (200, (1 << 17) + 1)])
 def test_blocks(device, oracle, bodies, blocks):
     scene = encode(mixed_pile(bodies, seed=4, kinds=5, hull_sources=4, spacing=1.4), config(**NO_SLEEP),
                    ellipsoid_hulls(4, seed=3))
