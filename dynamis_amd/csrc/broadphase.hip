@@ -217,9 +217,11 @@ __global__ void __launch_bounds__(1024) bp_scan_kernel(const uint32_t* __restric
 }
 
 // The passes above (reset, resolution, fold, count, scan) in one workgroup, for up to kFrontColliders
-// colliders: four launches saved, and each of them was a few hundred colliders' work.
+// colliders: four launches saved, and each of them was a few hundred colliders' work. A broadphase of 1,001
+// boxes takes 83 us so and 88 with the passes launched, of 1,500 106 and 109, of 2,048 112.4 and 112.7, of
+// 2,500 114.6 and 113.5, of 4,096 128 and 118.
 constexpr uint32_t kFrontThreads = 1024;
-constexpr uint32_t kFrontColliders = 4u * kFrontThreads;
+constexpr uint32_t kFrontColliders = 2u * kFrontThreads;
 
 __global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb* __restrict__ aabbs,
                                                                  const dyn_aabb* __restrict__ resolution,
@@ -304,9 +306,11 @@ __global__ void __launch_bounds__(kFrontThreads) bp_front_kernel(const dyn_aabb*
 }
 
 // Workgroups up to which the emission also counts the sort's digits, saving a launch and a read of the
-// keys. Every workgroup adds its counts to the same 1,024 words, one atomic after another: at 2^20
-// boxes that made the emission 111 us, against 74 us and a 20 us pass over the keys without it.
-constexpr uint32_t kEmitHistogramBlocks = 128;
+// keys. Every workgroup adds its counts to the same 1,024 words, one atomic after another: at 2^20 boxes
+// that made the emission 111 us, against 74 us and a 20 us pass over the keys without it (the whole 655 and
+// 637 us). At 33,000 boxes the whole takes 157 us so and 159 without, at 131,072 222.6 and 224.1, at 262,144
+// 279.6 and 278.7.
+constexpr uint32_t kEmitHistogramBlocks = 512;
 
 // collider_emit.wgsl:6-63 with slots from the scan.
 template <bool kHistogram>

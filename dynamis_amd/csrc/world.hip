@@ -680,7 +680,9 @@ __global__ void __launch_bounds__(kThreads) k_class_scatter(W w) {
     }
 }
 
-// The three passes above in one workgroup, for small pair capacities.
+// The three passes above in one workgroup, for small pair capacities. What it takes follows the live pairs,
+// of which the host knows only the capacity, mostly two to ten times as many: a narrowphase of 2,000 pairs
+// takes 60 us so and 64 by launches, of 4,000 375 and 389, of 8,000 439 and 436, of 16,000 470 and 450.
 constexpr uint32_t kClassSmall = 16384;
 __global__ void __launch_bounds__(1024) k_class_small(W w) {
     __shared__ uint32_t cursor[kClasses];

@@ -1,5 +1,6 @@
-"""The broadphase at the edges of its launch shapes: the one-workgroup front (4,096 colliders), the
-one-workgroup entry and pair sorts, the link modes (32,768 colliders), partial workgroups, a few large
+"""The broadphase at the edges of its launch shapes: the one-workgroup front (2,048 colliders), the
+one-workgroup entry and pair sorts, the link modes (32,768 colliders), the digits counted by the emission
+(131,072 colliders), partial workgroups, a few large
 boxes among small ones, and streams too short for the entries or the pairs. Against the oracle."""
 
 from __future__ import annotations
@@ -23,7 +24,8 @@ def boxes_of(count, large):
     return boxes
 
 
-@pytest.mark.parametrize("count", [1, 255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 32768, 32769])
+@pytest.mark.parametrize("count", [1, 255, 256, 257, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 32768,
+                                   32769, 131072, 131073])
 @pytest.mark.parametrize("large", [0, 5])
 def test_sizes(device, oracle, count, large):
     boxes = boxes_of(count, large)
