@@ -3676,15 +3676,17 @@ constexpr uint32_t kGroupWholeWorlds = 1024;
 
 // Whether k_group_position, a workgroup a world, beats the launched position iterations: `count` worlds
 // of `rows` rows in all, the largest of `largest`. In ns a substep of ten iterations: the launched ones
-// take 50,000 and 0.72 a row; a workgroup takes 34 a row of its world, and its share of the chip is 21
-// where it has 256 lanes and 62 where it has 1,024 (one a CU), however few rows its world has. A step by
-// k_group_position and by launches, in us: one world of 1,400 bodies 602 and 618, of 1,600 635 and 627, of
-// 2,300 718 and 662, 16 of 2,300 1,318 and 1,324; 2,048 worlds of 8 715 and 747, 4,096 878 and 832, 10,000
-// 1,368 and 1,083; 4,096 of 32 1,662 and 1,728; 2,000 of 100 beside one of 2,300 2,722 and 2,825, 10,000 of 8
-// beside it 2,276 and 1,248; 4,096 of 8 to 2,048 12,060 and 13,523.
-bool group_position_pays(uint32_t count, uint32_t largest, uint32_t rows) {
+// take `launched` (20 launches, in a captured step or issued by the host one by one) and 0.72 a row; a
+// workgroup takes 34 a row of its world, and its share of the chip is 21 where it has 256 lanes and 62
+// where it has 1,024 (one a CU), however few rows its world has. A step by k_group_position and by launches,
+// in us: one world of 1,400 bodies 602 and 618, of 1,600 635 and 627, of 2,300 718 and 662 (dyn_solve, which
+// is never captured: 320 and 387), 16 of 2,300 1,318 and 1,324; 2,048 worlds of 8 715 and 747, 4,096 878 and
+// 832, 10,000 1,368 and 1,083; 4,096 of 32 1,662 and 1,728; 2,000 of 100 beside one of 2,300 2,722 and 2,825,
+// 10,000 of 8 beside it 2,276 and 1,248; 4,096 of 8 to 2,048 12,060 and 13,523.
+constexpr double kLaunchedCaptured = 50000.0, kLaunchedAlone = 110000.0;
+bool group_position_pays(uint32_t count, uint32_t largest, uint32_t rows, double launched) {
     const double group = std::max(34.0 * largest, count * (largest <= 256u ? 21.0 : 62.0));
-    return group <= 50000.0 + 0.72 * rows;
+    return group <= launched + 0.72 * rows;
 }
 
 template <typename Kernel, typename... Args>
@@ -3718,9 +3720,9 @@ int group_position(const dyn::W& w, hipStream_t st, const GroupPlan& g, uint32_t
 }
 
 // The plan of one world of n rows.
-GroupPlan plan_group(uint32_t n) {
+GroupPlan plan_group(uint32_t n, double launched) {
     GroupPlan plan;
-    if (n && n <= kGroupRowLimit && group_position_pays(1u, n, n)) {
+    if (n && n <= kGroupRowLimit && group_position_pays(1u, n, n, launched)) {
         plan.count = 1u;
         plan.rows = n;
         plan.whole = n <= kGroupWholeRows;
@@ -3822,7 +3824,7 @@ int plan_groups(dyn_world* world, const uint32_t* collider_worlds, uint32_t coll
     plan.count = static_cast<uint32_t>(order.size());
     plan.rows = rows(order[0]);
     plan.whole = plan.rows <= kGroupWholeRows && plan.count <= kGroupWholeWorlds;
-    if (!plan.whole && !group_position_pays(plan.count, plan.rows, w.n)) return DYN_OK;
+    if (!plan.whole && !group_position_pays(plan.count, plan.rows, w.n, kLaunchedCaptured)) return DYN_OK;
     GroupWorld* device = nullptr;
     if (alloc(world, &device, order.size()) != DYN_OK ||
         hipMemcpy(device, order.data(), sizeof(GroupWorld) * order.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -4139,7 +4141,7 @@ int dyn_world_create(dyn_world** out, void* stream, const dyn_step_params* param
     up(w.row_of_body, row_of_body.data(), sizeof(uint32_t) * id_cap);
     up(w.owner, owners, 4u * collider_count);
     if (rc != DYN_OK) return cleanup(fail(DYN_E_HIP, "dyn_world_create: upload"));
-    world->groups = plan_group(w.n);
+    world->groups = plan_group(w.n, kLaunchedCaptured);
     *out = world;
     return DYN_OK;
 }
@@ -4689,7 +4691,7 @@ int dyn_solve(void* stream, const dyn_solve_io* io, float dt) {
     DYN_HIP(hipMemcpyAsync(&bad, words + 1, 4u, hipMemcpyDeviceToHost, st));
     DYN_HIP(hipStreamSynchronize(st));
     if (bad) return fail(DYN_E_INVALID, "dyn_solve: a contact names a collider or body outside the records");
-    return solver(w, st, plan_group(w.n));
+    return solver(w, st, plan_group(w.n, kLaunchedAlone));
 }
 
 size_t dyn_islands_scratch_bytes(uint32_t bodies) {

@@ -23,17 +23,37 @@ pytestmark = pytest.mark.gpu
 
 
 # bodies (a plane more): 64 | 65 rows (256 | 512 lanes), 160 | 161 (whole | position only),
-# 256 | 257 (256 | 1,024 lanes); 1502 | 1503 below (position only | launched)
+# 256 | 257 (256 | 1,024 lanes); 2304 | 2305 below (position only | launched)
 @pytest.mark.parametrize("count", [1, 63, 64, 159, 160, 255, 256])
 def test_row_edges(device, oracle, count):
     check_parity(oracle, drop_scene(count, footprint=1.2 + 0.35 * count ** 0.5), 60, 0 if count == 1 else count // 2)
 
 
-@pytest.mark.parametrize("count", [1501, 1502, 2303, 2304])
+@pytest.mark.parametrize("count", [2303, 2304])
 def test_row_limit(device, oracle, count):
     # a lattice of touching cubes on the plane: contacts from the first frames on
     side = 12.0
-    check_parity(oracle, drop_scene(count, footprint=side), 4, 4000 if count > 2000 else 1500)
+    profile_collect()
+    profile_enable(True)
+    check_parity(oracle, drop_scene(count, footprint=side), 4, 4000)
+    profile_enable(False)
+    assert ("k_group_position" in profile_collect()) == (count == 2303)
+
+
+@pytest.mark.parametrize("count", [1501, 1502])
+def test_world_row_limit(device, oracle, count):
+    """A world's captured steps launch their position iterations from 1,503 rows on."""
+    scene = drop_scene(count, footprint=12.0)
+    ref = oracle.world(scene)
+    with World() as world:
+        world.create(scene)
+        for _ in range(6):
+            ref.step(DT)
+            world.step(DT)
+        assert world.measured()["CONTACTS"] > 1500
+        assert world.states().tobytes() == ref.states().tobytes()
+        assert ("k_group_position" in kernels_of_a_step(world)) == (count == 1501)
+    ref.close()
 
 
 # Blocks that a workgroup of k_group_solve has a quad for each, kept in registers (64 of 256 lanes up to 64
